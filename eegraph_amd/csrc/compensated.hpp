@@ -65,4 +65,17 @@ __device__ __forceinline__ void rank_pair(float base, float d, Comp sum, float* 
     *lo = small - (h - q.s);
 }
 
+// The same with the product kept apart: contracted into an FMA with the base (as the compiler may
+// in rank_pair), d * s already carries the rounding error that pe adds again.
+__device__ __forceinline__ void rank_pair_split(float base, float d, Comp sum, float* hi, float* lo) {
+#pragma clang fp contract(off)
+    const float p = d * sum.s;
+    const float pe = fmaf(d, sum.s, -p);
+    const Comp q = two_sum(base, p);
+    const float small = q.e + (pe + d * sum.e);
+    const float h = q.s + small;
+    *hi = h;
+    *lo = small - (h - q.s);
+}
+
 }  // namespace eeg

@@ -104,6 +104,17 @@ struct PprSeg {
     bool built = false;
 };
 
+// In-edges of the streamed PageRank gather (pagerank.hip): the list in wave tiles of 1024, 16
+// consecutive edges per lane, with a word per lane (row-end bits and row ends before it), the
+// first row of every tile, the rows' vertices (bit 31: the row crosses tiles) and the positions
+// of the rows that do (few tiles from the front of span, many from its back).
+struct PrStream {
+    DevMem tcol, desc, tfirst, ent, span;
+    uint32_t ntiles = 0, nz = 0, nspan = 0, nlong = 0, span_cap = 0;
+    bool built = false;
+    bool refused = false;  // no edges, 32-bit vertex ids, or no memory: not tried again
+};
+
 // Reusable per-graph traversal state (one query at a time per handle).
 struct Work {
     DevMem lab;         // u32[n] (or f32 ranks), internal vertex order
@@ -117,6 +128,8 @@ struct Work {
     DevMem ctl;         // Ctl
     DevMem fx[2], fl[2], fc[2];  // PR: ranks as (hi, lo) pairs and contributions x/outdeg
     DevMem spill;       // PR: per-tile partial sums
+    DevMem psum;        // PR: row sums of the streamed gather
+    DevMem cerr;        // PR: rounding errors of the contributions (streamed gather)
     DevMem red;         // PR: per-workgroup residual partials
     uint32_t epoch = 1; // iteration stamps already used on stamp/flag
     DevMem devit;       // replayed iteration chunks: {iteration, stamp base}
@@ -153,6 +166,7 @@ struct eeg_graph {
     eeg::Work work;
     eeg::DevMem perm, inv;           // degree order: perm[original] = internal, inv = perm^-1
     eeg::DevMem outdeg;              // u32 out-degrees (built with the PageRank tables)
+    eeg::PrStream prstream;          // in-edges laid out for the streamed PageRank gather
     eeg::PprSeg pprseg;              // in-edge segments of the many-restart PageRank planes
     std::vector<uint32_t> h_perm;    // host copy of perm (sources map without a device read)
     uint32_t max_deg = 0, argmax_deg = 0, nonzero_out = 0;
@@ -192,7 +206,7 @@ eeg_status build_csr_from_device_edges(eeg_graph* g, const uint32_t* d_src, cons
 eeg_status ensure_tigr(eeg_graph* g, Csr& c, Tigr* table, uint32_t K);
 eeg_status ensure_sym(eeg_graph* g);
 eeg_status ensure_in(eeg_graph* g);
-eeg_status ensure_pr_span(eeg_graph* g, uint32_t K);  // pagerank.hip, after ensure_tigr(in)
+eeg_status ensure_pr_span(eeg_graph* g, uint32_t K, bool inplace);  // pagerank.hip, after ensure_tigr(in)
 eeg_status export_tigr(eeg_graph* g, uint32_t K, uint64_t* node_pointer, uint32_t* edge_list,
                        uint32_t* parts, uint64_t* num_parts);
 eeg_status orig_csr(eeg_graph* g, const Csr& src, Csr& out);

@@ -4,17 +4,19 @@
 // changes from run to run and every part of a multi-part vertex consumes the same delta
 // (D6).  Here:
 //   sync variants  - Jacobi iteration x' = (1-d)/N + d * sum_{u->v} x_u/outdeg(u), x0 = 1/N,
-//                    gathered per destination over the in-edge CSR with Tigr virtual nodes
-//                    (K in-edges each, K lanes, one edge per lane).  Each virtual node reduces
-//                    its K contributions with a fixed TwoSum tree, each vertex adds its virtual
-//                    nodes of a tile in order with compensation (TwoSum; runs longer than
-//                    PR_LONG as 64 in-order chunks joined by a fixed tree), vertices that span
-//                    tiles are finished by a fix-up pass in tile order.  Results are
-//                    deterministic.
+//                    gathered per destination over the in-edge list (k_pr_stream, then
+//                    k_pr_finish): 16 consecutive in-edges per lane summed with compensation
+//                    (TwoSum), rows that cross lanes joined by a segmented scan, rows that cross
+//                    wave tiles by their tiles' tails in tile order.  The order of every sum is
+//                    fixed, so results are deterministic.
 //                    The L1 residual is accumulated in FP64 and reduced in a fixed order.
-//   async variants - the same gather with ranks updated in place (Gauss-Seidel in tile order):
-//                    fewer sweeps, no atomics, order of reads not fixed (result within the
-//                    tolerance, not bit-reproducible).
+//   async variants - a gather with ranks updated in place (Gauss-Seidel in tile order,
+//                    k_pr_pull): Tigr virtual nodes of K in-edges, K lanes and one edge per
+//                    lane, a TwoSum tree per virtual node, each vertex's virtual nodes of a tile
+//                    in order, vertices that span tiles finished by a fix-up pass in tile order.
+//                    Fewer sweeps, no atomics, order of reads not fixed (result within the
+//                    tolerance, not bit-reproducible).  The sync variants run this kernel too
+//                    (out of place, deterministic) where the stream tables do not fit in memory.
 //   personalised   - the same iterations with a one-hot restart: x0 = e_s and
 //                    x' = (1-d) e_s + d * sum_{u->v} x_u/outdeg(u), stopped at the same L1
 //                    residual.  A residual push with a per-vertex threshold small enough for
@@ -369,6 +371,7 @@ __global__ __launch_bounds__(RED_WG) void k_pr_reduce(const double* __restrict__
 }
 
 // x0 = 1/N everywhere, or e_s when personalised (pers = s)
+template <bool PAIR>
 __global__ void k_pr_init(const uint32_t* __restrict__ outdeg, uint32_t n, float x0, uint32_t pers,
                           float* __restrict__ x, float* __restrict__ xl, float* __restrict__ c) {
     for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n;
@@ -377,7 +380,9 @@ __global__ void k_pr_init(const uint32_t* __restrict__ outdeg, uint32_t n, float
         x[v] = xv;
         xl[v] = 0.0f;
         const uint32_t d = outdeg[v];
-        c[v] = d ? xv / (float)d : 0.0f;
+        const float cv = d ? xv / (float)d : 0.0f;
+        if constexpr (PAIR) reinterpret_cast<float2*>(c)[v] = make_float2(cv, d ? (float)((double)xv / d - (double)cv) : 0.0f);
+        else c[v] = cv;
     }
 }
 
@@ -422,14 +427,413 @@ __global__ void k_list_spanning(const uint32_t* __restrict__ vscan, uint32_t nz,
     }
 }
 
+// ---------------------------------------------------------------- streamed Jacobi gather
+// The sync iteration as two kernels: k_pr_stream sums the contributions of every row of the
+// in-edge list, k_pr_finish turns the sums into ranks.
+//
+// What bounds a gather of c[src] over the in-edges is not HBM but the lines that each 4-byte
+// gather moves from the L2 to the CU (the K-lane pull: 0.82 line requests per edge).  In degree
+// order the first PS_HUBS vertices are the sources of most edges (57% on RMAT-22), so every
+// workgroup copies their contributions to LDS once (152 KB, one workgroup of 16 waves per CU)
+// and only the other sources are gathered from the L2: with half the hubs (76 KB, 44% of the
+// edges) a run was 13% slower.  Waves are independent: a wave takes tiles of 1024 edges, 16
+// consecutive edges per lane from a copy of the list laid out for 16-byte coalesced loads, sums
+// them in a register with a row-end bit per edge, and joins rows across lanes with one segmented
+// scan, so there is no staging of rows, no search and no barrier between tiles.  Issuing the
+// next tile's gathers before the current tile is summed (120 VGPRs) changed nothing: the
+// remaining gathers are bound by their lines, 145 G/s, not by latency.
+// Measured (PageRank to the 1e-7 stop on RMAT-22, 67 M edges, against the pull): 22.4 -> 14.2 ms,
+// an iteration 332 + 7.9 (fix-up) + 4.6 (residual) -> 198 + 23 us; personalised, 9.9 M edges over
+// 0.78 M vertices: 4.68 -> 2.85 ms.
+constexpr int PS_EPL = 16;               // edges per lane
+constexpr int PS_TILE = WAVE * PS_EPL;   // edges per wave tile
+constexpr int PS_WG = 1024;              // threads per workgroup: 16 waves, one workgroup per CU
+constexpr uint32_t PS_HUBS = 38912;      // contributions held in LDS
+// A contribution rounded to one float holds the ranks within a few ulps of their fixed point
+// (whatever stays inside its rounding interval is lost).  Where few vertices carry most of the
+// mass and the paths between them have a period (bipartite graphs, grids), the phases of the
+// iteration then settle at different points and the L1 change stays near 1e-7.  So:
+// - up to PS_PAIRS vertices contributions are (hi, lo) pairs, all of them in LDS (112 of 150
+//   random bipartite graphs of up to 10 vertices never met the 1e-7 stop with single floats, none
+//   with pairs);
+// - above, each contribution's rounding error is added to the vertex's next contribution while
+//   the L1 change is above PS_FEED, so that what is passed on is right on average; below it the
+//   errors are dropped, and the iteration settles on a fixed point for smaller stops.
+constexpr uint32_t PS_PAIRS = PS_HUBS / 2;
+constexpr double PS_FEED = 5e-8;
+constexpr uint32_t PS_PARTS = 2048;      // most workgroups of k_pr_finish (residual partials)
+// Lists above this size are read with nontemporal loads: one that fits the 256 MB Infinity Cache
+// beside the ranks is still there in the next iteration (us per iteration, cached / nontemporal:
+// 64 MiB 49.5 / 53.7, 128 MiB 94 / 104, 192 MiB 175.8 / 176.0, 256 MiB 227 / 219, 512 MiB 524 /
+// 504).
+constexpr uint64_t PS_STREAM_BYTES = 192ull << 20;
+
+struct StreamArgs {
+    const uint4* tcol;       // sources, tile by tile: [tile][4][lane] of 4 consecutive edges
+    const uint32_t* desc;    // per lane of a tile: row-end bits | row ends before it << 16
+    const uint32_t* tfirst;  // row (vlist position) of every tile's first edge
+    uint32_t ntiles;
+    uint32_t hubs;           // contributions in LDS: a multiple of 4, or every vertex (pairs)
+    const float* c_old;
+    float2* sums;            // per row: sum of its edges in the tile where it ends
+    float2* tail;            // per tile: sum of the row left open at its end
+    const double* parts;     // residual partials of the previous iteration
+    uint32_t nparts;
+    double eps;
+    Ctl* ctl;
+    uint32_t it;
+};
+
+// Residual of iteration a.it - 1 from its partials, in a fixed order (every workgroup gets the
+// same bits); sRed: PS_WG / WAVE entries.  Records it and returns whether the run has converged.
+__device__ __forceinline__ bool previous_converged(const StreamArgs& a, double* sRed) {
+    double t = 0;
+    for (uint32_t i = threadIdx.x; i < a.nparts; i += PS_WG) t += a.parts[i];
+    t = wave_sum(t);
+    if (lane_id() == 0) sRed[threadIdx.x / WAVE] = t;
+    __syncthreads();
+    double r = 0;
+    for (int i = 0; i < PS_WG / WAVE; ++i) r += sRed[i];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        a.ctl->residual[(a.it - 1) & 3] = r;
+        a.ctl->iters = a.it - 1;
+        if (r < a.eps) a.ctl->done = 1;
+    }
+    return r < a.eps;
+}
+
+__global__ __launch_bounds__(PS_WG) void k_pr_check(StreamArgs a) {
+    __shared__ double sRed[PS_WG / WAVE];
+    if (a.ctl->done) return;
+    (void)previous_converged(a, sRed);
+}
+
+// NT: the list is read past the caches (see PS_STREAM_BYTES).
+template <bool NT>
+__device__ __forceinline__ uint4 load_quad(const uint4* p) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const u32x4* q = reinterpret_cast<const u32x4*>(p);
+    u32x4 x;
+    if constexpr (NT) x = __builtin_nontemporal_load(q);
+    else x = *q;
+    return make_uint4(x.x, x.y, x.z, x.w);
+}
+
+template <bool NT, bool PAIR>
+__global__ __launch_bounds__(PS_WG) void k_pr_stream(StreamArgs a) {
+    __shared__ __attribute__((aligned(16))) float sHub[PS_HUBS];
+    __shared__ double sRed[PS_WG / WAVE];
+    if (a.ctl->done) return;
+    if (a.it > 1 && previous_converged(a, sRed)) return;
+    {
+        const float4* src = reinterpret_cast<const float4*>(a.c_old);
+        float4* dst = reinterpret_cast<float4*>(sHub);
+        const uint32_t quads = PAIR ? (a.hubs + 1) / 2 : a.hubs / 4;
+        for (uint32_t i = threadIdx.x; i < quads; i += PS_WG) dst[i] = src[i];
+    }
+    __syncthreads();
+    const uint32_t lane = (uint32_t)lane_id();
+    const uint32_t nw = gridDim.x * (PS_WG / WAVE);
+    // consecutive tiles go to different workgroups, so a remainder spreads over all CUs
+    uint32_t t = (threadIdx.x / WAVE) * gridDim.x + blockIdx.x;
+    if (t >= a.ntiles) return;
+    // the next tile's sources are loaded while the current tile's contributions arrive
+    uint4 q[PS_EPL / 4];
+#pragma unroll
+    for (int k = 0; k < PS_EPL / 4; ++k) q[k] = load_quad<NT>(a.tcol + ((uint64_t)t * (PS_EPL / 4) + k) * WAVE + lane);
+    uint32_t d = a.desc[(uint64_t)t * WAVE + lane];
+    while (true) {
+        float v[PS_EPL], vl[PS_EPL];  // vl: low words of pairs
+        // a hub's lane reads the hub from LDS and contribution 0 from memory (one shared line
+        // per wave, dropped); branch-free, so all 16 gathers are in flight
+#pragma unroll
+        for (int k = 0; k < PS_EPL / 4; ++k) {
+            const uint32_t u[4] = {q[k].x, q[k].y, q[k].z, q[k].w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                vl[4 * k + j] = 0.0f;
+                if constexpr (PAIR) {
+                    const float2 h = reinterpret_cast<const float2*>(sHub)[u[j]];
+                    v[4 * k + j] = h.x;
+                    vl[4 * k + j] = h.y;
+                    continue;
+                }
+                const bool hub = u[j] < a.hubs;
+                const float g = a.c_old[hub ? 0u : u[j]];
+                const float h = sHub[hub ? u[j] : 0u];
+                v[4 * k + j] = hub ? h : g;
+            }
+        }
+        const uint32_t ends = d & 0xffffu, row0 = a.tfirst[t] + (d >> 16);
+        const uint32_t cur = t;
+        t += nw;
+        if (t < a.ntiles) {
+#pragma unroll
+            for (int k = 0; k < PS_EPL / 4; ++k) q[k] = load_quad<NT>(a.tcol + ((uint64_t)t * (PS_EPL / 4) + k) * WAVE + lane);
+            d = a.desc[(uint64_t)t * WAVE + lane];
+        }
+        const uint64_t has = __ballot(ends != 0);
+        Comp acc{0.0f, 0.0f}, first{0.0f, 0.0f};
+        if (has == 0) {  // inside one row
+#pragma unroll
+            for (int j = 0; j < PS_EPL; ++j) acc = comp_add(acc, Comp{v[j], vl[j]});
+        } else {
+            uint32_t row = row0;
+#pragma unroll
+            for (int j = 0; j < PS_EPL; ++j) {
+                acc = comp_add(acc, Comp{v[j], vl[j]});
+                if ((ends >> j) & 1u) {
+                    if (row == row0) first = acc;  // waits for what earlier lanes hold of the row
+                    else a.sums[row] = make_float2(acc.s, acc.e);
+                    ++row;
+                    acc = Comp{0.0f, 0.0f};
+                }
+            }
+        }
+        // open sums scanned over the lanes since the last lane with a row end
+        const uint64_t upto = has & (lanemask_lt() | (1ull << lane));
+        const int from = upto ? 63 - __clzll((long long)upto) : 0;
+#pragma unroll
+        for (int off = 1; off < WAVE; off <<= 1) {
+            Comp o;
+            o.s = __shfl_up(acc.s, off, WAVE);
+            o.e = __shfl_up(acc.e, off, WAVE);
+            if ((int)lane - off >= from) acc = comp_add(o, acc);
+        }
+        Comp carry;
+        carry.s = __shfl_up(acc.s, 1, WAVE);
+        carry.e = __shfl_up(acc.e, 1, WAVE);
+        if (ends) {
+            if (lane) first = comp_add(carry, first);
+            a.sums[row0] = make_float2(first.s, first.e);
+        }
+        if (lane == WAVE - 1) a.tail[cur] = make_float2(acc.s, acc.e);
+        if (t >= a.ntiles) break;
+    }
+}
+
+constexpr uint32_t PS_SPANS = 0x80000000u;  // entry flag: the row crosses wave tiles
+
+struct FinishArgs {
+    PullArgs p;                 // rank buffers, degrees, teleport terms, in-edge rows
+    const uint32_t* ent;        // vertices with in-edges in vlist order | PS_SPANS
+    const float2* sums;
+    const float2* tail;
+    const uint32_t* span;       // rows crossing at most FIX_LONG tiles, then those crossing more
+    uint32_t nspan;
+    const uint32_t* span_long;
+    uint32_t nlong;
+    uint32_t n;
+    double* parts;
+    float* cerr;                // per vertex: rounding error of its last contribution (no pairs)
+};
+
+// Contribution x / d of a vertex of rank x = hi + lo and out-degree d.
+template <bool PAIR>
+__device__ __forceinline__ void store_contribution(const FinishArgs& f, uint32_t v, double x, uint32_t d, bool feed) {
+    if constexpr (PAIR) {
+        const double y = d ? x / (double)d : 0.0;
+        const float h = (float)y;
+        reinterpret_cast<float2*>(f.p.c_new)[v] = make_float2(h, (float)(y - (double)h));
+    } else {
+        double y = d ? x / (double)d : 0.0;
+        if (feed) y += (double)f.cerr[v];
+        const float h = (float)y;
+        f.p.c_new[v] = h;
+        f.cerr[v] = (float)(y - (double)h);
+    }
+}
+
+template <bool PAIR>
+__device__ __forceinline__ void finish_row(const FinishArgs& f, uint32_t v, Comp sum, bool feed, double& res) {
+    const PullArgs& a = f.p;
+    const double xo = (double)a.x_old[v] + (double)a.xl_old[v];
+    const uint32_t d = a.outdeg[v];
+    float hi, lo;
+    rank_pair_split(v == a.pers ? a.pers_base : a.base, a.damping, sum, &hi, &lo);
+    a.x_new[v] = hi;
+    a.xl_new[v] = lo;
+    const double x = (double)hi + (double)lo;
+    store_contribution<PAIR>(f, v, x, d, feed);
+    res += fabs(x - xo);
+}
+
+// Ranks from the row sums: a thread per row; rows that cross tiles add the tails of the tiles
+// they leave open in tile order (a wave per row when they are many: lane-strided, then a fixed
+// tree).  Streams ~44 B per row.  Vertices without in-edges hold their teleport term from the
+// first iteration on; the two buffers get it in iterations 1 and 2.
+template <bool PAIR>
+__global__ __launch_bounds__(WG) void k_pr_finish(FinishArgs f) {
+    __shared__ double sRed[WG / WAVE];
+    const PullArgs& a = f.p;
+    if (a.ctl->done) return;
+    // (the errors start at the second contribution; the residual of the iteration before is known)
+    const bool feed = !PAIR && a.it > 1 && a.ctl->residual[(a.it - 1) & 3] > PS_FEED;
+    double res = 0.0;
+    const uint32_t tid = blockIdx.x * WG + threadIdx.x, nt = gridDim.x * WG;
+    for (uint64_t i = tid; i < a.nz; i += nt) {
+        const uint32_t v = f.ent[i];
+        if (v & PS_SPANS) continue;
+        const float2 s = f.sums[i];
+        finish_row<PAIR>(f, v, Comp{s.x, s.y}, feed, res);
+    }
+    for (uint32_t i = tid; i < f.nspan; i += nt) {
+        const uint32_t pos = f.span[i], v = f.ent[pos] & ~PS_SPANS;
+        const uint32_t ta = (uint32_t)(a.row[v] / PS_TILE), tb = (uint32_t)((a.row[v + 1] - 1) / PS_TILE);
+        Comp acc{0.0f, 0.0f};
+        for (uint32_t t = ta; t < tb; ++t) acc = comp_add(acc, Comp{f.tail[t].x, f.tail[t].y});
+        acc = comp_add(acc, Comp{f.sums[pos].x, f.sums[pos].y});
+        finish_row<PAIR>(f, v, acc, feed, res);
+    }
+    const uint32_t lane = (uint32_t)lane_id();
+    for (uint32_t j = tid / WAVE; j < f.nlong; j += nt / WAVE) {
+        const uint32_t pos = f.span_long[j], v = f.ent[pos] & ~PS_SPANS;
+        const uint32_t ta = (uint32_t)(a.row[v] / PS_TILE), tb = (uint32_t)((a.row[v + 1] - 1) / PS_TILE);
+        Comp acc{0.0f, 0.0f};
+        for (uint32_t t = ta + lane; t < tb; t += WAVE) acc = comp_add(acc, Comp{f.tail[t].x, f.tail[t].y});
+#pragma unroll
+        for (int off = WAVE / 2; off > 0; off >>= 1) {
+            Comp o;
+            o.s = __shfl_down(acc.s, off, WAVE);
+            o.e = __shfl_down(acc.e, off, WAVE);
+            acc = comp_add(acc, o);
+        }
+        if (lane == 0) {
+            acc = comp_add(acc, Comp{f.sums[pos].x, f.sums[pos].y});
+            finish_row<PAIR>(f, v, acc, feed, res);
+        }
+    }
+    if (a.it <= 2) {
+        for (uint64_t v = tid; v < f.n; v += nt) {
+            if (a.row[v + 1] != a.row[v]) continue;
+            const float base = (v == a.pers) ? a.pers_base : a.base;
+            const double xo = (double)a.x_old[v] + (double)a.xl_old[v];
+            a.x_new[v] = base;
+            a.xl_new[v] = 0.0f;
+            store_contribution<PAIR>(f, (uint32_t)v, (double)base, a.outdeg[v], false);
+            res += fabs((double)base - xo);
+        }
+    }
+    res = wave_sum(res);
+    if (lane == 0) sRed[threadIdx.x / WAVE] = res;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0;
+        for (int i = 0; i < WG / WAVE; ++i) t += sRed[i];
+        f.parts[blockIdx.x] = t;
+    }
+}
+
+// Tables of k_pr_stream, from the in-edge CSR and its list of rows (vertices with in-edges).
+// desc starts as zeros; a row's last edge e sets bit e % 16 of its lane's word.
+__global__ void k_ps_rows(const uint64_t* __restrict__ row, const uint32_t* __restrict__ vlist, uint32_t nz,
+                          uint32_t* __restrict__ desc, uint32_t* __restrict__ ent, uint32_t* __restrict__ span,
+                          uint32_t cap, uint32_t* __restrict__ count) {
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nz;
+         i += (uint64_t)gridDim.x * blockDim.x) {
+        const uint32_t v = vlist[i];
+        const uint64_t last = row[v + 1] - 1;
+        atomicOr(&desc[last / PS_EPL], 1u << (last % PS_EPL));
+        const uint32_t ta = (uint32_t)(row[v] / PS_TILE), tb = (uint32_t)(last / PS_TILE);
+        ent[i] = v | (ta != tb ? PS_SPANS : 0u);
+        if (ta == tb) continue;
+        if (tb - ta + 1 > FIX_LONG) span[cap - 1 - atomicAdd(&count[1], 1u)] = (uint32_t)i;
+        else span[atomicAdd(&count[0], 1u)] = (uint32_t)i;
+    }
+}
+// Per tile: the row of its first edge, and row ends before each lane.  A wave per tile.
+__global__ __launch_bounds__(WG) void k_ps_tiles(const uint64_t* __restrict__ row, const uint32_t* __restrict__ vlist,
+                                                 uint32_t nz, uint32_t ntiles, uint32_t* __restrict__ desc,
+                                                 uint32_t* __restrict__ tfirst) {
+    const uint32_t lane = (uint32_t)lane_id();
+    const uint32_t nw = gridDim.x * (WG / WAVE);
+    for (uint32_t t = blockIdx.x * (WG / WAVE) + threadIdx.x / WAVE; t < ntiles; t += nw) {
+        const uint64_t o = (uint64_t)t * WAVE + lane;
+        const uint32_t ends = desc[o] & 0xffffu;
+        const uint32_t cnt = (uint32_t)__popc(ends);
+        desc[o] = ends | ((wave_incl_scan(cnt) - cnt) << 16);
+        if (lane == 0) {
+            const uint64_t e = (uint64_t)t * PS_TILE;
+            uint32_t lo = 0, hi = nz;  // last row that starts at or before e
+            while (hi - lo > 1) {
+                const uint32_t mid = lo + (hi - lo) / 2;
+                if (row[vlist[mid]] <= e) lo = mid; else hi = mid;
+            }
+            tfirst[t] = lo;
+        }
+    }
+}
+// out[tile][k][lane] = edges 4k .. 4k+3 of that lane's 16 (source 0 past the last edge)
+__global__ void k_ps_layout(const uint32_t* __restrict__ col, uint64_t m, uint64_t quads, uint4* __restrict__ out) {
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < quads;
+         i += (uint64_t)gridDim.x * blockDim.x) {
+        const uint64_t tile = i / (PS_TILE / 4), r = i % (PS_TILE / 4), k = r / WAVE, lane = r % WAVE;
+        const uint64_t e = tile * PS_TILE + lane * PS_EPL + 4 * k;
+        uint4 x = make_uint4(0, 0, 0, 0);
+        if (e + 4 <= m) {
+            x = *reinterpret_cast<const uint4*>(col + e);
+        } else {
+            if (e < m) x.x = col[e];
+            if (e + 1 < m) x.y = col[e + 1];
+            if (e + 2 < m) x.z = col[e + 2];
+        }
+        out[i] = x;
+    }
+}
+
 }  // namespace
 
-// Vertices of the in-edge Tigr table whose virtual nodes cross a pull tile, listed once per
-// graph and K (their partial sums are combined by k_pr_fix).  Called with the graph's lock held
-// or before concurrent queries start.
-eeg_status ensure_pr_span(eeg_graph* g, uint32_t K) {
+// Tables of the streamed gather, built once per graph (the rows do not depend on K).  Called
+// with the graph's lock held or before concurrent queries start, after ensure_tigr(in, K).
+// Leaves ps.built false where they do not fit in memory or vertex ids need 32 bits: the sync
+// variants then run the pull.
+static eeg_status ensure_pr_stream(eeg_graph* g, uint32_t K) {
+    PrStream& ps = g->prstream;
+    if (ps.built || ps.refused) return EEG_OK;
+    const Tigr& t = g->tin[k_index(K)];
+    const Csr& in = g->in;
+    ps.refused = true;
+    if (g->n >= PS_SPANS || t.nz == 0) return EEG_OK;
+    const uint64_t ntiles = (in.m + PS_TILE - 1) / PS_TILE;
+    const uint32_t cap = (uint32_t)ntiles + 1;
+    DevMem cnt;
+    if (ps.tcol.alloc(ntiles * PS_TILE * 4) != EEG_OK || ps.desc.alloc(ntiles * WAVE * 4) != EEG_OK ||
+        ps.tfirst.alloc(ntiles * 4) != EEG_OK || ps.ent.alloc((size_t)t.nz * 4) != EEG_OK ||
+        ps.span.alloc((size_t)cap * 4) != EEG_OK || cnt.alloc(8) != EEG_OK) {
+        clear_error();
+        for (DevMem* d : {&ps.tcol, &ps.desc, &ps.tfirst, &ps.ent, &ps.span}) d->release();
+        return EEG_OK;
+    }
+    hipStream_t s = g->stream;
+    auto grid = [](uint64_t work) { return (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(16384, (work + WG - 1) / WG)); };
+    EEG_HIP(hipMemsetAsync(ps.desc.p, 0, ntiles * WAVE * 4, s));
+    EEG_HIP(hipMemsetAsync(cnt.p, 0, 8, s));
+    k_ps_rows<<<grid(t.nz), WG, 0, s>>>(in.rowp(), t.vlist.as<uint32_t>(), t.nz, ps.desc.as<uint32_t>(),
+                                        ps.ent.as<uint32_t>(), ps.span.as<uint32_t>(), cap, cnt.as<uint32_t>());
+    k_ps_tiles<<<grid(ntiles * WAVE), WG, 0, s>>>(in.rowp(), t.vlist.as<uint32_t>(), t.nz, (uint32_t)ntiles,
+                                                  ps.desc.as<uint32_t>(), ps.tfirst.as<uint32_t>());
+    k_ps_layout<<<grid(ntiles * (PS_TILE / 4)), WG, 0, s>>>(in.colp(), in.m, ntiles * (PS_TILE / 4), ps.tcol.as<uint4>());
+    EEG_HIP(hipGetLastError());
+    uint32_t ns[2] = {0, 0};
+    EEG_HIP(hipMemcpyAsync(ns, cnt.p, 8, hipMemcpyDeviceToHost, s));
+    EEG_HIP(hipStreamSynchronize(s));
+    if ((uint64_t)ns[0] + ns[1] > cap) return fail(EEG_ERR_DEVICE, "PageRank span list overflow");
+    ps.nspan = ns[0];
+    ps.nlong = ns[1];
+    ps.span_cap = cap;
+    ps.ntiles = (uint32_t)ntiles;
+    ps.nz = t.nz;
+    ps.refused = false;
+    ps.built = true;
+    return EEG_OK;
+}
+
+// Tables of the PageRank gathers: the streamed one's, or where it is not available and for the
+// in-place sweeps the vertices of the in-edge Tigr table whose virtual nodes cross a pull tile,
+// listed once per graph and K (their partial sums are combined by k_pr_fix).  Called with the
+// graph's lock held or before concurrent queries start.
+eeg_status ensure_pr_span(eeg_graph* g, uint32_t K, bool inplace) {
     Tigr& t = g->tin[k_index(K)];
-    if (t.span_built) return EEG_OK;
     if (!g->outdeg.p) {  // out-degrees as u32, read by every PageRank iteration
         EEG_TRY(g->outdeg.alloc((size_t)g->n * 4 + 4));
         if (g->n) {
@@ -438,6 +842,11 @@ eeg_status ensure_pr_span(eeg_graph* g, uint32_t K) {
             EEG_HIP(hipGetLastError());
         }
     }
+    if (!inplace) {
+        EEG_TRY(ensure_pr_stream(g, K));
+        if (g->prstream.built) return EEG_OK;
+    }
+    if (t.span_built) return EEG_OK;
     const uint32_t TV = PR_TILE / K;
     const uint64_t ntiles = (t.P + TV - 1) / TV;
     hipStream_t s = g->stream;
@@ -485,20 +894,25 @@ eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_
     Work& w = wk ? *wk : g->work;
     EEG_TRY(ensure_in(g));
     EEG_TRY(ensure_tigr(g, g->in, g->tin, K));
+    EEG_TRY(ensure_pr_span(g, K, inplace));
     const Tigr& t = g->tin[k_index(K)];
+    const PrStream& ps = g->prstream;
+    const bool stream = !inplace && ps.built;
+    const bool pairs = stream && n <= PS_PAIRS;
     const uint32_t TV = PR_TILE / K;
-    const uint64_t ntiles = (t.P + TV - 1) / TV;
+    const uint64_t ntiles = stream ? ps.ntiles : (t.P + TV - 1) / TV;
 
     EEG_TRY(w.ctl.alloc(sizeof(Ctl)));
     if (!w.host_ctl) EEG_HIP(hipHostMalloc((void**)&w.host_ctl, 2 * sizeof(Ctl), hipHostMallocDefault));
     for (int i = 0; i < 2; ++i) {
         EEG_TRY(w.fx[i].alloc((size_t)n * 4 + 4));
-        EEG_TRY(w.fc[i].alloc((size_t)n * 4 + 4));
+        EEG_TRY(w.fc[i].alloc((size_t)n * (pairs ? 8 : 4) + 8));
         EEG_TRY(w.fl[i].alloc((size_t)n * 4 + 4));
     }
     EEG_TRY(w.spill.alloc((size_t)(ntiles + 1) * 2 * sizeof(float2)));
+    if (stream) EEG_TRY(w.psum.alloc((size_t)ps.nz * sizeof(float2)));
+    if (stream && !pairs) EEG_TRY(w.cerr.alloc((size_t)n * 4));
     // vertices whose virtual nodes cross a tile boundary (finished by k_pr_fix)
-    EEG_TRY(ensure_pr_span(g, K));
     const DevMem& span = t.span;
     const uint32_t nshort = t.nspan, nlong = t.nspan_long;
     const uint32_t nspan = nshort + nlong;
@@ -513,7 +927,14 @@ eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_
     const unsigned grid_pull = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(ntiles, (uint64_t)cus * wpc));
     const unsigned grid_fix = std::max(1u, std::min(1024u, std::max((nshort + WG - 1) / WG, (nlong + 3) / 4)));
     const unsigned grid_iso = std::max(1u, std::min(4096u, (n + WG - 1) / WG));
-    const uint32_t nparts = grid_pull + grid_fix + grid_iso;
+    // streamed gather: its LDS admits one workgroup of 1024 threads per CU, which keeps its hubs
+    // for all its tiles; a given wgs_per_cu counts 256-thread workgroups, so more take turns (a
+    // serving lane leaves gaps for others).  At least 4 tiles per workgroup, and no more hubs
+    // than the workgroup has edges, so copying them stays below what they save.
+    const unsigned grid_stream = (unsigned)std::max<uint64_t>(
+        1, std::min<uint64_t>((ntiles + 3) / 4, (uint64_t)cus * (o.wgs_per_cu ? (o.wgs_per_cu + 3) / 4 : 1)));
+    const unsigned grid_finish = std::max(1u, std::min(PS_PARTS, (n + WG - 1) / WG));
+    const uint32_t nparts = stream ? grid_finish : grid_pull + grid_fix + grid_iso;
     EEG_TRY(w.red.alloc((size_t)nparts * sizeof(double)));
     EEG_HIP(hipMemsetAsync(w.red.p, 0, (size_t)nparts * sizeof(double), s));
 
@@ -522,8 +943,8 @@ eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_
     const float x0 = 1.0f / (float)n;
     const float base = personalised ? 0.0f : (1.0f - d) / (float)n;
     const uint32_t pers = personalised ? source : 0xffffffffu;
-    k_pr_init<<<grid_iso, WG, 0, s>>>(g->outdeg.as<uint32_t>(), n, x0, pers, w.fx[0].as<float>(), w.fl[0].as<float>(),
-                                      w.fc[0].as<float>());
+    (pairs ? k_pr_init<true> : k_pr_init<false>)<<<grid_iso, WG, 0, s>>>(
+        g->outdeg.as<uint32_t>(), n, x0, pers, w.fx[0].as<float>(), w.fl[0].as<float>(), w.fc[0].as<float>());
     EEG_HIP(hipGetLastError());
 
     PullArgs pa{};
@@ -544,6 +965,33 @@ eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_
     pa.tstart = t.prstart.as<uint32_t>();
     double* red = w.red.as<double>();
     auto pull_fn = (K == 4) ? k_pr_pull<4> : (K == 8) ? k_pr_pull<8> : (K == 16) ? k_pr_pull<16> : k_pr_pull<32>;
+
+    const bool nontemporal = (uint64_t)ps.ntiles * PS_TILE * 4 > PS_STREAM_BYTES;
+    StreamArgs sa{};
+    FinishArgs fa{};
+    if (stream) {
+        sa.tcol = ps.tcol.as<uint4>();
+        sa.desc = ps.desc.as<uint32_t>();
+        sa.tfirst = ps.tfirst.as<uint32_t>();
+        sa.ntiles = ps.ntiles;
+        sa.hubs = pairs ? n : (uint32_t)std::min<uint64_t>(std::min(n, PS_HUBS), ntiles * PS_TILE / grid_stream) & ~3u;
+        sa.sums = w.psum.as<float2>();
+        sa.tail = w.spill.as<float2>();
+        sa.parts = red;
+        sa.nparts = nparts;
+        sa.eps = eps;
+        sa.ctl = ctl;
+        fa.ent = ps.ent.as<uint32_t>();
+        fa.sums = w.psum.as<float2>();
+        fa.tail = w.spill.as<float2>();
+        fa.span = ps.span.as<uint32_t>();
+        fa.nspan = ps.nspan;
+        fa.span_long = ps.span.as<uint32_t>() + (ps.span_cap - ps.nlong);
+        fa.nlong = ps.nlong;
+        fa.n = n;
+        fa.parts = red;
+        fa.cerr = w.cerr.as<float>();
+    }
 
     hipEvent_t ev_start;
     EEG_TRY(w.event(0, &ev_start));
@@ -567,27 +1015,36 @@ eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_
             EEG_TRY(w.event(2 * (size_t)it - 1, &eb));
             EEG_HIP(hipEventRecord(eb, s));
         }
-        if (t.P) {
+        if (stream) {
+            sa.c_old = pa.c_old;
+            sa.it = it;
+            (nontemporal ? (pairs ? k_pr_stream<true, true> : k_pr_stream<true, false>)
+                         : (pairs ? k_pr_stream<false, true> : k_pr_stream<false, false>))<<<grid_stream, PS_WG, 0, s>>>(sa);
+            fa.p = pa;
+            (pairs ? k_pr_finish<true> : k_pr_finish<false>)<<<grid_finish, WG, 0, s>>>(fa);
+            EEG_HIP(hipGetLastError());
+        } else if (t.P) {
             void* args[] = {&pa};
             EEG_HIP(hipLaunchKernel((const void*)pull_fn, dim3(grid_pull), dim3(WG), args, 0, s));
         } else {
             EEG_HIP(hipMemsetAsync(red, 0, grid_pull * sizeof(double), s));
         }
-        if (nspan) {
+        if (!stream && nspan) {
             k_pr_fix<<<grid_fix, WG, 0, s>>>(pa, span.as<uint32_t>(), nshort, span_long, nlong, TV,
                                              red + grid_pull);
             EEG_HIP(hipGetLastError());
         }
         const uint32_t iso_iters = inplace ? 1 : 2;  // vertices without in-edges settle at once
-        if (it <= iso_iters) {
+        if (!stream && it <= iso_iters) {
             k_pr_isolated<<<grid_iso, WG, 0, s>>>(g->in.rowp(), g->outdeg.as<uint32_t>(), n, pa.x_old, pa.xl_old,
                                                   pa.x_new, pa.xl_new, pa.c_new, base, pers, 1.0f - d,
                                                   red + grid_pull + grid_fix, ctl);
             EEG_HIP(hipGetLastError());
-        } else if (it == iso_iters + 1) {
+        } else if (!stream && it == iso_iters + 1) {
             EEG_HIP(hipMemsetAsync(red + grid_pull + grid_fix, 0, grid_iso * sizeof(double), s));
         }
-        k_pr_reduce<<<1, RED_WG, 0, s>>>(red, nparts, ctl, it, eps);
+        // (the streamed gather sums the residual at the start of the next iteration)
+        if (!stream) k_pr_reduce<<<1, RED_WG, 0, s>>>(red, nparts, ctl, it, eps);
         EEG_HIP(hipGetLastError());
         if (recorded.size() <= it) recorded.resize((size_t)it + 64, 0);
         recorded[it] = (rec || o.timing) ? 1 : 0;
@@ -599,7 +1056,7 @@ eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_
         (void)ea;
         return EEG_OK;
     };
-    if (!nspan) EEG_HIP(hipMemsetAsync(red + grid_pull, 0, grid_fix * sizeof(double), s));
+    if (!stream && !nspan) EEG_HIP(hipMemsetAsync(red + grid_pull, 0, grid_fix * sizeof(double), s));
 
     EEG_HIP(hipEventRecord(ev_start, s));
     uint32_t it = 1;
@@ -614,6 +1071,11 @@ eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_
             const uint32_t cnt = std::min<uint32_t>(chunk, max_iters + 1 - it);
             for (uint32_t k = 0; k < cnt; ++k, ++it)
                 EEG_TRY(launch(it, k + 1 == cnt || (predicted_end != 0xffffffffu && it + 2 >= predicted_end)));
+            if (stream) {
+                sa.it = it;
+                k_pr_check<<<1, PS_WG, 0, s>>>(sa);
+                EEG_HIP(hipGetLastError());
+            }
             EEG_HIP(hipMemcpyAsync(&w.host_ctl[slot], ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s));
             EEG_HIP(hipEventRecord(poll[slot], s));
             pending[slot] = true;
