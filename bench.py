@@ -400,7 +400,9 @@ def single_query_section(g, K):
             gbs = c["bytes_alg"] / (ms * 1e-3) / 1e9
             out[f"{alg}/{var}"] = {"ms": round(ms, 4), "gteps": round(m / ms / 1e6, 2),
                                    "iterations": c["iterations"], "alg_bytes": c["bytes_alg"],
-                                   "alg_gbs": round(gbs, 1), "hbm_frac": round(gbs / HBM_PEAK_GBS, 4)}
+                                   # CC is timed as union-find, its counted run propagates labels
+                                   "alg_gbs": round(gbs, 1) if alg != "cc" else None,
+                                   "hbm_frac": round(gbs / HBM_PEAK_GBS, 4) if alg != "cc" else None}
             log(f"single query rmat24 {alg}/{var}: {out[f'{alg}/{var}']}")
     return out
 
@@ -486,7 +488,8 @@ def grid_section(eg, a):
             _, st = g.run(alg, 0, variant=var, frontier=fr, K=a.K, want_labels=False)
             r[name] = {"ms": round(st["ms_traversal"], 3), "gteps": round(m / st["ms_traversal"] / 1e6, 2),
                        "iterations": st["iterations"], "alg_bytes": c["bytes_alg"],
-                       "hbm_frac": round(c["bytes_alg"] / (st["ms_traversal"] * 1e-3) / 8e12, 4)}
+                       "hbm_frac": round(c["bytes_alg"] / (st["ms_traversal"] * 1e-3) / 8e12, 4)
+                       if alg != "cc" or fr != "sorted" and var != "async_push_dd" else None}
         res[alg] = r
         log(f"grid {alg}: {r}")
     g.close()
@@ -667,14 +670,15 @@ def main():
                         "edges_relaxed": c["edges_relaxed"], "label_updates": c["label_updates"],
                         "alg_bytes": c["bytes_alg"],
                         "kernel_ms_avg": round(avg_launch_ms, 5),
-                        "alg_gbs": bytes_per_launch / avg_launch_ms / 1e6 if kn else None}
+                        # CC is timed as union-find, its counted run propagates labels
+                        "alg_gbs": bytes_per_launch / avg_launch_ms / 1e6 if kn and alg != "cc" else None}
         if alg == "pr":
             per_alg[key]["residual"] = sts[0]["pr_residual"]
         if kn and (best is None or ksum > best[0]):
             best = (ksum, alg, var, bytes_per_launch, avg_launch_ms, kn)
 
-    kernel_names = {"bfs": "k_relax<BFS>", "sssp": "k_relax<SSSP>", "sswp": "k_relax<SSWP>",
-                    "cc": "k_relax<CC>", "pr": "k_pr_pull+k_pr_fix+k_pr_reduce"}
+    kernel_names = {"bfs": "k_relax<BFS>", "sssp": "k_relax<SSSP>", "sswp": "k_relax<SSWP>", "cc": "k_cc_*",
+                    "pr": "k_pr_stream+k_pr_finish" if best and best[2].startswith("sync") else "k_pr_pull+k_pr_fix+k_pr_reduce"}
     roofline = None
     if best:
         _, alg, var, bpl, avg_ms, kn = best

@@ -222,6 +222,8 @@ eeg_status generate_rmat_device(uint32_t scale, uint32_t ef, double a, double b,
 eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_opts& o,
                          eeg_stats* st, const uint32_t* d_seeds = nullptr, uint32_t nseeds = 0,
                          Work* wk = nullptr, hipStream_t sk = nullptr);
+// CC labels by union-find (components.hip), into w.lab; run_traversal's answer.
+eeg_status run_components(eeg_graph* g, eeg_stats* st, Work& w, hipStream_t s);
 eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_opts& o,
                         eeg_stats* st, Work* wk = nullptr, hipStream_t sk = nullptr);
 

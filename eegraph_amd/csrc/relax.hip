@@ -733,14 +733,20 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
     const int alg = (int)algo;  // EEG_BFS..EEG_CC map onto A_BFS..A_CC
     if ((alg == A_SSSP || alg == A_SSWP) && !g->weighted)
         return fail(EEG_ERR_INVALID_ARG, "SSSP/SSWP need a weighted graph");
+    hipStream_t s = wk ? sk : g->stream;
+    Work& w = wk ? *wk : g->work;
+    // Components by union-find where only the labels are asked for: a run that counts, times or
+    // limits iterations, names a frontier kind other than the default or sweeps every virtual
+    // node propagates labels (device time of that against this: RMAT-22 1.9 / 0.21 ms,
+    // 4096^2 grid 29 / 2.6 ms)
+    if (alg == A_CC && (sorted || mode == M_ASYNC) && !o.collect_activity && !o.count_work && !o.timing && !o.max_iters)
+        return run_components(g, st, w, s);
     if (alg == A_CC) EEG_TRY(ensure_sym(g));
     Csr& c = (alg == A_CC) ? g->sym : g->out;
     Tigr* tt = (alg == A_CC) ? g->tsym : g->tout;
     EEG_TRY(ensure_tigr(g, c, tt, K));
     const Tigr& t = tt[k_index(K)];
     const uint32_t n = g->n;
-    hipStream_t s = wk ? sk : g->stream;
-    Work& w = wk ? *wk : g->work;
 
     EEG_TRY(w.lab.alloc((size_t)n * 4 + 4));
     EEG_TRY(w.ctl.alloc(sizeof(Ctl)));

@@ -61,6 +61,9 @@ typedef enum eeg_algo {
  *   SYNC_PUSH_TD  : same sweep as ASYNC_PUSH_TD (the reference differs only in thread order).
  *   SYNC_PUSH_DD  : frontier-synchronous: the current frontier is processed, improved vertices
  *                   form the next frontier (compacted queue, or per-vertex flags).
+ * CC in ASYNC_PUSH_DD and SYNC_PUSH_DD (default frontier) is answered by union-find, unless the
+ * run counts, times or limits iterations (count_work, collect_activity, timing, max_iters): then,
+ * and in the other variants, minimum labels are propagated.  The labels are the same.
  * For PR the sync variants run a Jacobi iteration with destination-owned compensated sums
  * (deterministic); the async variants run the same gather updating ranks in place.
  * Personalised PageRank runs the same gather with a one-hot restart at the source. */
