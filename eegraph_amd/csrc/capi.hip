@@ -28,9 +28,14 @@ eeg_status Work::poll_events() {
     return EEG_OK;
 }
 
-// Runs end with a stream synchronisation, so no record of these events is pending here.
+eeg_status Work::progress() {
+    if (!status) EEG_HIP(hipHostMalloc((void**)&status, sizeof(RunStatus), hipHostMallocMapped | hipHostMallocCoherent));
+    return EEG_OK;
+}
+
+// The owner has synchronised the stream: no record of these events is pending here.
 Work::~Work() {
-    for (auto& ge : graphs) (void)hipGraphExecDestroy(ge.exec);
+    if (status) (void)hipHostFree(status);
     for (auto e : events) (void)hipEventDestroy(e);
     for (auto e : poll)
         if (e) (void)hipEventDestroy(e);

@@ -115,6 +115,12 @@ struct PrStream {
     bool refused = false;  // no edges, 32-bit vertex ids, or no memory: not tried again
 };
 
+// What a traversal tells the host while it runs, in pinned memory: iteration started last << 8 |
+// state, and the device clock at the start of the first iteration and at the end.
+struct RunStatus {
+    unsigned long long word, t0, t1;
+};
+
 // Reusable per-graph traversal state (one query at a time per handle).
 struct Work {
     DevMem lab;         // u32[n] (or f32 ranks), internal vertex order
@@ -132,16 +138,8 @@ struct Work {
     DevMem cerr;        // PR: rounding errors of the contributions (streamed gather)
     DevMem red;         // PR: per-workgroup residual partials
     uint32_t epoch = 1; // iteration stamps already used on stamp/flag
-    DevMem devit;       // replayed iteration chunks: {iteration, stamp base}
-    // executable graphs of replayed iteration chunks, by the argument bytes they were built
-    // with (most recently used last, at most kGraphCache): queries that alternate algorithms
-    // on one handle reuse their graphs
-    struct GraphEntry {
-        std::vector<uint8_t> key;
-        hipGraphExec_t exec;
-    };
-    static constexpr size_t kGraphCache = 8;
-    std::vector<GraphEntry> graphs;
+    RunStatus* status = nullptr;  // pinned: progress of the running traversal (RunStatus)
+    eeg_status progress();        // makes it
     Ctl* host_ctl = nullptr;  // pinned mirrors of Ctl (two, for overlapped polling)
     std::vector<hipEvent_t> events;  // pool: one or two per launch
     eeg_status event(size_t i, hipEvent_t* out);

@@ -55,12 +55,7 @@ struct RelaxArgs {
     uint32_t it;        // 1-based iteration of this traversal
     uint32_t stampv;    // stamp value of this iteration
     uint32_t count_stats;
-    // Replayed graph (M_QUEUE): when dev_it is set, dev_it[0] is the iteration and dev_it[1]
-    // the stamp base, read from device memory; it, stampv, the control slots and the queue
-    // ping-pong are derived from them, so one captured chunk serves every later chunk and run.
-    const uint32_t* dev_it;
-    uint32_t it_off;              // replayed graph: this node's iteration is dev_it[0] + it_off
-    uint32_t *qa, *sa, *qb, *sb;  // queue buffers 0 and 1
+    RunStatus* status;  // pinned: progress for the host (null: the host reads ctl)
     // Tile skipping of the static sweeps (M_ASYNC; M_FLAGS except CC, whose flag scan measured
     // slower with it): an improvement of vertex u in iteration it stamps u's 64-vertex block
     // with tbase + it, and iteration it runs only the tiles whose entries cover a block stamped
@@ -74,24 +69,23 @@ struct RelaxArgs {
     uint32_t all_first;      // iteration 1 runs every tile (CC: every vertex starts active)
 };
 
+// Progress of a run as its iterations start, written to pinned memory by one thread.  The words
+// are independent (the host waits for each on its own), so relaxed stores do.
+enum RunState : uint32_t { RUN_GOING = 0, RUN_DONE = 1, RUN_ERROR = 2 };
+__device__ __forceinline__ void publish(RunStatus* st, const Ctl* ctl, uint32_t it, uint32_t state) {
+    if (!st) return;
+    const unsigned long long now = (unsigned long long)wall_clock64();
+    if (it == 1) __hip_atomic_store(&st->t0, now, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (state == RUN_DONE) __hip_atomic_store(&st->t1, now, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (ctl->err) state = RUN_ERROR;
+    __hip_atomic_store(&st->word, ((unsigned long long)it << 8) | state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // BS threads per workgroup (256, 512 or 1024): a tile keeps TILE_EDGES edge slots, so a larger
 // workgroup runs fewer rounds of one edge per lane.
 template <int ALG, int K, int MODE, int BS>
-__global__ __launch_bounds__(BS) void k_relax(RelaxArgs args) {
+__global__ __launch_bounds__(BS) void k_relax(RelaxArgs a) {
     using R = Rule<ALG>;
-    RelaxArgs a = args;
-    if (MODE == M_QUEUE && a.dev_it) {
-        const uint32_t it = *a.dev_it + a.it_off;
-        const bool odd = ((it - 1) & 1) != 0;  // input queue = buffer (it-1)&1
-        a.it = it;
-        a.stampv = a.dev_it[1] + it;
-        a.qslot_in = (int)((it - 1) % 3);
-        a.qslot_out = (int)(it % 3);
-        a.qin = odd ? a.qb : a.qa;
-        a.sin = odd ? a.sb : a.sa;
-        a.qout = odd ? a.qa : a.qb;
-        a.sout = odd ? a.sa : a.sb;
-    }
     constexpr int VPR = BS / K;             // virtual nodes per round
     constexpr int TV = TILE_EDGES / K;      // virtual nodes per tile
     constexpr int ROUNDS = TILE_EDGES / BS;
@@ -122,14 +116,21 @@ __global__ __launch_bounds__(BS) void k_relax(RelaxArgs args) {
     const bool lead = (blockIdx.x == 0 && threadIdx.x == 0);
     if (MODE == M_QUEUE) {
         if (nE == 0 || T == 0) {
-            if (lead) ctl->done = 1;
+            if (lead) {
+                ctl->done = 1;
+                publish(a.status, ctl, a.it, RUN_DONE);
+            }
             return;
         }
     } else if (a.it > 1 && ctl->changed[(a.it - 1) & 3] == 0) {
-        if (lead) ctl->done = 1;
+        if (lead) {
+            ctl->done = 1;
+            publish(a.status, ctl, a.it, RUN_DONE);
+        }
         return;
     }
     if (lead) {
+        publish(a.status, ctl, a.it, RUN_GOING);
         ctl->iters = a.it;
         if (MODE == M_QUEUE) ctl->qpack[(a.it + 1) % 3] = 0;
         else ctl->changed[(a.it + 1) & 3] = 0;
@@ -433,17 +434,11 @@ __global__ void k_tile_blocks(const uint32_t* __restrict__ vlist, const uint32_t
         tblk[t] = (uint64_t)(vlist[e0] >> 6) | ((uint64_t)(vlist[e1] >> 6) << 32);
     }
 }
-// Stamps the blocks of the seed vertices (or of `single` when seeds is null) with `val`.
-__global__ void k_mark_blocks(const uint32_t* __restrict__ seeds, uint32_t nseeds, uint32_t single,
+// Stamps the blocks of the seed vertices with `val`.
+__global__ void k_mark_blocks(const uint32_t* __restrict__ seeds, uint32_t nseeds,
                               uint32_t* __restrict__ vdirty, uint32_t val) {
-    const uint32_t cnt = seeds ? nseeds : 1u;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += gridDim.x * blockDim.x)
-        vdirty[(seeds ? seeds[i] : single) >> 6] = val;
-}
-
-// Advances the device iteration counter of a replayed chunk (one thread, vector store).
-__global__ void k_tick(uint32_t* it, uint32_t step) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *it += step;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nseeds; i += gridDim.x * blockDim.x)
+        vdirty[seeds[i] >> 6] = val;
 }
 
 __global__ void k_fill_u32(uint32_t* __restrict__ a, uint64_t n, uint32_t val) {
@@ -452,10 +447,9 @@ __global__ void k_fill_u32(uint32_t* __restrict__ a, uint64_t n, uint32_t val) {
         a[i] = val;
 }
 
-// Clears the control block and seeds the first frontier with `source` (when seed != 0).
-__global__ void k_init_ctl(Ctl* ctl, const uint64_t* row, uint32_t K, int seed, uint32_t source,
-                           uint32_t* q0, uint32_t* s0) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// Clears the control block and seeds the first frontier with `source` (when seed != 0); one thread.
+__device__ void init_ctl(Ctl* ctl, const uint64_t* row, uint32_t K, int seed, uint32_t source, uint32_t* q0,
+                         uint32_t* s0) {
     for (int i = 0; i < 3; ++i) ctl->qpack[i] = 0;
     for (int i = 0; i < 4; ++i) {
         ctl->changed[i] = 0;
@@ -473,6 +467,43 @@ __global__ void k_init_ctl(Ctl* ctl, const uint64_t* row, uint32_t K, int seed, 
             s0[0] = 0;
             ctl->qpack[0] = ((unsigned long long)((d + K - 1) / K) << 32) | 1ull;
         }
+    }
+}
+
+__global__ void k_init_ctl(Ctl* ctl, const uint64_t* row, uint32_t K, int seed, uint32_t source,
+                           uint32_t* q0, uint32_t* s0) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) init_ctl(ctl, row, K, seed, source, q0, s0);
+}
+
+// Everything a run starts from, in one launch: labels (as k_init_labels), control block and first
+// frontier, and one array cleared or filled (the bitmap of sorted frontiers, the labels last
+// pushed by virtual nodes, the flags of CC).
+struct InitArgs {
+    uint32_t* lab;
+    uint32_t n;
+    uint32_t fill, at_source, source;
+    const uint32_t* ids;
+    uint32_t* extra;
+    uint64_t nextra;
+    uint32_t extra_val;
+    uint32_t* one;  // one word set to one_val (a single source's flag or block stamp)
+    uint32_t one_val;
+    Ctl* ctl;
+    const uint64_t* row;
+    uint32_t K;
+    int seed;
+    uint32_t *q0, *s0;
+};
+__global__ void k_init_run(InitArgs a) {
+    const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, nt = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t v = tid; v < a.n; v += nt) {
+        const uint32_t x = (v == a.source) ? a.at_source : a.fill;
+        a.lab[v] = a.ids ? a.ids[v] : x;
+    }
+    for (uint64_t i = tid; i < a.nextra; i += nt) a.extra[i] = a.extra_val;
+    if (tid == 0) {
+        if (a.one) *a.one = a.one_val;
+        init_ctl(a.ctl, a.row, a.K, a.seed, a.source, a.q0, a.s0);
     }
 }
 
@@ -581,6 +612,13 @@ int cu_count(int device) {
     return c;
 }
 
+// Ticks of the device clock (wall_clock64) per millisecond.
+double clock_khz(int device) {
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) != hipSuccess || khz <= 0) khz = 100000;
+    return (double)khz;
+}
+
 }  // namespace
 
 // Memory the traversal state needs beyond the graph (used by admission control too).
@@ -612,102 +650,16 @@ eeg_status ensure_tiles(Tigr& t, uint32_t K, hipStream_t s) {
     return EEG_OK;
 }
 
-// Iterations per replayed chunk: a multiple of 2 (queue ping-pong) and 3 (control slots), so
-// every replay starts in the same state pattern.
-constexpr uint32_t GRAPH_CHUNK = 6;
+// Iterations queued beyond the one that the device is known to have started: enough that it never
+// waits for the host (an iteration takes 9 us or more, seeing it start and queueing the next about
+// 8), and what is left to run dry after the last one is short.
+constexpr uint32_t RUN_AHEAD = 2;
 
-// The executable graph of one chunk for these kernel arguments (buffers, grid, kernel): built
-// on first use and kept in the work state with the last few others, so queries that
-// alternate algorithms reuse theirs.  It holds kernel nodes only.
-eeg_status chunk_graph(Work& w, KernelFn kfn, unsigned grid, unsigned block, const RelaxArgs& ga, hipStream_t s,
-                       hipGraphExec_t* out, const CompactArgs* ca = nullptr, unsigned grid_c = 0) {
-    const size_t kc = ca ? sizeof(CompactArgs) + sizeof(grid_c) : 0;
-    std::vector<uint8_t> key(sizeof(RelaxArgs) + sizeof(kfn) + sizeof(grid) + sizeof(block) + kc);
-    memcpy(key.data(), &ga, sizeof(RelaxArgs));
-    memcpy(key.data() + sizeof(RelaxArgs), &kfn, sizeof(kfn));
-    memcpy(key.data() + sizeof(RelaxArgs) + sizeof(kfn), &grid, sizeof(grid));
-    memcpy(key.data() + sizeof(RelaxArgs) + sizeof(kfn) + sizeof(grid), &block, sizeof(block));
-    if (ca) {
-        uint8_t* kp = key.data() + sizeof(RelaxArgs) + sizeof(kfn) + sizeof(grid) + sizeof(block);
-        memcpy(kp, ca, sizeof(CompactArgs));
-        memcpy(kp + sizeof(CompactArgs), &grid_c, sizeof(grid_c));
-    }
-    for (size_t i = 0; i < w.graphs.size(); ++i) {
-        if (w.graphs[i].key == key) {
-            Work::GraphEntry hit = std::move(w.graphs[i]);
-            w.graphs.erase(w.graphs.begin() + (long)i);
-            w.graphs.push_back(std::move(hit));
-            *out = w.graphs.back().exec;
-            return EEG_OK;
-        }
-    }
-    if (w.graphs.size() >= Work::kGraphCache) {  // every earlier run has finished on its stream
-        (void)hipGraphExecDestroy(w.graphs.front().exec);
-        w.graphs.erase(w.graphs.begin());
-    }
-    // built node by node (no stream capture, which would interact with other threads'
-    // HIP calls): GRAPH_CHUNK relaxations in one dependency chain, node i running iteration
-    // dev_it[0] + i (each followed by its frontier compaction for sorted frontiers), then one
-    // tick that advances dev_it[0] by GRAPH_CHUNK
-    hipGraph_t graph = nullptr;
-    EEG_HIP(hipGraphCreate(&graph, 0));
-    RelaxArgs a = ga;
-    uint32_t* itp = const_cast<uint32_t*>(ga.dev_it);
-    void* rargs[] = {&a};
-    hipError_t e = hipSuccess;
-    hipGraphNode_t prev = nullptr;
-    for (uint32_t i = 0; i < GRAPH_CHUNK && e == hipSuccess; ++i) {
-        a.it_off = i;  // the node keeps its own copy of the arguments
-        hipKernelNodeParams kp{};
-        kp.func = (void*)kfn;
-        kp.gridDim = dim3(grid);
-        kp.blockDim = dim3(block);
-        kp.sharedMemBytes = 0;
-        kp.kernelParams = rargs;
-        kp.extra = nullptr;
-        hipGraphNode_t nr = nullptr;
-        e = hipGraphAddKernelNode(&nr, graph, prev ? &prev : nullptr, prev ? 1 : 0, &kp);
-        prev = nr;
-        if (ca && e == hipSuccess) {
-            CompactArgs cx = *ca;
-            cx.it_off = i;
-            void* cargs[] = {&cx};
-            hipKernelNodeParams cp{};
-            cp.func = (void*)k_compact_frontier;
-            cp.gridDim = dim3(grid_c);
-            cp.blockDim = dim3(WG);
-            cp.sharedMemBytes = 0;
-            cp.kernelParams = cargs;
-            cp.extra = nullptr;
-            hipGraphNode_t nc = nullptr;
-            e = hipGraphAddKernelNode(&nc, graph, &prev, 1, &cp);
-            prev = nc;
-        }
-    }
-    uint32_t step = GRAPH_CHUNK;
-    void* targs[] = {&itp, &step};
-    if (e == hipSuccess) {
-        hipKernelNodeParams tp{};
-        tp.func = (void*)k_tick;
-        tp.gridDim = dim3(1);
-        tp.blockDim = dim3(64);
-        tp.sharedMemBytes = 0;
-        tp.kernelParams = targs;
-        tp.extra = nullptr;
-        hipGraphNode_t nt = nullptr;
-        e = hipGraphAddKernelNode(&nt, graph, &prev, 1, &tp);
-    }
-    if (e != hipSuccess) {
-        (void)hipGraphDestroy(graph);
-        return fail(EEG_ERR_DEVICE, "building the iteration chunk failed: %s", hipGetErrorString(e));
-    }
-    hipGraphExec_t exec = nullptr;
-    e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(graph);
-    if (e != hipSuccess) return fail(EEG_ERR_DEVICE, "hipGraphInstantiate failed: %s", hipGetErrorString(e));
-    w.graphs.push_back(Work::GraphEntry{std::move(key), exec});
-    *out = exec;
-    return EEG_OK;
+// Iterations launched for a limit of max_iters (>= 1): the fixpoint must be seen among them.  Whole
+// chunks, of 6 after the first iteration for queues, of 2, 4, 8, 8, ... for sweeps.
+uint64_t launch_limit(bool queue, uint64_t max_iters) {
+    if (queue) return max_iters < 8 ? 7 : 1 + 6 * ((max_iters - 2) / 6 + 1);
+    return max_iters < 7 ? 6 : 6 + 8 * ((max_iters + 1) / 8);
 }
 
 }  // namespace
@@ -750,7 +702,7 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
 
     EEG_TRY(w.lab.alloc((size_t)n * 4 + 4));
     EEG_TRY(w.ctl.alloc(sizeof(Ctl)));
-    if (!w.host_ctl) EEG_HIP(hipHostMalloc((void**)&w.host_ctl, 2 * sizeof(Ctl), hipHostMallocDefault));
+    EEG_TRY(w.progress());
     if (mode == M_QUEUE) {
         for (int i = 0; i < 2; ++i) {
             EEG_TRY(w.q[i].alloc((size_t)n * 4 + 4));
@@ -761,11 +713,8 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
     const uint32_t nwords = (n + 31) / 32;
     if (sorted) {
         EEG_TRY(w.bitmap.alloc((size_t)nwords * 4 + 4));
-        // a run that stopped early (error, iteration limit) may have left bits behind
-        k_fill_u32<<<grid_for(nwords, 8192), WG, 0, s>>>(w.bitmap.as<uint32_t>(), nwords, 0u);
-        EEG_HIP(hipGetLastError());
     }
-    if (mode == M_QUEUE && !w.stamp.p) {
+    if (mode == M_QUEUE && !sorted && !w.stamp.p) {
         EEG_TRY(w.stamp.alloc((size_t)n * 4 + 4));
         EEG_HIP(hipMemsetAsync(w.stamp.p, 0, w.stamp.bytes, s));
     }
@@ -791,49 +740,64 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
     }
     if (mode == M_ASYNC) EEG_TRY(w.vnpush.alloc((size_t)t.P * 4 + 4));
 
-    // ---- labels and control block
-    {
-        const uint32_t fill = (alg == A_SSWP) ? 0u : INF;
-        const uint32_t at_src = (alg == A_SSWP) ? INF : 0u;
-        k_init_labels<<<grid_for(n, 8192), WG, 0, s>>>(w.lab.as<uint32_t>(), n, fill, at_src,
-                                                       d_seeds ? 0xffffffffu : source,
-                                                       alg == A_CC ? g->inv.as<uint32_t>() : nullptr);
-        if (d_seeds && alg != A_CC && nseeds)
-            k_seed_labels<<<grid_for(nseeds, 1024), WG, 0, s>>>(w.lab.as<uint32_t>(), d_seeds, nseeds, at_src);
-    }
-    EEG_HIP(hipGetLastError());
-    if (mode == M_ASYNC) {
-        const uint32_t never = (alg == A_SSWP) ? 0u : 0xffffffffu;
-        k_fill_u32<<<grid_for(t.P, 8192), WG, 0, s>>>(w.vnpush.as<uint32_t>(), t.P, never);
-        EEG_HIP(hipGetLastError());
-    }
+    // ---- labels, control block and first frontier
     const uint32_t base = w.epoch;  // iteration it uses stamp base + it
     const bool seeded = (alg != A_CC);
-    if (skip && seeded) {  // the first sweep starts from the seeds' blocks
-        const uint32_t cnt = d_seeds ? nseeds : 1u;
-        k_mark_blocks<<<std::max(1u, std::min(1024u, (cnt + WG - 1) / WG)), WG, 0, s>>>(
-            d_seeds, nseeds, source, w.vdirty.as<uint32_t>(), base);
-        EEG_HIP(hipGetLastError());
-    }
     Ctl* ctl = w.ctl.as<Ctl>();
-    k_init_ctl<<<1, 64, 0, s>>>(ctl, c.rowp(), K, (seeded && mode == M_QUEUE && !d_seeds) ? 1 : 0, source,
-                                mode == M_QUEUE ? w.q[0].as<uint32_t>() : nullptr,
-                                mode == M_QUEUE ? w.s[0].as<uint32_t>() : nullptr);
-    EEG_HIP(hipGetLastError());
-    if (seeded && mode == M_QUEUE && d_seeds && nseeds) {
-        k_seed_queue<<<1, WG, 0, s>>>(ctl, c.rowp(), K, d_seeds, nseeds, w.q[0].as<uint32_t>(),
-                                      w.s[0].as<uint32_t>());
-        EEG_HIP(hipGetLastError());
-    }
-    if (mode == M_FLAGS) {
-        if (seeded && d_seeds) {
-            if (nseeds) k_seed_flags<<<grid_for(nseeds, 1024), WG, 0, s>>>(w.flag.as<uint32_t>(), d_seeds, nseeds, base + 1);
-        } else if (seeded) {
-            k_fill_u32<<<1, 64, 0, s>>>(w.flag.as<uint32_t>() + source, 1, base + 1);
-        } else {
-            k_fill_u32<<<grid_for(n, 8192), WG, 0, s>>>(w.flag.as<uint32_t>(), n, base + 1);
+    {
+        const uint32_t at_src = (alg == A_SSWP) ? INF : 0u;
+        InitArgs ia{};
+        ia.lab = w.lab.as<uint32_t>();
+        ia.n = n;
+        ia.fill = (alg == A_SSWP) ? 0u : INF;
+        ia.at_source = at_src;
+        ia.source = d_seeds ? 0xffffffffu : source;
+        ia.ids = alg == A_CC ? g->inv.as<uint32_t>() : nullptr;
+        if (sorted) {  // a run that stopped early (error, iteration limit) may have left bits behind
+            ia.extra = w.bitmap.as<uint32_t>();
+            ia.nextra = nwords;
+        } else if (mode == M_ASYNC) {
+            ia.extra = w.vnpush.as<uint32_t>();
+            ia.nextra = t.P;
+            ia.extra_val = (alg == A_SSWP) ? 0u : 0xffffffffu;  // never pushed
+        } else if (mode == M_FLAGS && !seeded) {
+            ia.extra = w.flag.as<uint32_t>();
+            ia.nextra = n;
+            ia.extra_val = base + 1;
         }
+        if (seeded && !d_seeds) {
+            if (mode == M_FLAGS) {
+                ia.one = w.flag.as<uint32_t>() + source;
+                ia.one_val = base + 1;
+            } else if (skip) {  // the first sweep starts from the seed's block
+                ia.one = w.vdirty.as<uint32_t>() + (source >> 6);
+                ia.one_val = base;
+            }
+        }
+        ia.ctl = ctl;
+        ia.row = c.rowp();
+        ia.K = K;
+        ia.seed = (seeded && mode == M_QUEUE && !d_seeds) ? 1 : 0;
+        ia.source = d_seeds ? 0xffffffffu : source;
+        if (mode == M_QUEUE) {
+            ia.q0 = w.q[0].as<uint32_t>();
+            ia.s0 = w.s[0].as<uint32_t>();
+        }
+        k_init_run<<<grid_for(std::max<uint64_t>(n, ia.nextra), 8192), WG, 0, s>>>(ia);
         EEG_HIP(hipGetLastError());
+        const unsigned gs = std::max(1u, std::min(1024u, (nseeds + WG - 1) / WG));
+        if (seeded && !d_seeds && skip && mode == M_FLAGS) {
+            k_fill_u32<<<1, 64, 0, s>>>(w.vdirty.as<uint32_t>() + (source >> 6), 1, base);
+            EEG_HIP(hipGetLastError());
+        }
+        if (seeded && d_seeds && nseeds) {
+            k_seed_labels<<<gs, WG, 0, s>>>(w.lab.as<uint32_t>(), d_seeds, nseeds, at_src);
+            if (skip) k_mark_blocks<<<gs, WG, 0, s>>>(d_seeds, nseeds, w.vdirty.as<uint32_t>(), base);
+            if (mode == M_QUEUE)
+                k_seed_queue<<<1, WG, 0, s>>>(ctl, c.rowp(), K, d_seeds, nseeds, w.q[0].as<uint32_t>(), w.s[0].as<uint32_t>());
+            if (mode == M_FLAGS) k_seed_flags<<<gs, WG, 0, s>>>(w.flag.as<uint32_t>(), d_seeds, nseeds, base + 1);
+            EEG_HIP(hipGetLastError());
+        }
     }
 
     // ---- launch geometry: a resident grid that walks tiles
@@ -864,6 +828,7 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
     ra.vnpush = w.vnpush.as<uint32_t>();
     ra.bitmap = sorted ? w.bitmap.as<uint32_t>() : nullptr;
     ra.ctl = ctl;
+    ra.status = w.status;
     ra.cap_out = n;
     ra.n_static = t.nz;
     ra.P_static = (uint32_t)t.P;
@@ -892,10 +857,7 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
         grid_c = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(((uint64_t)nwords + WG - 1) / WG, (uint64_t)cus * 4));
     }
 
-    // Event pool: per launch L (it = L+1) an "after" event at 2L+1 and, with timing, a
-    // "before" event at 2L; event 0 of the pool tail marks the traversal start.
-    hipEvent_t ev_start;
-    EEG_TRY(w.event(0, &ev_start));
+    // with timing, an event before (2 it - 1) and after (2 it) every launch
     auto launch = [&](uint32_t it) -> eeg_status {
         ra.it = it;
         ra.stampv = base + it;
@@ -931,15 +893,22 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
             void* cargs[] = {&ca};
             EEG_HIP(hipLaunchKernel((const void*)k_compact_frontier, dim3(grid_c), dim3(WG), cargs, 0, s));
         }
-        EEG_TRY(w.event(2 * (size_t)it, &ea));
-        EEG_HIP(hipEventRecord(ea, s));
+        if (o.timing) {
+            EEG_TRY(w.event(2 * (size_t)it, &ea));
+            EEG_HIP(hipEventRecord(ea, s));
+        }
         return EEG_OK;
     };
 
-    EEG_HIP(hipEventRecord(ev_start, s));
+    // (nothing of an earlier run writes the status any more: a run ends when its last status is
+    // seen, or with its stream synchronised)
+    volatile RunStatus* vs = w.status;
+    vs->word = 0;
+    vs->t0 = 0;
+    vs->t1 = 0;
     uint32_t it = 1;
     eeg_status rc = EEG_OK;
-    uint32_t graph_launches = 0;  // nonzero: the replayed-graph path ran
+    Ctl hc{};
     std::vector<uint32_t> activity;
     if (o.collect_activity) {
         // One launch at a time so every iteration's activity can be read back (the reference's
@@ -949,6 +918,7 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
         unsigned long long upd_before = 0;
         while (true) {
             EEG_TRY(launch(it));
+            if (!w.host_ctl) EEG_HIP(hipHostMalloc((void**)&w.host_ctl, 2 * sizeof(Ctl), hipHostMallocDefault));
             EEG_HIP(hipMemcpyAsync(w.host_ctl, ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s));
             EEG_HIP(hipStreamSynchronize(s));
             const Ctl& h = w.host_ctl[0];
@@ -961,111 +931,54 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
                 break;
             }
         }
-    } else if (mode == M_QUEUE && !o.timing) {
-        // Iteration 1 eagerly (it may read the static entry list), then a graph of GRAPH_CHUNK
-        // iterations (relaxation + counter tick each) replayed until the control block reports
-        // done.  The next replay is queued before the previous one's control
-        // block is inspected.
-        EEG_TRY(launch(1));
-        it = 2;
-        EEG_TRY(w.devit.alloc(8));
-        uint32_t* dit = w.devit.as<uint32_t>();
-        k_fill_u32<<<1, 64, 0, s>>>(dit, 1, 2u);
-        k_fill_u32<<<1, 64, 0, s>>>(dit + 1, 1, base);
-        EEG_HIP(hipGetLastError());
-        RelaxArgs ga = ra;
-        ga.it = 0;
-        ga.stampv = 0;
-        ga.qslot_in = 0;
-        ga.qslot_out = 0;
-        ga.qin = ga.sin = nullptr;
-        ga.qout = ga.sout = nullptr;
-        ga.dev_it = dit;
-        ga.qa = w.q[0].as<uint32_t>();
-        ga.sa = w.s[0].as<uint32_t>();
-        ga.qb = w.q[1].as<uint32_t>();
-        ga.sb = w.s[1].as<uint32_t>();
-        hipGraphExec_t exec = nullptr;
-        CompactArgs gca = ca;
-        gca.it = 0;
-        gca.dev_it = dit;
-        EEG_TRY(chunk_graph(w, kfn, grid_queue, block, ga, s, &exec, sorted ? &gca : nullptr, grid_c));
-        EEG_TRY(w.poll_events());
-        hipEvent_t* poll = w.poll;
-        uint32_t replays = 0;
-        auto submit = [&](int slot) -> eeg_status {
-            EEG_HIP(hipGraphLaunch(exec, s));
-            ++replays;
-            it += GRAPH_CHUNK;
-            hipEvent_t er;
-            EEG_TRY(w.event(2 + replays, &er));
-            EEG_HIP(hipEventRecord(er, s));
-            EEG_HIP(hipMemcpyAsync(&w.host_ctl[slot], ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s));
-            EEG_HIP(hipEventRecord(poll[slot], s));
-            return EEG_OK;
-        };
-        int cur = 0;
-        rc = submit(0);
-        while (rc == EEG_OK) {
-            if (it <= max_iters + GRAPH_CHUNK) rc = submit(cur ^ 1);
-            if (rc != EEG_OK) break;
-            EEG_HIP(hipEventSynchronize(poll[cur]));
-            const Ctl& h = w.host_ctl[cur];
-            if (h.err || h.done) break;
-            if (it > max_iters + GRAPH_CHUNK) {
-                rc = fail(EEG_ERR_NOT_CONVERGED, "no fixpoint after %u iterations", max_iters);
-                break;
-            }
-            cur ^= 1;
-        }
-        graph_launches = 1 + replays * GRAPH_CHUNK;
+        hc = w.host_ctl[0];
     } else {
-        // Chunks of launches; the next chunk is queued before the previous chunk's control
-        // block is inspected, so the GPU never waits for the host between chunks.
-        uint32_t chunk = 2;
-        EEG_TRY(w.poll_events());
-        hipEvent_t* poll = w.poll;
-        auto submit = [&](int slot) -> eeg_status {
-            for (uint32_t k = 0; k < chunk; ++k, ++it) EEG_TRY(launch(it));
-            EEG_HIP(hipMemcpyAsync(&w.host_ctl[slot], ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s));
-            EEG_HIP(hipEventRecord(poll[slot], s));
-            chunk = std::min<uint32_t>(chunk * 2, 8);
-            return EEG_OK;
-        };
-        int cur = 0;
-        rc = submit(0);
-        while (rc == EEG_OK) {
-            if (it <= max_iters + 8) rc = submit(cur ^ 1);
-            if (rc != EEG_OK) break;
-            EEG_HIP(hipEventSynchronize(poll[cur]));
-            const Ctl& h = w.host_ctl[cur];
-            if (h.err || h.done) break;
-            if (it > max_iters + 8) {
-                rc = fail(EEG_ERR_NOT_CONVERGED, "no fixpoint after %u iterations", max_iters);
-                break;
+        // The device reports each iteration as it starts; the host keeps RUN_AHEAD iterations
+        // queued beyond it and stops with the one that finds nothing to do.  (Replayed graphs of
+        // six iterations, polled by copies of the control block, ran up to 12 launches of ~4.5 us
+        // past the end and took ~0.3 ms to instantiate: RMAT-14 SSSP 360 -> 240 us a call, RMAT-22
+        // BFS 855 -> 753, first call 1189 -> 987; in-place SSWP, whose launches had events
+        // between them, 1624 -> 1445.)
+        const uint64_t limit = launch_limit(mode == M_QUEUE, max_iters);
+        uint32_t state = RUN_GOING;
+        uint64_t started = 0;
+        for (uint32_t spins = 1;; ++spins) {
+            while (it <= limit && it <= started + RUN_AHEAD) EEG_TRY(launch(it++));
+            const unsigned long long word = vs->word;
+            state = (uint32_t)(word & 0xff);
+            if (state != RUN_GOING) break;
+            if (word >> 8 != started) {
+                started = word >> 8;
+                spins = 0;
+                continue;
             }
-            cur ^= 1;
+            if ((spins & 0x3fff) == 0) {  // a device error ends the wait; so does the last iteration
+                const hipError_t e = hipStreamQuery(s);
+                if (e == hipSuccess && it > limit && vs->word == word) break;
+                if (e != hipSuccess && e != hipErrorNotReady)
+                    return fail(EEG_ERR_DEVICE, "traversal failed: %s", hipGetErrorString(e));
+            }
+            __builtin_ia32_pause();
+        }
+        if (state == RUN_DONE && !ra.count_stats) {
+            hc.done = 1;
+            hc.iters = (uint32_t)(vs->word >> 8) - 1;
+        } else {
+            EEG_HIP(hipStreamSynchronize(s));
+            EEG_HIP(hipMemcpy(&hc, ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+            if (!hc.done && !hc.err)
+                rc = fail(EEG_ERR_NOT_CONVERGED, "no fixpoint after %u iterations", max_iters);
         }
     }
-    EEG_HIP(hipStreamSynchronize(s));
-    EEG_HIP(hipMemcpy(w.host_ctl, ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
-    const Ctl hc = w.host_ctl[0];
     if (rc == EEG_OK && hc.err) rc = fail(EEG_ERR_DEVICE, "frontier queue overflow (err=%u)", hc.err);
-    if (rc == EEG_OK && !hc.done) rc = fail(EEG_ERR_NOT_CONVERGED, "no fixpoint after %u iterations", max_iters);
     w.epoch = base + it + 2;
 
     if (st) {
-        // end of the last working iteration: its launch, or the replay that contains it
-        hipEvent_t ev_end;
-        if (graph_launches && hc.iters > 1)
-            EEG_TRY(w.event(2 + (hc.iters - 1 + GRAPH_CHUNK - 1) / GRAPH_CHUNK, &ev_end));
-        else
-            EEG_TRY(w.event(2 * (size_t)std::max<uint32_t>(hc.iters, 1), &ev_end));
-        float ms = 0;
-        EEG_HIP(hipEventElapsedTime(&ms, ev_start, ev_end));
+        // device clock from the start of the first iteration to the one that found nothing to do
+        while (hc.done && !vs->t1) __builtin_ia32_pause();
         st->iterations = hc.iters;
-        st->launches = graph_launches ? graph_launches : it - 1;
-        st->ms_traversal = ms;
+        st->launches = it - 1;
+        st->ms_traversal = hc.done ? (double)(vs->t1 - vs->t0) / clock_khz(g->device) : 0.0;
         st->edges_relaxed = hc.stat[2];
         st->vnodes_processed = hc.stat[1];
         st->vertices_touched = hc.stat[0];
@@ -1079,6 +992,7 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
         double ksum = 0;
         uint32_t kn = 0;
         if (o.timing) {
+            EEG_HIP(hipStreamSynchronize(s));
             for (uint32_t i = 1; i <= hc.iters; ++i) {
                 hipEvent_t eb, ea;
                 EEG_TRY(w.event(2 * (size_t)i - 1, &eb));

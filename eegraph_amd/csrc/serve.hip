@@ -175,7 +175,9 @@ struct Lane {
     std::shared_ptr<BatchWork> bw;  // multi-source passes of this lane (made on first use)
     std::thread th;
     ~Lane() {
-        if (st) (void)hipStreamDestroy(st);
+        if (!st) return;
+        (void)hipStreamSynchronize(st);
+        (void)hipStreamDestroy(st);
     }
 };
 
