@@ -82,8 +82,8 @@ struct PlaneArgs {
     int widest;           // 0: SSSP (min, +w), 1: SSWP (max, min(.,w))
     const uint32_t* dev_it;  // replayed graph, as in MsArgs
     uint32_t *qa, *sa, *qb, *sb;
-    uint32_t* bitmap;     // dense passes of eeg_run_batch: improved vertices set their bit and
-                          // k_compact_frontier builds the next queue in vertex order (null: the
+    uint8_t* mark;        // dense passes of eeg_run_batch: improved vertices are marked and
+    uint8_t* cmark;       // k_compact_frontier builds the next queue in vertex order (null: the
                           // push appends to the queue itself)
     uint64_t* ovq;        // 8-bit distance passes: W words, queries to answer again wider
 };

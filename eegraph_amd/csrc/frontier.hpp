@@ -1,6 +1,11 @@
 // Sorted frontier queues, shared by the single-query traversals (relax.hip) and the batched
-// plane passes (batch.hip): a kernel that improved a vertex sets its bit in a 1-bit-per-vertex
-// bitmap, and k_compact_frontier turns the bits into the next queue in vertex order.
+// plane passes (batch.hip): a kernel that improved a vertex marks it (a byte per vertex and a byte
+// per 16384 vertices), and k_compact_frontier turns the marks into the next queue in vertex order.
+//
+// Marks are bytes written by plain stores because atomics are performed past the L2 at about 24 G/s
+// whatever they do: as bits set with atomicOr they were half of the atomics of a traversal
+// (SSSP on the 4096^2 grid: relaxations 8.0 -> 5.3 ms).  The byte per chunk lets thin frontiers skip
+// the rest: a compaction reads n / 16384 bytes and the chunks that were touched.
 #pragma once
 
 #include "device.hpp"
@@ -8,13 +13,35 @@
 namespace eeg {
 namespace {
 
-// Sorted frontier: the vertices whose bit iteration `it` set, with out-edges, as the next
-// queue (buffer it & 1, Ctl slot it % 3), in ascending id order within each block's 8192-vertex
-// chunk; chunks take their queue ranges in the order their atomic lands.  Bits are cleared as
-// they are read.  One thread per 32-bit word; replayed graphs resolve `it` from dev_it.
+// Threads and vertices of one workgroup's compaction step.  Each step ends in one atomicAdd on the
+// same word, which takes its turn for about 12 ns: with 256 threads the 2048 of a 16.8 M vertex
+// graph took 20 us more than these 1024 (thin frontiers over the whole 4096^2 grid: 32 -> 24 us).
+constexpr int COMPACT_WG = 1024;
+constexpr int COMPACT_PER = 16;  // vertices per thread
+constexpr uint32_t MARK_CHUNK = COMPACT_PER * COMPACT_WG;
+
+inline uint32_t mark_chunks(uint32_t n) { return (uint32_t)(((uint64_t)n + MARK_CHUNK - 1) / MARK_CHUNK); }
+// one allocation: the vertices' bytes (whole chunks), then the chunks' bytes, as whole words
+inline size_t mark_bytes(uint32_t n) {
+    const size_t c = mark_chunks(n);
+    return c * MARK_CHUNK + (c + 3) / 4 * 4;
+}
+inline uint8_t* chunk_marks(void* marks, uint32_t n) {
+    return static_cast<uint8_t*>(marks) + (size_t)mark_chunks(n) * MARK_CHUNK;
+}
+
+__device__ __forceinline__ void set_mark(uint8_t* mark, uint8_t* cmark, uint32_t u) {
+    mark[u] = 1;
+    cmark[u / MARK_CHUNK] = 1;
+}
+
+// Sorted frontier: the vertices that iteration `it` marked, with out-edges, as the next queue
+// (buffer it & 1, Ctl slot it % 3), in ascending id order within each block's 16384-vertex
+// chunk; chunks take their queue ranges in the order their atomic lands.  Marks are cleared as
+// they are read.  One thread per 16 vertices; replayed graphs resolve `it` from dev_it.
 struct CompactArgs {
-    uint32_t* bitmap;
-    uint32_t nwords;
+    uint8_t* mark;
+    uint8_t* cmark;
     uint32_t n;
     const uint32_t* vnc;
     Ctl* ctl;
@@ -25,29 +52,35 @@ struct CompactArgs {
     uint32_t it_off;
 };
 
-__global__ __launch_bounds__(WG) void k_compact_frontier(CompactArgs a) {
+// four bytes of 0 or 1 -> four bits
+__device__ __forceinline__ uint32_t mark_bits(uint32_t x) { return (x * 0x10204080u) >> 28; }
+
+__global__ __launch_bounds__(COMPACT_WG) void k_compact_frontier(CompactArgs a) {
     const uint32_t it = a.dev_it ? *a.dev_it + a.it_off : a.it;
     Ctl* ctl = a.ctl;
     if (ctl->done) return;
     uint32_t* qout = (it & 1u) ? a.qb : a.qa;
     uint32_t* sout = (it & 1u) ? a.sb : a.sa;
     const int slot = (int)(it % 3u);
-    __shared__ uint64_t sScan[WG / WAVE + 1];
+    __shared__ uint64_t sScan[COMPACT_WG / WAVE + 1];
     __shared__ uint32_t sBase[2];
-    for (uint32_t c0 = blockIdx.x * WG; c0 < a.nwords; c0 += gridDim.x * WG) {
-        const uint32_t wi = c0 + threadIdx.x;
-        const uint32_t word = wi < a.nwords ? a.bitmap[wi] : 0u;
-        if (!__syncthreads_or(word != 0u)) continue;  // the same answer in every thread
-        // the word's 32 virtual-node counts, read once: one 128-byte line as 8 vector loads
-        // (a last word past n reads only the counts that exist)
-        uint32_t cv[32];
+    const uint32_t chunks = (uint32_t)(((uint64_t)a.n + MARK_CHUNK - 1) / MARK_CHUNK);
+    for (uint32_t c = blockIdx.x; c < chunks; c += gridDim.x) {
+        if (!__syncthreads_or(a.cmark[c] != 0)) continue;  // the same answer in every thread
+        if (threadIdx.x == 0) a.cmark[c] = 0;              // read by every thread above
+        const uint32_t v0 = c * MARK_CHUNK + threadIdx.x * COMPACT_PER;
+        uint4* mp = reinterpret_cast<uint4*>(a.mark + v0);
+        const uint4 m = *mp;
+        const uint32_t word = mark_bits(m.x) | mark_bits(m.y) << 4 | mark_bits(m.z) << 8 | mark_bits(m.w) << 12;
+        // the virtual-node counts, read once as vector loads (the last vertices read only the
+        // counts that exist)
+        uint32_t cv[COMPACT_PER];
         if (word) {
-            a.bitmap[wi] = 0u;
-            const uint32_t v0 = wi * 32u;
-            if (v0 + 32u <= a.n) {
+            *mp = make_uint4(0, 0, 0, 0);
+            if (v0 + COMPACT_PER <= a.n) {
                 const uint4* p = reinterpret_cast<const uint4*>(a.vnc + v0);
 #pragma unroll
-                for (int k = 0; k < 8; ++k) {
+                for (int k = 0; k < COMPACT_PER / 4; ++k) {
                     const uint4 x = p[k];
                     cv[4 * k] = x.x;
                     cv[4 * k + 1] = x.y;
@@ -56,21 +89,21 @@ __global__ __launch_bounds__(WG) void k_compact_frontier(CompactArgs a) {
                 }
             } else {
 #pragma unroll
-                for (int b = 0; b < 32; ++b) cv[b] = (v0 + (uint32_t)b < a.n) ? a.vnc[v0 + b] : 0u;
+                for (int b = 0; b < COMPACT_PER; ++b) cv[b] = (v0 + (uint32_t)b < a.n) ? a.vnc[v0 + b] : 0u;
             }
         } else {
 #pragma unroll
-            for (int b = 0; b < 32; ++b) cv[b] = 0u;
+            for (int b = 0; b < COMPACT_PER; ++b) cv[b] = 0u;
         }
         uint32_t cnt = 0, vs = 0;
 #pragma unroll
-        for (int b = 0; b < 32; ++b) {
+        for (int b = 0; b < COMPACT_PER; ++b) {
             const bool on = ((word >> b) & 1u) && cv[b];
             cnt += on ? 1u : 0u;
             vs += on ? cv[b] : 0u;
         }
         uint64_t tot;
-        const uint64_t pre = block_excl_scan<uint64_t>(((uint64_t)vs << 32) | cnt, sScan, &tot);
+        const uint64_t pre = block_excl_scan<uint64_t, COMPACT_WG>(((uint64_t)vs << 32) | cnt, sScan, &tot);
         if (threadIdx.x == 0) {
             const unsigned long long old = tot ? atomicAdd(&ctl->qpack[slot], (unsigned long long)tot) : 0ull;
             sBase[0] = (uint32_t)(old & 0xffffffffull);
@@ -80,11 +113,11 @@ __global__ __launch_bounds__(WG) void k_compact_frontier(CompactArgs a) {
         uint32_t e = sBase[0] + (uint32_t)(pre & 0xffffffffull);
         uint32_t vv = sBase[1] + (uint32_t)(pre >> 32);
 #pragma unroll
-        for (int b = 0; b < 32; ++b) {
+        for (int b = 0; b < COMPACT_PER; ++b) {
             // vertices without out-edges are left out: their labels are final, nothing to push
             if (!((word >> b) & 1u) || !cv[b]) continue;
             if (e < a.cap) {
-                qout[e] = wi * 32u + (uint32_t)b;
+                qout[e] = v0 + (uint32_t)b;
                 sout[e] = vv;
             } else {
                 atomicOr(&ctl->err, 2u);

@@ -44,8 +44,8 @@ struct RelaxArgs {
     uint32_t* stamp;
     uint32_t* flag;
     uint32_t* vnpush;
-    uint32_t* bitmap;   // sorted frontiers (M_QUEUE): improved vertices set their bit here and
-                        // k_compact_frontier builds the next queue; null: queued by the kernel
+    uint8_t* mark;      // sorted frontiers (M_QUEUE): improved vertices are marked and
+    uint8_t* cmark;     // k_compact_frontier builds the next queue; null: queued by the kernel
     Ctl* ctl;
     uint32_t n_static;  // entries / vnodes when qslot_in < 0
     uint32_t P_static;
@@ -288,15 +288,15 @@ __global__ __launch_bounds__(BS) void k_relax(RelaxArgs a) {
             }
             // Phase 4: frontier bookkeeping.  The queue needs each improved vertex's
             // virtual-node count and a dedup stamp; both are issued for all rounds first.
-            // Sorted frontiers only set the vertex's bit (an OR whose old value nobody waits
-            // for); counts, dedup and order come from k_compact_frontier.
+            // Sorted frontiers only mark the vertex; counts, dedup and order come from
+            // k_compact_frontier.
             uint32_t env[ROUNDS];
             if constexpr (MODE == M_QUEUE) {
-                if (a.bitmap) {
+                if (a.mark) {
 #pragma unroll
                     for (int r = 0; r < ROUNDS; ++r) {
                         env[r] = 0u;
-                        if (eu[r]) atomicOr(&a.bitmap[ed[r] >> 5], 1u << (ed[r] & 31u));
+                        if (eu[r]) set_mark(a.mark, a.cmark, ed[r]);
                     }
                 } else {
 #pragma unroll
@@ -476,7 +476,7 @@ __global__ void k_init_ctl(Ctl* ctl, const uint64_t* row, uint32_t K, int seed, 
 }
 
 // Everything a run starts from, in one launch: labels (as k_init_labels), control block and first
-// frontier, and one array cleared or filled (the bitmap of sorted frontiers, the labels last
+// frontier, and one array cleared or filled (the marks of sorted frontiers, the labels last
 // pushed by virtual nodes, the flags of CC).
 struct InitArgs {
     uint32_t* lab;
@@ -621,15 +621,6 @@ double clock_khz(int device) {
 
 }  // namespace
 
-// Memory the traversal state needs beyond the graph (used by admission control too).
-size_t traversal_state_bytes(uint32_t n, uint64_t P, int mode) {
-    size_t b = (size_t)n * 4 + sizeof(Ctl);
-    if (mode == M_QUEUE) b += (size_t)n * 4 * 5 + ((size_t)n + 31) / 32 * 4;  // queues, stamps, bitmap
-    if (mode == M_FLAGS) b += (size_t)n * 4;
-    if (mode == M_ASYNC) b += (size_t)P * 4;
-    return b;
-}
-
 namespace {
 
 // Tile tables of a Tigr layout for the static sweeps (built once per graph and K).
@@ -710,9 +701,9 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
         }
     }
     const uint32_t max_iters = o.max_iters ? o.max_iters : (n + 2);
-    const uint32_t nwords = (n + 31) / 32;
     if (sorted) {
-        EEG_TRY(w.bitmap.alloc((size_t)nwords * 4 + 4));
+        if (w.mark.bytes < mark_bytes(n)) w.marks_clear = false;
+        EEG_TRY(w.mark.alloc(mark_bytes(n)));
     }
     if (mode == M_QUEUE && !sorted && !w.stamp.p) {
         EEG_TRY(w.stamp.alloc((size_t)n * 4 + 4));
@@ -753,9 +744,14 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
         ia.at_source = at_src;
         ia.source = d_seeds ? 0xffffffffu : source;
         ia.ids = alg == A_CC ? g->inv.as<uint32_t>() : nullptr;
-        if (sorted) {  // a run that stopped early (error, iteration limit) may have left bits behind
-            ia.extra = w.bitmap.as<uint32_t>();
-            ia.nextra = nwords;
+        if (sorted) {
+            // a finished run has cleared its marks; one that stopped early (error, iteration
+            // limit) may have left some behind
+            if (!w.marks_clear) {
+                ia.extra = w.mark.as<uint32_t>();
+                ia.nextra = mark_bytes(n) / 4;
+            }
+            w.marks_clear = false;
         } else if (mode == M_ASYNC) {
             ia.extra = w.vnpush.as<uint32_t>();
             ia.nextra = t.P;
@@ -826,7 +822,8 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
     ra.stamp = w.stamp.as<uint32_t>();
     ra.flag = w.flag.as<uint32_t>();
     ra.vnpush = w.vnpush.as<uint32_t>();
-    ra.bitmap = sorted ? w.bitmap.as<uint32_t>() : nullptr;
+    ra.mark = sorted ? w.mark.as<uint8_t>() : nullptr;
+    ra.cmark = sorted ? chunk_marks(w.mark.p, n) : nullptr;
     ra.ctl = ctl;
     ra.status = w.status;
     ra.cap_out = n;
@@ -844,8 +841,8 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
     CompactArgs ca{};
     unsigned grid_c = 1;
     if (sorted) {
-        ca.bitmap = w.bitmap.as<uint32_t>();
-        ca.nwords = nwords;
+        ca.mark = ra.mark;
+        ca.cmark = ra.cmark;
         ca.n = n;
         ca.vnc = t.vnc.as<uint32_t>();
         ca.ctl = ctl;
@@ -854,7 +851,7 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
         ca.qb = w.q[1].as<uint32_t>();
         ca.sb = w.s[1].as<uint32_t>();
         ca.cap = n;
-        grid_c = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(((uint64_t)nwords + WG - 1) / WG, (uint64_t)cus * 4));
+        grid_c = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(mark_chunks(n), (uint64_t)cus * 4));
     }
 
     // with timing, an event before (2 it - 1) and after (2 it) every launch
@@ -891,7 +888,7 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
         if (sorted) {
             ca.it = it;
             void* cargs[] = {&ca};
-            EEG_HIP(hipLaunchKernel((const void*)k_compact_frontier, dim3(grid_c), dim3(WG), cargs, 0, s));
+            EEG_HIP(hipLaunchKernel((const void*)k_compact_frontier, dim3(grid_c), dim3(COMPACT_WG), cargs, 0, s));
         }
         if (o.timing) {
             EEG_TRY(w.event(2 * (size_t)it, &ea));
@@ -972,6 +969,7 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
     }
     if (rc == EEG_OK && hc.err) rc = fail(EEG_ERR_DEVICE, "frontier queue overflow (err=%u)", hc.err);
     w.epoch = base + it + 2;
+    if (sorted && hc.done && !hc.err) w.marks_clear = true;
 
     if (st) {
         // device clock from the start of the first iteration to the one that found nothing to do
@@ -1035,7 +1033,7 @@ eeg_status run_traversal_fixed(eeg_graph* g, uint32_t algo, uint32_t source, con
         case EEG_ASYNC_PUSH_TD:
         case EEG_SYNC_PUSH_TD: mode = M_TD; break;
         case EEG_SYNC_PUSH_DD:
-            // sorted frontiers keep a bitmap: the compact queue stands in (same answers)
+            // sorted frontiers keep marks: the compact queue stands in (same answers)
             if (o.frontier == EEG_FRONTIER_FLAGS)
                 return fail(EEG_ERR_UNSUPPORTED, "flag-scan frontiers are not available without allocation");
             if (o.frontier > EEG_FRONTIER_COMPACT)
