@@ -20,6 +20,7 @@
 #include "batch.hpp"
 #include "bytes8.hpp"
 #include "frontier.hpp"
+#include "hostcopy.hpp"
 
 namespace eeg {
 namespace {
@@ -918,25 +919,45 @@ __global__ void k_plane_rotate(const uint32_t* q, const Ctl* ctl, int slot,
         atomicOr((unsigned long long*)&act[threadIdx.x], sAct[threadIdx.x]);
 }
 
-// out[q * n + u] = planes[perm[u] * B + q0 + q]: answers of queries q0 .. q0+nq-1 in
-// query-major, original vertex order, narrow labels widened (their all-ones INF to INF)
-__global__ void k_planes_out(const uint32_t* __restrict__ planes, const uint32_t* __restrict__ perm,
-                             uint32_t n, uint32_t B, uint32_t q0, uint32_t nq, int lm, uint32_t* __restrict__ out) {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < (uint64_t)n * nq;
-         i += (uint64_t)gridDim.x * blockDim.x) {
-        const uint32_t q = (uint32_t)(i / n), u = (uint32_t)(i % n);
-        const uint64_t j = (uint64_t)perm[u] * B + q0 + q;
-        uint32_t x;
-        if (lm == LM_W8 || lm == LM_D8) {
-            x = reinterpret_cast<const uint8_t*>(planes)[j];
-            if (x == 0xffu) x = INF;
-        } else if (lm == LM_D16) {
-            x = reinterpret_cast<const uint16_t*>(planes)[j];
-            if (x == 0xffffu) x = INF;
-        } else {
-            x = planes[j];
+// out[q * stride + i] = planes[perm[i] * B + q] for q < nq, i < count: answers in query-major,
+// original vertex order, narrow labels widened (their all-ones INF to INF).
+//
+// Bound by memory traffic: a vertex's labels are one contiguous row and a query's answers are
+// another, so a tile of 64 vertices x 64 queries goes through LDS and both sides move whole lines
+// (each lane taking one label from its own vertex's row read every line up to 32 times: 256 answers
+// of 2^18 vertices in 1.31 ms).  The answers usually go over PCIe, to pinned memory.
+constexpr uint32_t OUT_TILE = 64;
+template <int LM>
+__global__ __launch_bounds__(WG) void k_planes_out(const uint32_t* __restrict__ planes,
+                                                   const uint32_t* __restrict__ perm, uint32_t count, uint32_t B,
+                                                   uint32_t nq, uint64_t stride, uint32_t* __restrict__ out) {
+    constexpr uint32_t QPL = (LM == LM_W8 || LM == LM_D8) ? 4 : LM == LM_D16 ? 2 : 1;  // labels per word
+    constexpr uint32_t WORDS = OUT_TILE / QPL;                                         // words per vertex
+    __shared__ uint32_t sL[OUT_TILE][OUT_TILE + 1];  // [query][vertex]
+    const uint32_t q0 = blockIdx.y * OUT_TILE;
+    for (uint32_t u0 = blockIdx.x * OUT_TILE; u0 < count; u0 += gridDim.x * OUT_TILE) {
+        const uint32_t nu = min(OUT_TILE, count - u0);
+        for (uint32_t i = threadIdx.x; i < nu * WORDS; i += WG) {
+            const uint32_t u = i / WORDS, wd = i % WORDS;
+            // q0 and B are multiples of 64: whole words, within the vertex's row
+            const uint32_t x = planes[((uint64_t)perm[u0 + u] * B + q0) / QPL + wd];
+            if constexpr (QPL == 1) {
+                sL[wd][u] = x;
+            } else {
+                constexpr uint32_t BITS = 32 / QPL, ONES = (1u << BITS) - 1;
+#pragma unroll
+                for (uint32_t k = 0; k < QPL; ++k) {
+                    const uint32_t l = (x >> (k * BITS)) & ONES;
+                    sL[wd * QPL + k][u] = l == ONES ? INF : l;
+                }
+            }
         }
-        out[i] = x;
+        __syncthreads();
+        const uint32_t u = threadIdx.x % OUT_TILE;
+        if (u < nu)
+            for (uint32_t q = threadIdx.x / OUT_TILE; q < OUT_TILE && q0 + q < nq; q += WG / OUT_TILE)
+                out[(uint64_t)(q0 + q) * stride + u0 + u] = sL[q][u];
+        __syncthreads();
     }
 }
 // Largest edge weight (atomicMax into *out, zeroed by the caller).
@@ -1105,7 +1126,7 @@ struct BatchWork {
     DevMem mark;            // dense plane passes: vertices improved this iteration (frontier.hpp)
     int64_t wmax = -1;      // largest edge weight of the graph (-1: not measured yet)
     DevMem ovq;             // 8-bit SSSP passes: queries whose distances outgrew 8 bits
-    DevMem rowbuf;          // one answer (n words) on its way to a host row
+    DevMem rowbuf;          // small answers on their way to the host (below HOST_COPY_FROM)
     bool d8_off = false;    // a previous 8-bit SSSP pass flagged more than a quarter of its queries
     DevMem q[2], s[2], cand, stamp, seeds, ctl;
     DevMem devit;           // replayed chunks: {iteration, stamp base}
@@ -1533,29 +1554,51 @@ eeg_status batch_pass(eeg_graph* g, BatchWork& bw, hipStream_t s, uint32_t algo,
         if (lm == LM_D8) EEG_HIP(hipMemcpyAsync(ovq_out, bw.ovq.p, MAXW * 8, hipMemcpyDeviceToHost, s));
     }
     // answers: query-major, original vertex order
-    const uint64_t outn = (uint64_t)nsrc * n;
-    if (bo.out) {
-        uint32_t* dst = nullptr;
-        DevMem tmp;
-        if (bo.device) {
-            dst = (uint32_t*)bo.out;
-        } else {
-            EEG_TRY(tmp.alloc(outn * 4 + 4));
-            dst = tmp.as<uint32_t>();
-        }
-        k_planes_out<<<grid_n(outn, 65536), WG, 0, s>>>(bw.planes.as<uint32_t>(), g->perm.as<uint32_t>(), n, B, 0u,
-                                                        nsrc, lm, dst);
+    auto planes_out = [&](uint32_t u0, uint32_t count, uint64_t stride, uint32_t* dst) -> eeg_status {
+        const dim3 gr(std::max(1u, std::min(4096u, (count + OUT_TILE - 1) / OUT_TILE)), W);
+        const uint32_t* pl = bw.planes.as<uint32_t>();
+        const uint32_t* pm = g->perm.as<uint32_t>() + u0;
+        if (lm == LM_W8) k_planes_out<LM_W8><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, stride, dst);
+        else if (lm == LM_D8) k_planes_out<LM_D8><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, stride, dst);
+        else if (lm == LM_D16) k_planes_out<LM_D16><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, stride, dst);
+        else k_planes_out<LM_U32><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, stride, dst);
         EEG_HIP(hipGetLastError());
-        if (!bo.device) EEG_HIP(hipMemcpyAsync(bo.out, dst, outn * 4, hipMemcpyDeviceToHost, s));
-        EEG_HIP(hipStreamSynchronize(s));
-    } else if (bo.rows) {  // one row at a time through one device row
-        EEG_TRY(bw.rowbuf.alloc((size_t)n * 4 + 4));
-        for (uint32_t q = 0; q < nsrc; ++q) {
-            if (!bo.rows[q]) continue;
-            k_planes_out<<<grid_n(n, 65536), WG, 0, s>>>(bw.planes.as<uint32_t>(), g->perm.as<uint32_t>(), n, B, q, 1u,
-                                                         lm, bw.rowbuf.as<uint32_t>());
-            EEG_HIP(hipGetLastError());
-            EEG_HIP(hipMemcpyAsync(bo.rows[q], bw.rowbuf.p, (size_t)n * 4, hipMemcpyDeviceToHost, s));
+        return EEG_OK;
+    };
+    if (bo.out && bo.device) {
+        EEG_TRY(planes_out(0, n, n, (uint32_t*)bo.out));
+    } else if (bo.out || bo.rows) {
+        auto row = [&](uint32_t q) { return bo.rows ? bo.rows[q] : (uint32_t*)bo.out + (uint64_t)q * n; };
+        const uint64_t bytes = (uint64_t)nsrc * n * 4;
+        LentRing lent(g->device, bytes >= HOST_COPY_FROM);
+        if (lent.r) {
+            // a slot holds the same vertices of every query; a thread copies its own queries, or with
+            // fewer queries than threads its own slots (the first to touch a page pays for it)
+            const uint32_t per = (uint32_t)(HOST_SLOT_BYTES / 4 / nsrc / OUT_TILE * OUT_TILE);
+            const uint32_t chunks = (uint32_t)(((uint64_t)n + per - 1) / per);
+            const unsigned threads = host_copy_threads(bytes);
+            auto part = [&](uint32_t i) { return std::min(per, n - i * per); };
+            EEG_TRY(stage_to_host(
+                *lent.r, s, chunks, threads, nsrc < threads,
+                [&](uint32_t i, void* slot) { return planes_out(i * per, part(i), part(i), (uint32_t*)slot); },
+                [&](uint32_t i, const void* slot, unsigned w, unsigned nw) {
+                    const uint32_t cnt = part(i);
+                    const uint32_t qa = (uint32_t)((uint64_t)w * nsrc / nw), qb = (uint32_t)((uint64_t)(w + 1) * nsrc / nw);
+                    for (uint32_t q = qa; q < qb; ++q)
+                        if (uint32_t* dst = row(q))
+                            memcpy(dst + (size_t)i * per, (const uint32_t*)slot + (size_t)q * cnt, (size_t)cnt * 4);
+                }));
+        } else {
+            EEG_TRY(bw.rowbuf.alloc(bytes + 4));
+            EEG_TRY(planes_out(0, n, n, bw.rowbuf.as<uint32_t>()));
+            if (bo.out) {
+                EEG_HIP(hipMemcpyAsync(bo.out, bw.rowbuf.p, bytes, hipMemcpyDeviceToHost, s));
+            } else {
+                for (uint32_t q = 0; q < nsrc; ++q)
+                    if (bo.rows[q])
+                        EEG_HIP(hipMemcpyAsync(bo.rows[q], bw.rowbuf.as<uint32_t>() + (size_t)q * n, (size_t)n * 4,
+                                               hipMemcpyDeviceToHost, s));
+            }
             EEG_HIP(hipStreamSynchronize(s));
         }
     }
@@ -1650,7 +1693,7 @@ eeg_status run_batch_core(eeg_graph* g, BatchWork& bw, Work* wk, hipStream_t s, 
                     void* hdst = bo.rows ? (void*)bo.rows[qs[i]]
                                          : bo.out ? (void*)((uint8_t*)bo.out + (uint64_t)qs[i] * row) : nullptr;
                     if (!hdst) continue;
-                    EEG_TRY(unpermute(g, w.lab.p, host ? bw.rowbuf.p : hdst, s));
+                    EEG_TRY(unpermute(g, w.lab.p, host ? bw.rowbuf.p : hdst, s, 0, n));
                     if (host) EEG_HIP(hipMemcpyAsync(hdst, bw.rowbuf.p, row, hipMemcpyDeviceToHost, s));
                     EEG_HIP(hipStreamSynchronize(s));
                 }

@@ -92,7 +92,7 @@ __global__ void k_relabel(const uint32_t* __restrict__ perm, const uint32_t* __r
         bo[i] = perm[b[i]];
     }
 }
-// out[u] = in[perm[u]]: results of the relabeled graph in original vertex order
+// out[i] = in[perm[i]] for i < n: results of the relabeled graph in original vertex order
 __global__ void k_unpermute(const uint32_t* __restrict__ perm, uint32_t n, const uint32_t* __restrict__ in,
                             uint32_t* __restrict__ out) {
     for (uint64_t u = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; u < n;
@@ -432,9 +432,9 @@ eeg_status orig_csr(eeg_graph* g, const Csr& src, Csr& out) {
     return EEG_OK;
 }
 
-eeg_status unpermute(eeg_graph* g, const void* d_in, void* d_out, hipStream_t st) {
-    if (!g->n) return EEG_OK;
-    k_unpermute<<<grid_for(g->n, 8192), WG, 0, st>>>(g->perm.as<uint32_t>(), g->n,
+eeg_status unpermute(eeg_graph* g, const void* d_in, void* d_out, hipStream_t st, uint32_t first, uint32_t count) {
+    if (!count) return EEG_OK;
+    k_unpermute<<<grid_for(count, 8192), WG, 0, st>>>(g->perm.as<uint32_t>() + first, count,
                                                       (const uint32_t*)d_in, (uint32_t*)d_out);
     EEG_HIP(hipGetLastError());
     return EEG_OK;

@@ -8,6 +8,7 @@
 #include <string>
 
 #include "engine.hpp"
+#include "hostcopy.hpp"
 #include "ppr_plane.hpp"
 
 namespace eeg {
@@ -31,6 +32,57 @@ eeg_status Work::poll_events() {
 eeg_status Work::progress() {
     if (!status) EEG_HIP(hipHostMalloc((void**)&status, sizeof(RunStatus), hipHostMallocMapped | hipHostMallocCoherent));
     return EEG_OK;
+}
+
+// ---------------------------------------------------------------- pinned rings (hostcopy.hpp)
+HostRing::~HostRing() {
+    for (auto e : ev)
+        if (e) (void)hipEventDestroy(e);
+    if (base) (void)hipHostFree(base);
+}
+
+namespace {
+std::mutex g_rings_mu;
+std::vector<HostRing*> g_rings;  // idle; what is left at the end goes with the process
+}  // namespace
+
+HostRing* take_host_ring(int device) {
+    {
+        std::lock_guard<std::mutex> lk(g_rings_mu);
+        for (size_t i = 0; i < g_rings.size(); ++i)
+            if (g_rings[i]->device == device) {
+                HostRing* r = g_rings[i];
+                g_rings.erase(g_rings.begin() + (ptrdiff_t)i);
+                return r;
+            }
+    }
+    HostRing* r = new (std::nothrow) HostRing();
+    if (!r) return nullptr;
+    r->device = device;
+    bool ok = hipHostMalloc((void**)&r->base, HOST_SLOTS * HOST_SLOT_BYTES, hipHostMallocDefault) == hipSuccess;
+    if (!ok) r->base = nullptr;
+    for (uint32_t i = 0; ok && i < HOST_SLOTS; ++i)
+        ok = hipEventCreateWithFlags(&r->ev[i], hipEventDisableTiming) == hipSuccess;
+    if (!ok) {
+        (void)hipGetLastError();
+        delete r;
+        return nullptr;
+    }
+    return r;
+}
+
+void give_host_ring(HostRing* r) {
+    {
+        std::lock_guard<std::mutex> lk(g_rings_mu);
+        if (g_rings.size() < HOST_RINGS_KEPT) {
+            try {
+                g_rings.push_back(r);
+                return;
+            } catch (const std::exception&) {
+            }
+        }
+    }
+    delete r;
 }
 
 // The owner has synchronised the stream: no record of these events is pending here.
@@ -284,6 +336,28 @@ extern "C" eeg_status eeg_csr_export_derived(eeg_graph* g, uint32_t which, uint6
     return EEG_OK;
 }
 
+// Labels in internal order to `out`, n words of host memory, in original order.
+static eeg_status labels_to_host(eeg_graph* g, const void* lab, void* out, DevMem& buf, hipStream_t st) {
+    const size_t bytes = (size_t)g->n * 4;
+    LentRing lent(g->device, bytes >= HOST_COPY_FROM);
+    if (lent.r) {
+        constexpr uint32_t words = HOST_SLOT_BYTES / 4;
+        const uint32_t n = g->n, chunks = (uint32_t)(((uint64_t)n + words - 1) / words);
+        auto part = [&](uint32_t i) { return std::min(words, n - i * words); };
+        return stage_to_host(
+            *lent.r, st, chunks, host_copy_threads(bytes), true,
+            [&](uint32_t i, void* slot) { return unpermute(g, lab, slot, st, i * words, part(i)); },
+            [&](uint32_t i, const void* slot, unsigned, unsigned) {
+                memcpy((uint32_t*)out + (size_t)i * words, slot, (size_t)part(i) * 4);
+            });
+    }
+    EEG_TRY(buf.alloc(bytes + 4));
+    EEG_TRY(unpermute(g, lab, buf.p, st, 0, g->n));
+    EEG_HIP(hipMemcpyAsync(out, buf.p, bytes, hipMemcpyDeviceToHost, st));
+    EEG_HIP(hipStreamSynchronize(st));
+    return EEG_OK;
+}
+
 static eeg_status run_common(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_opts* opts,
                              void* out, bool out_is_device, hipStream_t ustream, eeg_stats* stats) {
     clear_error();
@@ -318,17 +392,13 @@ static eeg_status run_common(eeg_graph* g, uint32_t algo, uint32_t source, const
     else clear_error();
     if (s != EEG_OK && s != EEG_ERR_NOT_CONVERGED) return s;
     if (out && g->n) {  // back to original vertex order
-        const size_t bytes = (size_t)g->n * 4;
         if (out_is_device) {
             hipStream_t us = ustream ? ustream : g->stream;
             if (us != g->stream) EEG_HIP(hipStreamSynchronize(g->stream));
-            EEG_TRY(unpermute(g, g->work.lab.p, out, us));
+            EEG_TRY(unpermute(g, g->work.lab.p, out, us, 0, g->n));
             EEG_HIP(hipStreamSynchronize(us));
         } else {
-            EEG_TRY(g->work.out.alloc(bytes + 4));
-            EEG_TRY(unpermute(g, g->work.lab.p, g->work.out.p, g->stream));
-            EEG_HIP(hipMemcpyAsync(out, g->work.out.p, bytes, hipMemcpyDeviceToHost, g->stream));
-            EEG_HIP(hipStreamSynchronize(g->stream));
+            EEG_TRY(labels_to_host(g, g->work.lab.p, out, g->work.out, g->stream));
         }
     }
     st->ms_total = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();

@@ -209,7 +209,8 @@ eeg_status ensure_pr_span(eeg_graph* g, uint32_t K, bool inplace);  // pagerank.
 eeg_status export_tigr(eeg_graph* g, uint32_t K, uint64_t* node_pointer, uint32_t* edge_list,
                        uint32_t* parts, uint64_t* num_parts);
 eeg_status orig_csr(eeg_graph* g, const Csr& src, Csr& out);
-eeg_status unpermute(eeg_graph* g, const void* d_in, void* d_out, hipStream_t st);
+// d_out[i] = label of original vertex first + i, for i < count (d_in: labels in internal order)
+eeg_status unpermute(eeg_graph* g, const void* d_in, void* d_out, hipStream_t st, uint32_t first, uint32_t count);
 eeg_status generate_rmat_device(uint32_t scale, uint32_t ef, double a, double b, double c,
                                 uint64_t seed, uint32_t wmin, uint32_t wmax, uint32_t* d_src,
                                 uint32_t* d_dst, uint32_t* d_w, hipStream_t stream);

@@ -92,7 +92,7 @@ extern "C" eeg_status eeg_run_device_noalloc(eeg_graph* g, uint32_t algo, uint32
     eeg_status rc = run_traversal_fixed(g, algo, isrc, o, fs, s, st);
     if (rc != EEG_OK && rc != EEG_ERR_NOT_CONVERGED) return rc;
     const std::string detail = (rc != EEG_OK) ? eeg_last_error() : "";
-    EEG_TRY(unpermute(g, fs.lab, d_labels_out, s));  // back to original vertex order
+    EEG_TRY(unpermute(g, fs.lab, d_labels_out, s, 0, g->n));  // back to original vertex order
     EEG_HIP(hipStreamSynchronize(s));
     if (rc != EEG_OK) fail(rc, "%s", detail.c_str());
     return rc;

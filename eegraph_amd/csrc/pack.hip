@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "engine.hpp"
+#include "hostcopy.hpp"
 
 namespace eeg {
 namespace {
@@ -184,18 +185,45 @@ extern "C" eeg_status eeg_run_packed(eeg_graph* const* graphs, uint32_t ngraphs,
     const eeg_status keep = rc;
     if (labels_out && u->n) {
         EEG_TRY(u->work.out.alloc((size_t)u->n * 4 + 4));
-        EEG_TRY(unpermute(u, u->work.lab.p, u->work.out.p, s));
+        EEG_TRY(unpermute(u, u->work.lab.p, u->work.out.p, s, 0, u->n));
         uint32_t* outd = u->work.out.as<uint32_t>();
         for (uint32_t i = 0; i < ngraphs; ++i) {
             const uint32_t ni = pk.voff[i + 1] - pk.voff[i];
-            if (!ni || !labels_out[i]) continue;
-            if (algo == EEG_CC && pk.voff[i]) {
-                k_unoffset<<<grid_pk(ni), WG, 0, s>>>(outd + pk.voff[i], ni, pk.voff[i]);
-                EEG_HIP(hipGetLastError());
-            }
-            EEG_HIP(hipMemcpyAsync(labels_out[i], outd + pk.voff[i], (size_t)ni * 4, hipMemcpyDeviceToHost, s));
+            if (!ni || !labels_out[i] || algo != EEG_CC || !pk.voff[i]) continue;
+            k_unoffset<<<grid_pk(ni), WG, 0, s>>>(outd + pk.voff[i], ni, pk.voff[i]);
+            EEG_HIP(hipGetLastError());
         }
-        EEG_HIP(hipStreamSynchronize(s));
+        const size_t bytes = (size_t)u->n * 4;
+        LentRing lent(u->device, bytes >= HOST_COPY_FROM);
+        if (lent.r) {
+            // the union's labels in slots, each cut at the graphs' bounds
+            constexpr uint32_t words = HOST_SLOT_BYTES / 4;
+            const uint32_t N = u->n, chunks = (uint32_t)(((uint64_t)N + words - 1) / words);
+            EEG_TRY(stage_to_host(
+                *lent.r, s, chunks, host_copy_threads(bytes), true,
+                [&](uint32_t c, void* slot) -> eeg_status {
+                    EEG_HIP(hipMemcpyAsync(slot, outd + (size_t)c * words, (size_t)std::min(words, N - c * words) * 4,
+                                           hipMemcpyDeviceToHost, s));
+                    return EEG_OK;
+                },
+                [&](uint32_t c, const void* slot, unsigned, unsigned) {
+                    const uint32_t b = c * words, e = b + std::min(words, N - b);
+                    uint32_t i = (uint32_t)(std::upper_bound(pk.voff.begin(), pk.voff.end(), b) - pk.voff.begin()) - 1;
+                    for (; i < ngraphs && pk.voff[i] < e; ++i) {
+                        const uint32_t lo = std::max(b, pk.voff[i]), hi = std::min(e, pk.voff[i + 1]);
+                        if (lo < hi && labels_out[i])
+                            memcpy((uint32_t*)labels_out[i] + (lo - pk.voff[i]), (const uint32_t*)slot + (lo - b),
+                                   (size_t)(hi - lo) * 4);
+                    }
+                }));
+        } else {
+            for (uint32_t i = 0; i < ngraphs; ++i) {
+                const uint32_t ni = pk.voff[i + 1] - pk.voff[i];
+                if (!ni || !labels_out[i]) continue;
+                EEG_HIP(hipMemcpyAsync(labels_out[i], outd + pk.voff[i], (size_t)ni * 4, hipMemcpyDeviceToHost, s));
+            }
+            EEG_HIP(hipStreamSynchronize(s));
+        }
     }
     st->ms_total = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     if (keep != EEG_OK) return fail(keep, "no fixpoint within max_iters");

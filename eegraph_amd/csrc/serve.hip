@@ -910,7 +910,7 @@ void lane_loop(eeg_server* srv, Lane* ln) {
         if (rc == EEG_OK && !srv->discard) {  // answer in original vertex order
             out.resize(g->n);
             rc = ln->out.alloc((size_t)g->n * 4 + 4);
-            if (rc == EEG_OK) rc = unpermute(g, ln->w.lab.p, ln->out.p, ln->st);
+            if (rc == EEG_OK) rc = unpermute(g, ln->w.lab.p, ln->out.p, ln->st, 0, g->n);
             if (rc == EEG_OK &&
                 (hipMemcpyAsync(out.data(), ln->out.p, (size_t)g->n * 4, hipMemcpyDeviceToHost, ln->st) != hipSuccess ||
                  hipStreamSynchronize(ln->st) != hipSuccess))
