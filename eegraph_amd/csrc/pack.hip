@@ -11,7 +11,9 @@
 #include <algorithm>
 #include <chrono>
 #include <cstring>
+#include <memory>
 #include <mutex>
+#include <utility>
 #include <vector>
 
 #include "engine.hpp"
@@ -26,43 +28,95 @@ unsigned grid_pk(uint64_t work, unsigned cap = 16384) {
     return (unsigned)(g > cap ? cap : g);
 }
 
-// out[v] = row[v] + eoff for v <= n (entry n is rewritten with the same value by the next graph)
-__global__ void k_pack_rows(const uint64_t* __restrict__ row, uint32_t n, uint64_t eoff,
-                            uint64_t* __restrict__ out) {
-    for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v <= n;
-         v += (uint64_t)gridDim.x * blockDim.x)
-        out[v] = row[v] + eoff;
-}
+// One member of a union and its place there, in device memory.
+struct PackMember {
+    const uint64_t* row;
+    const uint32_t *col, *w, *perm, *inv;
+    uint64_t m, eoff;
+    uint32_t n, voff;
+};
+// A run of at most PACK_CHUNK edges (first of them, bit 63 clear) or vertices (bit 63 set) of a
+// member; the workgroups take chunks, so graphs of 2^12 and 2^20 vertices fill the chip alike.
+constexpr uint32_t PACK_CHUNK = 16384;
+constexpr uint64_t PACK_VERTS = 1ull << 63;
+struct PackChunk {
+    uint64_t first;
+    uint32_t member;
+    uint32_t pad;
+};
 
-__global__ void k_add_u32(const uint32_t* __restrict__ in, uint64_t cnt, uint32_t off,
-                          uint32_t* __restrict__ out) {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cnt;
-         i += (uint64_t)gridDim.x * blockDim.x)
-        out[i] = in[i] + off;
+// Copies the members' rows, edges and orders into the union, shifted by their offsets.  Bound by
+// the 16 bytes that an edge moves; one launch for all members (five for each of 64 graphs took
+// their turn at ~5 us).
+__global__ __launch_bounds__(WG) void k_pack(const PackChunk* __restrict__ chunks, const PackMember* __restrict__ mem,
+                                             uint64_t* __restrict__ row, uint32_t* __restrict__ col,
+                                             uint32_t* __restrict__ w, uint32_t* __restrict__ perm,
+                                             uint32_t* __restrict__ inv) {
+    const PackChunk c = chunks[blockIdx.x];
+    const PackMember g = mem[c.member];
+    if (c.first & PACK_VERTS) {
+        const uint64_t f = c.first & ~PACK_VERTS, e = min(f + PACK_CHUNK, (uint64_t)g.n);
+        for (uint64_t v = f + threadIdx.x; v < e; v += WG) {
+            row[g.voff + v] = g.row[v] + g.eoff;
+            perm[g.voff + v] = g.perm[v] + g.voff;
+            inv[g.voff + v] = g.inv[v] + g.voff;
+        }
+        // the row after the last is the next member's first, written with the same value by both
+        if (e == g.n && threadIdx.x == 0) row[g.voff + e] = g.row[e] + g.eoff;
+        return;
+    }
+    const uint64_t e = min(c.first + PACK_CHUNK, g.m);
+    uint32_t* cd = col + g.eoff;
+    uint32_t* wd = w + g.eoff;
+#pragma unroll 4
+    for (uint64_t i = c.first + threadIdx.x; i < e; i += WG) {
+        cd[i] = __builtin_nontemporal_load(&g.col[i]) + g.voff;
+        if (w) wd[i] = __builtin_nontemporal_load(&g.w[i]);
+    }
 }
 
 struct Packed {
     std::vector<uint64_t> serials;
     std::vector<uint32_t> voff;  // ngraphs + 1 vertex offsets
-    eeg_graph* g = nullptr;      // the union
+    eeg_graph* g = nullptr;      // the union (no host copy of the order: members have theirs)
     DevMem seeds;
+    DevMem table;                // members and chunks of the copy
     ~Packed() { delete g; }
 };
+
+// Hands an allocation of the union before to the next one, unless that needs less than a quarter
+// of it (a hipFree and hipMalloc of 1 GiB take milliseconds).  Only for memory whose size is
+// checked where it is used.
+void carry(DevMem& from, DevMem& to, uint64_t need) {
+    if (from.p && from.bytes / 4 <= need) {
+        std::swap(from.p, to.p);
+        std::swap(from.bytes, to.bytes);
+    }
+}
 
 std::mutex g_pack_mu;
 Packed* g_pack = nullptr;  // most recent union (one at a time bounds the HBM held)
 
-eeg_status build_union(eeg_graph* const* gs, uint32_t k, Packed* pk) {
+// `old`: the union before (or null), whose memory is taken over where it fits; the rest is freed
+// before anything is allocated.
+eeg_status build_union(eeg_graph* const* gs, uint32_t k, Packed* pk, std::unique_ptr<Packed> old) {
     uint64_t N = 0, M = 0;
     const bool weighted = gs[0]->weighted;
     pk->voff.assign(k + 1, 0);
+    std::vector<PackMember> mem(k);
+    std::vector<PackChunk> chunks;
     for (uint32_t i = 0; i < k; ++i) {
-        if (gs[i]->device != gs[0]->device) return fail(EEG_ERR_INVALID_ARG, "graphs live on different devices");
-        if (gs[i]->weighted != weighted)
+        const eeg_graph* gi = gs[i];
+        if (gi->device != gs[0]->device) return fail(EEG_ERR_INVALID_ARG, "graphs live on different devices");
+        if (gi->weighted != weighted)
             return fail(EEG_ERR_INVALID_ARG, "weighted and unweighted graphs cannot be packed together");
         pk->voff[i] = (uint32_t)N;
-        N += gs[i]->n;
-        M += gs[i]->m;
+        mem[i] = PackMember{gi->out.rowp(), gi->out.colp(), gi->out.wp(), gi->perm.as<uint32_t>(),
+                            gi->inv.as<uint32_t>(), gi->m, M, gi->n, (uint32_t)N};
+        for (uint64_t f = 0; f < gi->m; f += PACK_CHUNK) chunks.push_back(PackChunk{f, i, 0});
+        for (uint64_t f = 0; f < gi->n; f += PACK_CHUNK) chunks.push_back(PackChunk{f | PACK_VERTS, i, 0});
+        N += gi->n;
+        M += gi->m;
         if (N > 0xfffffff0ull) return fail(EEG_ERR_UNSUPPORTED, "packed vertex count exceeds 2^32 - 16");
     }
     pk->voff[k] = (uint32_t)N;
@@ -73,41 +127,59 @@ eeg_status build_union(eeg_graph* const* gs, uint32_t k, Packed* pk) {
     Csr& c = u->out;
     c.n = (uint32_t)N;
     c.m = M;
+    if (old && old->g && old->g->device == u->device) {
+        eeg_graph* o = old->g;
+        (void)hipStreamSynchronize(o->stream);
+        carry(o->out.row, c.row, (N + 1) * 8);
+        carry(o->out.col, c.col, M * 4);
+        if (weighted) carry(o->out.w, c.w, M * 4);
+        carry(o->perm, u->perm, N * 4);
+        carry(o->inv, u->inv, N * 4);
+        for (int i = 0; i < 4; ++i) {
+            carry(o->tout[i].vlist, u->tout[i].vlist, N * 4);
+            carry(o->tout[i].vscan, u->tout[i].vscan, N * 4);
+            carry(o->tout[i].vnc, u->tout[i].vnc, N * 4);
+        }
+        carry(o->work.lab, u->work.lab, N * 4);
+        carry(o->work.out, u->work.out, N * 4);
+        for (int i = 0; i < 2; ++i) {
+            carry(o->work.q[i], u->work.q[i], N * 4);
+            carry(o->work.s[i], u->work.s[i], N * 4);
+        }
+        carry(o->work.mark, u->work.mark, N);
+        carry(old->table, pk->table, k * sizeof(PackMember));
+    }
+    old.reset();
     EEG_TRY(c.row.alloc((N + 1) * 8));
     EEG_TRY(c.col.alloc(M * 4 + 4));
     if (weighted) EEG_TRY(c.w.alloc(M * 4 + 4));
     EEG_TRY(u->perm.alloc(N * 4 + 4));
     EEG_TRY(u->inv.alloc(N * 4 + 4));
-    u->h_perm.resize(N);
+    EEG_TRY(pk->seeds.alloc((size_t)k * 4 + 4));
+    const size_t mbytes = k * sizeof(PackMember);
+    EEG_TRY(pk->table.alloc(mbytes + chunks.size() * sizeof(PackChunk)));
+    uint8_t* tab = pk->table.as<uint8_t>();
+    EEG_HIP(hipMemcpyAsync(tab, mem.data(), mbytes, hipMemcpyHostToDevice, s));
+    if (!chunks.empty())
+        EEG_HIP(hipMemcpyAsync(tab + mbytes, chunks.data(), chunks.size() * sizeof(PackChunk), hipMemcpyHostToDevice, s));
     // the members' streams may still be writing their tables: wait for them first
     for (uint32_t i = 0; i < k; ++i) EEG_HIP(hipStreamSynchronize(gs[i]->stream));
-    uint64_t eoff = 0;
+    if (!chunks.empty()) {
+        k_pack<<<(unsigned)chunks.size(), WG, 0, s>>>(reinterpret_cast<const PackChunk*>(tab + mbytes),
+                                                      reinterpret_cast<const PackMember*>(tab), c.row.as<uint64_t>(),
+                                                      c.col.as<uint32_t>(), weighted ? c.w.as<uint32_t>() : nullptr,
+                                                      u->perm.as<uint32_t>(), u->inv.as<uint32_t>());
+        EEG_HIP(hipGetLastError());
+    }
     for (uint32_t i = 0; i < k; ++i) {
-        const eeg_graph* gi = gs[i];
-        const uint32_t off = pk->voff[i];
-        if (gi->n) {
-            k_pack_rows<<<grid_pk((uint64_t)gi->n + 1), WG, 0, s>>>(gi->out.rowp(), gi->n, eoff, c.row.as<uint64_t>() + off);
-            k_add_u32<<<grid_pk(gi->n), WG, 0, s>>>(gi->perm.as<uint32_t>(), gi->n, off, u->perm.as<uint32_t>() + off);
-            k_add_u32<<<grid_pk(gi->n), WG, 0, s>>>(gi->inv.as<uint32_t>(), gi->n, off, u->inv.as<uint32_t>() + off);
-            EEG_HIP(hipGetLastError());
-            for (uint32_t v = 0; v < gi->n; ++v) u->h_perm[off + v] = gi->h_perm[v] + off;
+        if (i == 0 || gs[i]->max_deg > u->max_deg) {  // lowest id among the maxima
+            u->max_deg = gs[i]->max_deg;
+            u->argmax_deg = gs[i]->argmax_deg + pk->voff[i];
         }
-        if (gi->m) {
-            k_add_u32<<<grid_pk(gi->m), WG, 0, s>>>(gi->out.colp(), gi->m, off, c.col.as<uint32_t>() + eoff);
-            EEG_HIP(hipGetLastError());
-            if (weighted)
-                EEG_HIP(hipMemcpyAsync(c.w.as<uint32_t>() + eoff, gi->out.wp(), gi->m * 4, hipMemcpyDeviceToDevice, s));
-        }
-        eoff += gi->m;
-        if (i == 0 || gi->max_deg > u->max_deg) {  // lowest id among the maxima
-            u->max_deg = gi->max_deg;
-            u->argmax_deg = gi->argmax_deg + off;
-        }
-        u->nonzero_out += gi->nonzero_out;
+        u->nonzero_out += gs[i]->nonzero_out;
     }
     if (N == 0) EEG_HIP(hipMemsetAsync(c.row.p, 0, 8, s));
     c.built = true;
-    EEG_TRY(pk->seeds.alloc((size_t)k * 4 + 4));
     EEG_HIP(hipStreamSynchronize(s));
     return EEG_OK;
 }
@@ -153,10 +225,16 @@ extern "C" eeg_status eeg_run_packed(eeg_graph* const* graphs, uint32_t ngraphs,
     std::vector<uint64_t> key(ngraphs);
     for (uint32_t i = 0; i < ngraphs; ++i) key[i] = graphs[i]->serial;
     if (!g_pack || g_pack->serials != key) {
-        delete g_pack;
+        std::unique_ptr<Packed> old(g_pack);
         g_pack = new (std::nothrow) Packed();
         if (!g_pack) return fail(EEG_ERR_OOM, "host allocation failed");
-        eeg_status s = build_union(graphs, ngraphs, g_pack);
+        eeg_status s = build_union(graphs, ngraphs, g_pack, std::move(old));
+        if (s == EEG_ERR_OOM) {  // memory taken over may be larger than needed: once more without
+            delete g_pack;
+            g_pack = new (std::nothrow) Packed();
+            if (!g_pack) return fail(EEG_ERR_OOM, "host allocation failed");
+            s = build_union(graphs, ngraphs, g_pack, nullptr);
+        }
         if (s != EEG_OK) {
             delete g_pack;
             g_pack = nullptr;
@@ -174,7 +252,7 @@ extern "C" eeg_status eeg_run_packed(eeg_graph* const* graphs, uint32_t ngraphs,
     eeg_status rc;
     if (sourced) {
         std::vector<uint32_t> seeds(ngraphs);
-        for (uint32_t i = 0; i < ngraphs; ++i) seeds[i] = u->h_perm[pk.voff[i] + sources[i]];
+        for (uint32_t i = 0; i < ngraphs; ++i) seeds[i] = graphs[i]->h_perm[sources[i]] + pk.voff[i];
         EEG_HIP(hipMemcpyAsync(pk.seeds.p, seeds.data(), (size_t)ngraphs * 4, hipMemcpyHostToDevice, s));
         rc = run_traversal(u, algo, 0, o, st, pk.seeds.as<uint32_t>(), ngraphs);
     } else {
