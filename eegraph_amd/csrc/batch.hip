@@ -370,12 +370,18 @@ struct Packed<LM_D8> : Bytes8Dist {};
 // rows.  Narrow labels: lane word x holds queries x*QPL .. x*QPL+QPL-1, so one row read (two
 // for 256 16-bit distances) covers all pending queries of the vertex.  Best when many queries are in flight together; the
 // two-pass kernel below is better when few are.
-template <int K, int LM>
+//
+// G: lanes that share a virtual node.  Rows of at most 16 or 32 narrow lane words (64 or 128
+// queries) leave most of a wavefront idle, so it takes 64 / G virtual nodes side by side: the row
+// reads are what it waits for, and as many more are in flight.  Traversal time, RMAT-20, weights to
+// 64: 64 SSSP queries 8.1 -> 3.8 ms, SSWP 4.5 -> 2.5; weights to 1000 (16 bits, 40 queries) 10.2 ->
+// 7.2; RMAT-19 x 128 SSSP 4.2 -> 2.7.  7 waves per SIMD for these (6: 4.4 ms, 8 with 17 spills: 4.4).
+template <int K, int LM, int G>
 // 32-bit labels: 72 VGPRs at K <= 8 (7 waves per SIMD instead of 6 at 77, no spills): the row
 // reads are latency-bound, so the extra resident wave is worth more (-7 to -8% per pass on
 // RMAT-24).  Narrow labels: at most 64 VGPRs, 8 waves per SIMD (from 4-5 waves at 85-118
 // VGPRs: 25-40% faster passes on RMAT-24 x 256).
-__global__ __launch_bounds__(WG, K <= 8 ? (LM == LM_U32 ? 7 : 8) : 1) void k_plane_push_wave(
+__global__ __launch_bounds__(WG, K <= 8 ? (LM == LM_U32 ? 7 : G == WAVE ? 8 : 7) : 1) void k_plane_push_wave(
     PlaneArgs args) {
     PlaneArgs a = args;
     plane_resolve(a);
@@ -449,7 +455,15 @@ __global__ __launch_bounds__(WG, K <= 8 ? (LM == LM_U32 ? 7 : 8) : 1) void k_pla
         // node's <= K edges (one per lane) and broadcast them, then for every 64-query word
         // with pending changes each lane (one query) issues all K destination-label reads
         // before any atomic, so K requests per lane are in flight
-        for (uint32_t t = t0 + wv; t < t1; t += NW) {
+        constexpr int SIDE = WAVE / G;            // virtual nodes side by side
+        const int sub = SIDE == 1 ? 0 : lane / G, gl = SIDE == 1 ? lane : lane % G;  // this lane's, its place there
+        // value of the group's lane e
+        auto edge = [&](uint32_t x, int e) -> uint32_t {
+            if constexpr (G == WAVE) return __builtin_amdgcn_readlane(x, e);
+            else return (uint32_t)__shfl((int)x, sub * G + e, WAVE);
+        };
+        for (uint32_t tb = t0 + wv * SIDE; tb < t1; tb += NW * SIDE) {
+            const uint32_t t = min(tb + sub, t1 - 1);
             int lo = 0, hi = nent;
             while (hi - lo > 1) {
                 const int mid = (lo + hi) >> 1;
@@ -458,11 +472,12 @@ __global__ __launch_bounds__(WG, K <= 8 ? (LM == LM_U32 ? 7 : 8) : 1) void k_pla
             const int k = lo;
             const uint32_t v = sV[k];
             const uint32_t e0 = (t - sS[k]) * K;
-            const uint32_t ne = min((uint32_t)K, sDeg[k] - e0);
+            const bool idle = SIDE > 1 && tb + sub >= t1;
+            const uint32_t ne = idle ? 0u : min((uint32_t)K, sDeg[k] - e0);
             uint32_t my_u = 0, my_w = 0;
-            if ((uint32_t)lane < ne) {
-                my_u = a.col[sRow[k] + e0 + lane];
-                my_w = a.wgt[sRow[k] + e0 + lane];
+            if ((uint32_t)gl < ne) {
+                my_u = a.col[sRow[k] + e0 + gl];
+                my_w = a.wgt[sRow[k] + e0 + gl];
             }
             if constexpr (LM != LM_U32) {
                 using P = Packed<LM>;
@@ -471,10 +486,10 @@ __global__ __launch_bounds__(WG, K <= 8 ? (LM == LM_U32 ? 7 : 8) : 1) void k_pla
                 constexpr uint32_t GM = (1u << QPL) - 1;
                 uint32_t* plane = a.lab;
                 const uint32_t nl = a.B / QPL;       // lane words per row
-                for (uint32_t x0 = 0; x0 < nl; x0 += WAVE) {  // passes of 64 lane words
-                    const uint32_t x = x0 + (uint32_t)lane;
+                for (uint32_t x0 = 0; x0 < nl; x0 += G) {  // passes of G lane words
+                    const uint32_t x = x0 + (uint32_t)gl;
                     uint32_t nib = 0;
-                    if (x < nl) nib = (uint32_t)(a.chg[(uint64_t)v * a.W + x / GL] >> (QPL * (x % GL))) & GM;
+                    if (x < nl && !idle) nib = (uint32_t)(a.chg[(uint64_t)v * a.W + x / GL] >> (QPL * (x % GL))) & GM;
                     if constexpr (LM == LM_D8) nib &= ~(uint32_t)(sOv[x / GL] >> (QPL * (x % GL)));
                     if (!__ballot(nib != 0)) continue;  // the same answer in every lane
                     const uint32_t lv = nib ? plane[(uint64_t)v * nl + x] : 0u;
@@ -484,15 +499,15 @@ __global__ __launch_bounds__(WG, K <= 8 ? (LM == LM_U32 ? 7 : 8) : 1) void k_pla
                     uint32_t ecur[K];
 #pragma unroll
                     for (int e = 0; e < K; ++e) {  // every destination row read before any update
-                        const uint32_t u = __builtin_amdgcn_readlane(my_u, e);
+                        const uint32_t u = edge(my_u, e);
                         ecur[e] = (nib && (uint32_t)e < ne) ? plane[(uint64_t)u * nl + x] : 0u;
                     }
                     uint32_t imp[K];
 #pragma unroll
                     for (int e = 0; e < K; ++e) {
                         imp[e] = 0;
-                        const uint32_t u = __builtin_amdgcn_readlane(my_u, e);
-                        const uint32_t wt = __builtin_amdgcn_readlane(my_w, e);
+                        const uint32_t u = edge(my_u, e);
+                        const uint32_t wt = edge(my_w, e);
                         if (nib && (uint32_t)e < ne) {
                             uint32_t ov = 0;
                             const uint32_t cd = P::cand(lv, wt, nib, ov);
@@ -526,11 +541,16 @@ __global__ __launch_bounds__(WG, K <= 8 ? (LM == LM_U32 ? 7 : 8) : 1) void k_pla
                     }
 #pragma unroll
                     for (int e = 0; e < K; ++e) {
-                        const uint32_t u = __builtin_amdgcn_readlane(my_u, e);
+                        const uint32_t u = edge(my_u, e);
                         if (!__ballot(imp[e] != 0)) continue;
                         // only vertices with out-edges carry changes and are queued (each
                         // queued entry owns >= 1 virtual node); a sink's label is final
-                        if (!a.vnc[u]) continue;
+                        if constexpr (G == WAVE) {
+                            if (!a.vnc[u]) continue;
+                        } else {
+                            if (imp[e] && !a.vnc[u]) imp[e] = 0;
+                            if (!__ballot(imp[e] != 0)) continue;
+                        }
                         // the improved queries of each 64-query word: its GL lane words
                         // are neighbouring lanes
                         uint64_t word = (uint64_t)imp[e] << (QPL * (x % GL));
@@ -538,7 +558,12 @@ __global__ __launch_bounds__(WG, K <= 8 ? (LM == LM_U32 ? 7 : 8) : 1) void k_pla
                         for (uint32_t off = GL / 2; off >= 1; off >>= 1) word |= __shfl_xor(word, (int)off, WAVE);
                         if ((x % GL) == 0 && word)
                             atomicOr((unsigned long long*)&a.nchg[(uint64_t)u * a.W + x / GL], (unsigned long long)word);
-                        if (lane == 0) {
+                        bool queue = gl == 0;
+                        if constexpr (G != WAVE) {
+                            const uint64_t any = __ballot(imp[e] != 0);  // of every lane, so not behind gl == 0
+                            queue = queue && ((any >> (sub * G)) & ((1ull << G) - 1)) != 0;
+                        }
+                        if (queue) {
                             if (a.mark) {
                                 set_mark(a.mark, a.cmark, u);
                             } else if (atomicExch(&a.stamp[u], a.stampv) != a.stampv) {
@@ -1177,26 +1202,28 @@ eeg_status add_node(hipGraph_t graph, hipGraphNode_t* prev, const void* fn, unsi
     return EEG_OK;
 }
 
-// Graph of BATCH_CHUNK iterations (BFS: push, finalize; planes: push, two rotations; each
-// followed by a counter tick), built node by node and kept until its arguments change.
-// Dense plane push for K and label width lm.
-const void* dense_push(uint32_t K, int lm) {
+// Dense plane push for K, label width lm and W mask words (rows of 16 W or 32 W narrow lane
+// words): the fewest lanes that hold a row, and an edge each.
+template <int LM, int G>
+const void* dense_push_k(uint32_t K) {
+    switch (K) {
+        case 4: return (const void*)k_plane_push_wave<4, LM, G>;
+        case 8: return (const void*)k_plane_push_wave<8, LM, G>;
+        case 16: return (const void*)k_plane_push_wave<16, LM, G>;
+        default: return (const void*)k_plane_push_wave<32, LM, G < 32 ? 32 : G>;
+    }
+}
+const void* dense_push(uint32_t K, int lm, uint32_t W) {
     switch (lm) {
-        case LM_W8:
-            return (K == 4) ? (const void*)k_plane_push_wave<4, LM_W8> : (K == 8) ? (const void*)k_plane_push_wave<8, LM_W8>
-                   : (K == 16) ? (const void*)k_plane_push_wave<16, LM_W8> : (const void*)k_plane_push_wave<32, LM_W8>;
-        case LM_D16:
-            return (K == 4) ? (const void*)k_plane_push_wave<4, LM_D16> : (K == 8) ? (const void*)k_plane_push_wave<8, LM_D16>
-                   : (K == 16) ? (const void*)k_plane_push_wave<16, LM_D16> : (const void*)k_plane_push_wave<32, LM_D16>;
-        case LM_D8:
-            return (K == 4) ? (const void*)k_plane_push_wave<4, LM_D8> : (K == 8) ? (const void*)k_plane_push_wave<8, LM_D8>
-                   : (K == 16) ? (const void*)k_plane_push_wave<16, LM_D8> : (const void*)k_plane_push_wave<32, LM_D8>;
-        default:
-            return (K == 4) ? (const void*)k_plane_push_wave<4, LM_U32> : (K == 8) ? (const void*)k_plane_push_wave<8, LM_U32>
-                   : (K == 16) ? (const void*)k_plane_push_wave<16, LM_U32> : (const void*)k_plane_push_wave<32, LM_U32>;
+        case LM_W8: return W == 1 ? dense_push_k<LM_W8, 16>(K) : W == 2 ? dense_push_k<LM_W8, 32>(K) : dense_push_k<LM_W8, 64>(K);
+        case LM_D16: return W == 1 ? dense_push_k<LM_D16, 32>(K) : dense_push_k<LM_D16, 64>(K);
+        case LM_D8: return W == 1 ? dense_push_k<LM_D8, 16>(K) : W == 2 ? dense_push_k<LM_D8, 32>(K) : dense_push_k<LM_D8, 64>(K);
+        default: return dense_push_k<LM_U32, 64>(K);
     }
 }
 
+// Graph of BATCH_CHUNK iterations (BFS: push, finalize; planes: push, two rotations; each
+// followed by a counter tick), built node by node and kept until its arguments change.
 eeg_status batch_graph(BatchWork& bw, bool bfs, uint32_t K, unsigned grid, const MsArgs& ma, const PlaneArgs& pa,
                        uint32_t nsrc, int lm, hipGraphExec_t* out) {
     const bool dense = nsrc > PLANE_DENSE_FROM;
@@ -1251,7 +1278,7 @@ eeg_status batch_graph(BatchWork& bw, bool bfs, uint32_t K, unsigned grid, const
     const void* fpush =
         bfs ? ((K == 4) ? (const void*)k_ms_push<4> : (K == 8) ? (const void*)k_ms_push<8>
                : (K == 16) ? (const void*)k_ms_push<16> : (const void*)k_ms_push<32>)
-        : dense ? dense_push(K, lm)
+        : dense ? dense_push(K, lm, pa.W)
                 : ((K == 4) ? (const void*)k_plane_push<4> : (K == 8) ? (const void*)k_plane_push<8>
                    : (K == 16) ? (const void*)k_plane_push<16> : (const void*)k_plane_push<32>);
     hipGraphNode_t prev = nullptr;
@@ -1768,7 +1795,7 @@ eeg_status launch_plane_iteration(PlaneArgs a, uint32_t K, unsigned grid, hipStr
     void* args[] = {&a};
     const void* fn = (K == 4) ? (const void*)k_plane_push<4> : (K == 8) ? (const void*)k_plane_push<8>
                      : (K == 16) ? (const void*)k_plane_push<16> : (const void*)k_plane_push<32>;
-    if (in_flight > PLANE_DENSE_FROM) fn = dense_push(K, lm);
+    if (in_flight > PLANE_DENSE_FROM) fn = dense_push(K, lm, a.W);
     EEG_HIP(hipLaunchKernel(fn, dim3(grid), dim3(WG), args, 0, s));
     if (a.mark) {  // sorted queue: the push only marked vertices
         CompactArgs ca = compact_args(a);
