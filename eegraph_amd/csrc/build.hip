@@ -55,15 +55,14 @@ __global__ void k_iota(uint32_t* __restrict__ a, uint64_t m) {
         a[i] = (uint32_t)i;
 }
 
-__global__ void k_gather(const uint32_t* __restrict__ perm, const uint32_t* __restrict__ a,
-                         const uint32_t* __restrict__ b, uint32_t* __restrict__ ao,
-                         uint32_t* __restrict__ bo, uint64_t m) {
+// Values of the sort by source: destination and weight of an edge in one word, so the sort carries
+// them (3 passes of 8 more bytes an edge) and nothing is gathered afterwards through a permutation
+// of the edges (0.63 ms for 16.8 M edges, two lines an edge; the sort takes 0.1 ms more).
+__global__ void k_edge_values(const uint32_t* __restrict__ dst, const uint32_t* __restrict__ w, uint64_t m,
+                              uint64_t* __restrict__ out) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m;
-         i += (uint64_t)gridDim.x * blockDim.x) {
-        const uint32_t p = perm[i];
-        ao[i] = a[p];
-        if (b) bo[i] = b[p];
-    }
+         i += (uint64_t)gridDim.x * blockDim.x)
+        out[i] = dst[i] | ((uint64_t)w[i] << 32);
 }
 
 // ---------------------------------------------------------------- degree-ordered relabeling
@@ -83,13 +82,27 @@ __global__ void k_invert(const uint32_t* __restrict__ inv, uint32_t n, uint32_t*
          i += (uint64_t)gridDim.x * blockDim.x)
         perm[inv[i]] = (uint32_t)i;
 }
-__global__ void k_relabel(const uint32_t* __restrict__ perm, const uint32_t* __restrict__ a,
-                          const uint32_t* __restrict__ b, uint32_t* __restrict__ ao,
-                          uint32_t* __restrict__ bo, uint64_t m) {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m;
-         i += (uint64_t)gridDim.x * blockDim.x) {
-        ao[i] = perm[a[i]];
-        bo[i] = perm[b[i]];
+// Where the edges of original vertex u go: edge e of the list sorted by source belongs at e +
+// shift[u] of the relabeled one.
+__global__ void k_row_shift(const uint32_t* __restrict__ perm, const uint64_t* __restrict__ orow,
+                            const uint64_t* __restrict__ row, uint32_t n, int64_t* __restrict__ shift) {
+    for (uint64_t u = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; u < n;
+         u += (uint64_t)gridDim.x * blockDim.x)
+        shift[u] = (int64_t)row[perm[u]] - (int64_t)orow[u];
+}
+// Rows of the relabeled CSR: whole rows move, in their order, and only the destinations are renamed
+// (a second sort by the new sources would move every edge three times more).  `val` holds
+// destinations, or destination | weight << 32.
+template <class V>
+__global__ void k_place_rows(const uint32_t* __restrict__ keys, const V* __restrict__ val, uint64_t m,
+                             const int64_t* __restrict__ shift, const uint32_t* __restrict__ perm,
+                             uint32_t* __restrict__ col, uint32_t* __restrict__ w) {
+    for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < m;
+         e += (uint64_t)gridDim.x * blockDim.x) {
+        const V x = val[e];
+        const uint64_t at = (uint64_t)((int64_t)e + shift[keys[e]]);
+        col[at] = perm[(uint32_t)x];
+        if constexpr (sizeof(V) == 8) w[at] = (uint32_t)(x >> 32);
     }
 }
 // out[i] = in[perm[i]] for i < n: results of the relabeled graph in original vertex order
@@ -99,6 +112,16 @@ __global__ void k_unpermute(const uint32_t* __restrict__ perm, uint32_t n, const
          u += (uint64_t)gridDim.x * blockDim.x)
         out[u] = in[perm[u]];
 }
+struct NewDegLoad {  // degree of internal vertex v (element n: 0)
+    const uint64_t* orow;
+    const uint32_t* inv;
+    uint32_t n;
+    __device__ uint64_t operator()(uint64_t v) const {
+        if (v >= n) return 0;
+        const uint32_t u = inv[v];
+        return orow[u + 1] - orow[u];
+    }
+};
 struct OrigDegLoad {  // degree of original vertex u (element n: 0)
     const uint64_t* row;
     const uint32_t* perm;
@@ -126,9 +149,12 @@ __global__ void k_orig_rows(const uint64_t* __restrict__ row, const uint32_t* __
     }
 }
 
-// max out-degree, lowest id among the maxima, and the count of vertices with edges
-__global__ void k_degree_stats(const uint64_t* __restrict__ row, uint32_t n,
-                               unsigned long long* __restrict__ best, uint32_t* __restrict__ nnz) {
+// max out-degree, lowest id among the maxima, and the count of vertices with edges: out[0], out[1].
+// Two atomics a workgroup (two a wavefront of 4096 workgroups took their turn for 0.19 ms).
+__global__ __launch_bounds__(WG) void k_degree_stats(const uint64_t* __restrict__ row, uint32_t n,
+                                                     unsigned long long* __restrict__ out) {
+    __shared__ unsigned long long sBest[WG / WAVE];
+    __shared__ uint32_t sCnt[WG / WAVE];
     unsigned long long b = 0;
     uint32_t c = 0;
     for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n;
@@ -145,8 +171,17 @@ __global__ void k_degree_stats(const uint64_t* __restrict__ row, uint32_t n,
     }
     c = wave_sum(c);
     if (lane_id() == 0) {
-        atomicMax(best, b);
-        atomicAdd(nnz, c);
+        sBest[threadIdx.x / WAVE] = b;
+        sCnt[threadIdx.x / WAVE] = c;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int i = 1; i < WG / WAVE; ++i) {
+            b = sBest[i] > b ? sBest[i] : b;
+            c += sCnt[i];
+        }
+        atomicMax(&out[0], b);
+        atomicAdd(&out[1], (unsigned long long)c);
     }
 }
 
@@ -162,51 +197,36 @@ uint32_t key_bits(uint32_t n) {
     return b;
 }
 
-// Builds rows of `c` from (keys, vals, w) with keys < n: a stable sort of (key, edge index)
-// pairs gives the order (input order within a key); row offsets are lower bounds of each
-// vertex id in the sorted keys.
-eeg_status build_rows(hipStream_t st, uint32_t n, const uint32_t* keys, const uint32_t* vals,
-                      const uint32_t* w, uint64_t m, Csr& c) {
+// Stable sort of (key, value) pairs with keys < n (input order within a key).
+template <class V>
+eeg_status sort_by_key(hipStream_t st, uint32_t n, const uint32_t* keys, uint32_t* kout, const V* vals, V* vout,
+                       uint64_t m, DevMem& tmp) {
+    size_t tbytes = 0;
+    const uint32_t bits = key_bits(n);
+    EEG_HIP(rocprim::radix_sort_pairs(nullptr, tbytes, keys, kout, vals, vout, (size_t)m, 0, bits, st));
+    EEG_TRY(tmp.alloc(tbytes));
+    EEG_HIP(rocprim::radix_sort_pairs(tmp.p, tbytes, keys, kout, vals, vout, (size_t)m, 0, bits, st));
+    return EEG_OK;
+}
+
+// Builds rows of `c` from (keys, vals) with keys < n, without weights: the sort carries the
+// values; row offsets are lower bounds of each vertex id in the sorted keys.
+eeg_status build_rows(hipStream_t st, uint32_t n, const uint32_t* keys, const uint32_t* vals, uint64_t m, Csr& c) {
     c.n = n;
     c.m = m;
     EEG_TRY(c.row.alloc((size_t)(n + 1ull) * 8));
     EEG_TRY(c.col.alloc(m * 4));
-    if (w) EEG_TRY(c.w.alloc(m * 4));
-    DevMem bad;
-    EEG_TRY(bad.alloc(8));
-    EEG_HIP(hipMemsetAsync(bad.p, 0, 8, st));
-    k_validate<<<grid_for(m), WG, 0, st>>>(keys, vals, m, n, bad.as<uint32_t>());
-    EEG_HIP(hipGetLastError());
-    uint32_t nbad = 0;
-    EEG_HIP(hipMemcpyAsync(&nbad, bad.p, 4, hipMemcpyDeviceToHost, st));
-    EEG_HIP(hipStreamSynchronize(st));
-    if (nbad) return fail(EEG_ERR_INVALID_ARG, "%u edges have an endpoint >= n (%u)", nbad, n);
     if (m == 0) {
         EEG_HIP(hipMemsetAsync(c.row.p, 0, (size_t)(n + 1ull) * 8, st));
         EEG_HIP(hipStreamSynchronize(st));
         c.built = true;
         return EEG_OK;
     }
-    DevMem kout, idx, perm, tmp;
+    DevMem kout, tmp;
     EEG_TRY(kout.alloc(m * 4));
-    EEG_TRY(idx.alloc(m * 4));
-    EEG_TRY(perm.alloc(m * 4));
-    k_iota<<<grid_for(m), WG, 0, st>>>(idx.as<uint32_t>(), m);
-    EEG_HIP(hipGetLastError());
-    size_t tbytes = 0;
-    const uint32_t bits = key_bits(n);
-    EEG_HIP(rocprim::radix_sort_pairs(nullptr, tbytes, keys, kout.as<uint32_t>(),
-                                      idx.as<uint32_t>(), perm.as<uint32_t>(), (size_t)m, 0, bits,
-                                      st));
-    EEG_TRY(tmp.alloc(tbytes));
-    EEG_HIP(rocprim::radix_sort_pairs(tmp.p, tbytes, keys, kout.as<uint32_t>(),
-                                      idx.as<uint32_t>(), perm.as<uint32_t>(), (size_t)m, 0, bits,
-                                      st));
+    EEG_TRY(sort_by_key(st, n, keys, kout.as<uint32_t>(), vals, c.col.as<uint32_t>(), m, tmp));
     k_rows_from_sorted<<<grid_for((uint64_t)n + 1), WG, 0, st>>>(kout.as<uint32_t>(), m, n,
                                                                  c.row.as<uint64_t>());
-    EEG_HIP(hipGetLastError());
-    k_gather<<<grid_for(m), WG, 0, st>>>(perm.as<uint32_t>(), vals, w, c.col.as<uint32_t>(),
-                                         w ? c.w.as<uint32_t>() : nullptr, m);
     EEG_HIP(hipGetLastError());
     EEG_HIP(hipStreamSynchronize(st));
     c.built = true;
@@ -309,15 +329,15 @@ __global__ void k_rmat(uint64_t key, uint64_t wkey, uint32_t scale, uint64_t ta,
 
 }  // namespace
 
-// Row offsets of the list sorted by `keys` (keys only; used for degrees in original ids).
+// Row offsets of the list sorted by `keys` (keys only; used for degrees in original ids).  `kout`
+// and `tmp` are scratch, free again in stream order.
 static eeg_status rows_from_keys(hipStream_t st, const uint32_t* keys, uint64_t m, uint32_t n,
-                                 DevMem& row) {
+                                 DevMem& row, DevMem& kout, DevMem& tmp) {
     EEG_TRY(row.alloc(((size_t)n + 1) * 8));
     if (m == 0) {
         EEG_HIP(hipMemsetAsync(row.p, 0, ((size_t)n + 1) * 8, st));
         return EEG_OK;
     }
-    DevMem kout, tmp;
     EEG_TRY(kout.alloc(m * 4));
     size_t tbytes = 0;
     const uint32_t bits = key_bits(n);
@@ -327,7 +347,6 @@ static eeg_status rows_from_keys(hipStream_t st, const uint32_t* keys, uint64_t 
     k_rows_from_sorted<<<grid_for((uint64_t)n + 1), WG, 0, st>>>(kout.as<uint32_t>(), m, n,
                                                                  row.as<uint64_t>());
     EEG_HIP(hipGetLastError());
-    EEG_HIP(hipStreamSynchronize(st));
     return EEG_OK;
 }
 
@@ -335,30 +354,57 @@ eeg_status build_csr_from_device_edges(eeg_graph* g, const uint32_t* d_src, cons
                                        const uint32_t* d_w, uint64_t m) {
     hipStream_t st = g->stream;
     const uint32_t n = g->n;
-    {
-        DevMem bad;
-        EEG_TRY(bad.alloc(8));
-        EEG_HIP(hipMemsetAsync(bad.p, 0, 8, st));
-        if (m) {
-            k_validate<<<grid_for(m), WG, 0, st>>>(d_src, d_dst, m, n, bad.as<uint32_t>());
-            EEG_HIP(hipGetLastError());
-        }
-        uint32_t nbad = 0;
-        EEG_HIP(hipMemcpyAsync(&nbad, bad.p, 4, hipMemcpyDeviceToHost, st));
-        EEG_HIP(hipStreamSynchronize(st));
-        if (nbad) return fail(EEG_ERR_INVALID_ARG, "%u edges have an endpoint >= n (%u)", nbad, n);
+    // zeroed words: bad edges, then the degree statistics
+    DevMem small;
+    EEG_TRY(small.alloc(24));
+    EEG_HIP(hipMemsetAsync(small.p, 0, 24, st));
+    if (m) {
+        k_validate<<<grid_for(m, 4096), WG, 0, st>>>(d_src, d_dst, m, n, small.as<uint32_t>());
+        EEG_HIP(hipGetLastError());
     }
-    // degrees in original ids, then the degree order
-    DevMem orow, irow;
-    EEG_TRY(rows_from_keys(st, d_src, m, n, orow));
-    EEG_TRY(rows_from_keys(st, d_dst, m, n, irow));
+    uint32_t nbad = 0;
+    EEG_HIP(hipMemcpyAsync(&nbad, small.p, 4, hipMemcpyDeviceToHost, st));
+    EEG_HIP(hipStreamSynchronize(st));
+    if (nbad) return fail(EEG_ERR_INVALID_ARG, "%u edges have an endpoint >= n (%u)", nbad, n);
+    Csr& c = g->out;
+    c.n = n;
+    c.m = m;
+    EEG_TRY(c.row.alloc(((size_t)n + 1) * 8));
     EEG_TRY(g->perm.alloc((size_t)n * 4 + 4));
     EEG_TRY(g->inv.alloc((size_t)n * 4 + 4));
+    // degrees in original ids: rows of the edges sorted by source (with what they carry), and of
+    // the destinations
+    DevMem orow, irow, keys, vals, vin, tmp;
+    EEG_TRY(rows_from_keys(st, d_dst, m, n, irow, keys, tmp));
+    EEG_TRY(orow.alloc(((size_t)n + 1) * 8));
+    if (m) {
+        if (d_w) {
+            EEG_TRY(vin.alloc(m * 8));
+            EEG_TRY(vals.alloc(m * 8));
+            k_edge_values<<<grid_for(m, 16384), WG, 0, st>>>(d_dst, d_w, m, vin.as<uint64_t>());
+            EEG_HIP(hipGetLastError());
+            EEG_TRY(sort_by_key(st, n, d_src, keys.as<uint32_t>(), vin.as<uint64_t>(), vals.as<uint64_t>(), m, tmp));
+        } else {
+            EEG_TRY(vals.alloc(m * 4));
+            EEG_TRY(sort_by_key(st, n, d_src, keys.as<uint32_t>(), d_dst, vals.as<uint32_t>(), m, tmp));
+        }
+        k_rows_from_sorted<<<grid_for((uint64_t)n + 1), WG, 0, st>>>(keys.as<uint32_t>(), m, n, orow.as<uint64_t>());
+        EEG_HIP(hipGetLastError());
+    } else {
+        EEG_HIP(hipMemsetAsync(orow.p, 0, ((size_t)n + 1) * 8, st));
+    }
+    if (m >= 1ull << 28) vin.release();  // (waits; 8 B an edge, which the rows below take again)
+    EEG_TRY(c.col.alloc(m * 4));
+    if (d_w) EEG_TRY(c.w.alloc(m * 4));
+    DevMem key, kout, ids, tmpn, shift;
+    unsigned long long stats[2] = {0, 0};
+    g->h_perm.resize(n);
     if (n) {
-        DevMem key, kout, ids, tmp;
+        // the degree order
         EEG_TRY(key.alloc((size_t)n * 4));
         EEG_TRY(kout.alloc((size_t)n * 4));
         EEG_TRY(ids.alloc((size_t)n * 4));
+        EEG_TRY(shift.alloc((size_t)n * 8));
         k_degree_key<<<grid_for(n), WG, 0, st>>>(orow.as<uint64_t>(), irow.as<uint64_t>(), n,
                                                  key.as<uint32_t>());
         k_iota<<<grid_for(n), WG, 0, st>>>(ids.as<uint32_t>(), n);
@@ -366,46 +412,35 @@ eeg_status build_csr_from_device_edges(eeg_graph* g, const uint32_t* d_src, cons
         size_t tbytes = 0;
         EEG_HIP(rocprim::radix_sort_pairs(nullptr, tbytes, key.as<uint32_t>(), kout.as<uint32_t>(),
                                           ids.as<uint32_t>(), g->inv.as<uint32_t>(), (size_t)n, 0, 32, st));
-        EEG_TRY(tmp.alloc(tbytes));
-        EEG_HIP(rocprim::radix_sort_pairs(tmp.p, tbytes, key.as<uint32_t>(), kout.as<uint32_t>(),
+        EEG_TRY(tmpn.alloc(tbytes));
+        EEG_HIP(rocprim::radix_sort_pairs(tmpn.p, tbytes, key.as<uint32_t>(), kout.as<uint32_t>(),
                                           ids.as<uint32_t>(), g->inv.as<uint32_t>(), (size_t)n, 0, 32, st));
         k_invert<<<grid_for(n), WG, 0, st>>>(g->inv.as<uint32_t>(), n, g->perm.as<uint32_t>());
+        k_degree_stats<<<grid_for(n, 512), WG, 0, st>>>(orow.as<uint64_t>(), n, small.as<unsigned long long>() + 1);
         EEG_HIP(hipGetLastError());
-        EEG_HIP(hipStreamSynchronize(st));
     }
-    irow.release();
-    {
-        DevMem s2, d2;
-        EEG_TRY(s2.alloc(m * 4 + 4));
-        EEG_TRY(d2.alloc(m * 4 + 4));
-        if (m) {
-            k_relabel<<<grid_for(m), WG, 0, st>>>(g->perm.as<uint32_t>(), d_src, d_dst,
-                                                  s2.as<uint32_t>(), d2.as<uint32_t>(), m);
-            EEG_HIP(hipGetLastError());
-        }
-        EEG_TRY(build_rows(st, n, s2.as<uint32_t>(), d2.as<uint32_t>(), d_w, m, g->out));
+    EEG_TRY(scan_exclusive(NewDegLoad{orow.as<uint64_t>(), g->inv.as<uint32_t>(), n}, RowStore{c.row.as<uint64_t>()},
+                           (uint64_t)n + 1, st, nullptr));
+    if (m) {
+        k_row_shift<<<grid_for(n), WG, 0, st>>>(g->perm.as<uint32_t>(), orow.as<uint64_t>(), c.rowp(), n,
+                                                shift.as<int64_t>());
+        const unsigned gr = grid_for(m, 16384);
+        if (d_w)
+            k_place_rows<<<gr, WG, 0, st>>>(keys.as<uint32_t>(), vals.as<uint64_t>(), m, shift.as<int64_t>(),
+                                            g->perm.as<uint32_t>(), c.col.as<uint32_t>(), c.w.as<uint32_t>());
+        else
+            k_place_rows<<<gr, WG, 0, st>>>(keys.as<uint32_t>(), vals.as<uint32_t>(), m, shift.as<int64_t>(),
+                                            g->perm.as<uint32_t>(), c.col.as<uint32_t>(), (uint32_t*)nullptr);
+        EEG_HIP(hipGetLastError());
     }
-    g->h_perm.resize(n);
-    if (n) EEG_HIP(hipMemcpy(g->h_perm.data(), g->perm.p, (size_t)n * 4, hipMemcpyDeviceToHost));
+    if (n) EEG_HIP(hipMemcpyAsync(g->h_perm.data(), g->perm.p, (size_t)n * 4, hipMemcpyDeviceToHost, st));
     // statistics in original ids
-    DevMem best, nnz;
-    EEG_TRY(best.alloc(8));
-    EEG_TRY(nnz.alloc(4));
-    EEG_HIP(hipMemsetAsync(best.p, 0, 8, st));
-    EEG_HIP(hipMemsetAsync(nnz.p, 0, 4, st));
-    if (n) {
-        k_degree_stats<<<grid_for(n, 4096), WG, 0, st>>>(orow.as<uint64_t>(), n,
-                                                         best.as<unsigned long long>(), nnz.as<uint32_t>());
-        EEG_HIP(hipGetLastError());
-    }
-    unsigned long long b = 0;
-    uint32_t c = 0;
-    EEG_HIP(hipMemcpyAsync(&b, best.p, 8, hipMemcpyDeviceToHost, st));
-    EEG_HIP(hipMemcpyAsync(&c, nnz.p, 4, hipMemcpyDeviceToHost, st));
+    EEG_HIP(hipMemcpyAsync(stats, small.as<unsigned long long>() + 1, 16, hipMemcpyDeviceToHost, st));
     EEG_HIP(hipStreamSynchronize(st));
-    g->max_deg = (uint32_t)(b >> 32);
-    g->argmax_deg = n ? ~(uint32_t)(b & 0xffffffffull) : 0;
-    g->nonzero_out = c;
+    c.built = true;
+    g->max_deg = (uint32_t)(stats[0] >> 32);
+    g->argmax_deg = n ? ~(uint32_t)(stats[0] & 0xffffffffull) : 0;
+    g->nonzero_out = (uint32_t)stats[1];
     return EEG_OK;
 }
 
@@ -504,14 +539,14 @@ eeg_status ensure_sym(eeg_graph* g) {
                                st));
     }
     src.release();
-    return build_rows(st, g->n, keys.as<uint32_t>(), vals.as<uint32_t>(), nullptr, 2 * m, g->sym);
+    return build_rows(st, g->n, keys.as<uint32_t>(), vals.as<uint32_t>(), 2 * m, g->sym);
 }
 
 eeg_status ensure_in(eeg_graph* g) {
     if (g->in.built) return EEG_OK;
     DevMem src;
     EEG_TRY(expand_sources(g, src));
-    return build_rows(g->stream, g->n, g->out.colp(), src.as<uint32_t>(), nullptr, g->m, g->in);
+    return build_rows(g->stream, g->n, g->out.colp(), src.as<uint32_t>(), g->m, g->in);
 }
 
 eeg_status export_tigr(eeg_graph* g, uint32_t K, uint64_t* node_pointer, uint32_t* edge_list,

@@ -5,6 +5,7 @@
 #include <atomic>
 #include <chrono>
 #include <cstring>
+#include <initializer_list>
 #include <string>
 
 #include "engine.hpp"
@@ -32,6 +33,82 @@ eeg_status Work::poll_events() {
 eeg_status Work::progress() {
     if (!status) EEG_HIP(hipHostMalloc((void**)&status, sizeof(RunStatus), hipHostMallocMapped | hipHostMallocCoherent));
     return EEG_OK;
+}
+
+// ---------------------------------------------------------------- device blocks (DevMem)
+namespace {
+// Blocks of one size are interchangeable, so sizes are rounded up to an eighth of the power of two
+// below (12.5% at most).
+size_t block_size(size_t n) {
+    if (n > DEV_BLOCK_MAX) return n;
+    if (n <= 4096) return 4096;
+    const size_t step = ((size_t)1 << (63 - __builtin_clzll(n))) / 8;
+    return (n + step - 1) / step * step;
+}
+std::mutex g_blocks_mu;
+std::vector<DevBlock> g_blocks;  // oldest first
+size_t g_blocks_bytes = 0;
+
+bool find_block(size_t size, int device, DevBlock* out) {
+    std::lock_guard<std::mutex> lk(g_blocks_mu);
+    for (size_t i = g_blocks.size(); i-- > 0;)
+        if (g_blocks[i].size == size && g_blocks[i].device == device) {
+            *out = g_blocks[i];
+            g_blocks.erase(g_blocks.begin() + (ptrdiff_t)i);
+            g_blocks_bytes -= size;
+            return true;
+        }
+    return false;
+}
+// Frees kept blocks, oldest first, until at most `keep` bytes are left.
+void drop_blocks(size_t keep) {
+    while (true) {
+        DevBlock b;
+        {
+            std::lock_guard<std::mutex> lk(g_blocks_mu);
+            if (g_blocks.empty() || g_blocks_bytes <= keep) return;
+            b = g_blocks.front();
+            g_blocks.erase(g_blocks.begin());
+            g_blocks_bytes -= b.size;
+        }
+        (void)hipFree(b.p);
+    }
+}
+}  // namespace
+
+hipError_t take_dev_block(size_t bytes, DevBlock* out) {
+    DevBlock b;
+    b.size = block_size(bytes);
+    (void)hipGetDevice(&b.device);
+    if (b.size <= DEV_BLOCK_MAX && find_block(b.size, b.device, out)) return hipSuccess;
+    hipError_t e = hipMalloc(&b.p, b.size);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        drop_blocks(0);
+        e = hipMalloc(&b.p, b.size);
+    }
+    if (e == hipSuccess) *out = b;
+    return e;
+}
+
+void free_dev_block(const DevBlock& b) {
+    int cur = -1;
+    if (b.size <= DEV_BLOCK_MAX && hipGetDevice(&cur) == hipSuccess && cur == b.device &&
+        hipDeviceSynchronize() == hipSuccess) {
+        bool kept = false;
+        try {
+            std::lock_guard<std::mutex> lk(g_blocks_mu);
+            g_blocks.push_back(b);
+            g_blocks_bytes += b.size;
+            kept = true;
+        } catch (const std::exception&) {
+        }
+        if (kept) {
+            drop_blocks(DEV_KEPT_MAX);
+            return;
+        }
+    }
+    (void)hipFree(b.p);
 }
 
 // ---------------------------------------------------------------- pinned rings (hostcopy.hpp)
@@ -171,6 +248,37 @@ extern "C" eeg_status eeg_graph_create_device(const uint32_t* d_src, const uint3
     return EEG_OK;
 }
 
+// Host arrays to device memory on the graph's stream, finished on return.
+struct Upload {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+static eeg_status upload(eeg_graph* g, std::initializer_list<Upload> parts) {
+    size_t total = 0;
+    for (const Upload& u : parts) total += u.bytes;
+    LentRing lent(g->device, total >= HOST_COPY_FROM);
+    if (!lent.r) {
+        for (const Upload& u : parts)
+            if (u.bytes) EEG_HIP(hipMemcpyAsync(u.dst, u.src, u.bytes, hipMemcpyHostToDevice, g->stream));
+        EEG_HIP(hipStreamSynchronize(g->stream));
+        return EEG_OK;
+    }
+    // slots hold runs of one array each
+    std::vector<Upload> chunks;
+    chunks.reserve(total / HOST_SLOT_BYTES + parts.size());
+    for (const Upload& u : parts)
+        for (size_t o = 0; o < u.bytes; o += HOST_SLOT_BYTES)
+            chunks.push_back(Upload{(uint8_t*)u.dst + o, (const uint8_t*)u.src + o, std::min(HOST_SLOT_BYTES, u.bytes - o)});
+    return stage_to_device(
+        *lent.r, g->stream, (uint32_t)chunks.size(), host_copy_threads(total),
+        [&](uint32_t i, void* slot) { memcpy(slot, chunks[i].src, chunks[i].bytes); },
+        [&](uint32_t i, const void* slot) -> eeg_status {
+            EEG_HIP(hipMemcpyAsync(chunks[i].dst, slot, chunks[i].bytes, hipMemcpyHostToDevice, g->stream));
+            return EEG_OK;
+        });
+}
+
 extern "C" eeg_status eeg_graph_create(const uint32_t* src, const uint32_t* dst,
                                        const uint32_t* w, uint64_t m, uint32_t n, int device,
                                        eeg_graph** out) {
@@ -187,11 +295,7 @@ extern "C" eeg_status eeg_graph_create(const uint32_t* src, const uint32_t* dst,
         if (s == EEG_OK) s = dd.alloc(m * 4 + 4);
         if (s == EEG_OK && w) s = dw.alloc(m * 4 + 4);
         if (s == EEG_OK && m) {
-            hipError_t e = hipMemcpyAsync(ds.p, src, m * 4, hipMemcpyHostToDevice, g->stream);
-            if (e == hipSuccess) e = hipMemcpyAsync(dd.p, dst, m * 4, hipMemcpyHostToDevice, g->stream);
-            if (e == hipSuccess && w) e = hipMemcpyAsync(dw.p, w, m * 4, hipMemcpyHostToDevice, g->stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(g->stream);
-            if (e != hipSuccess) s = fail(EEG_ERR_DEVICE, "edge upload failed: %s", hipGetErrorString(e));
+            s = upload(g, {{ds.p, src, m * 4}, {dd.p, dst, m * 4}, {dw.p, w, w ? m * 4 : 0}});
         }
         if (s == EEG_OK)
             s = build_csr_from_device_edges(g, ds.as<uint32_t>(), dd.as<uint32_t>(),

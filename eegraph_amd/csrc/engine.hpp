@@ -7,6 +7,7 @@
 #include <cstdint>
 #include <memory>
 #include <mutex>
+#include <utility>
 #include <vector>
 
 #include "device.hpp"
@@ -23,6 +24,21 @@
 
 namespace eeg {
 
+// Device memory behind DevMem: blocks of up to DEV_BLOCK_MAX bytes are kept when they are freed, at
+// most DEV_KEPT_MAX in all, and handed out again (a hipFree of 64 MiB takes 0.33 ms and a hipMalloc
+// 0.07; building a graph of 16.8 M edges, one query and the end of the handle spent 9 of 21 ms in
+// them).  Freeing waits for the device, as hipFree does, so a block handed out again has no users
+// on any stream.  When memory runs out, what is kept is freed and the request repeated.
+constexpr size_t DEV_BLOCK_MAX = (size_t)256 << 20;
+constexpr size_t DEV_KEPT_MAX = (size_t)1 << 30;
+struct DevBlock {
+    void* p = nullptr;
+    size_t size = 0;  // of the block; what was asked for or more
+    int device = 0;
+};
+hipError_t take_dev_block(size_t bytes, DevBlock* out);
+void free_dev_block(const DevBlock& b);
+
 // Owning device allocation.
 struct DevMem {
     void* p = nullptr;
@@ -32,7 +48,7 @@ struct DevMem {
     DevMem& operator=(const DevMem&) = delete;
     ~DevMem() { release(); }
     void release() {
-        if (p) (void)hipFree(p);
+        if (p) free_dev_block(block);
         p = nullptr;
         bytes = 0;
     }
@@ -40,17 +56,25 @@ struct DevMem {
         if (p && bytes >= n && n > 0) return EEG_OK;
         release();
         if (n == 0) n = 8;
-        hipError_t e = hipMalloc(&p, n);
+        hipError_t e = take_dev_block(n, &block);
         if (e != hipSuccess) {
-            p = nullptr;
             (void)hipGetLastError();
             return fail(EEG_ERR_OOM, "hipMalloc(%zu) failed: %s", n, hipGetErrorString(e));
         }
+        p = block.p;
         bytes = n;
         return EEG_OK;
     }
+    void swap(DevMem& o) {
+        std::swap(p, o.p);
+        std::swap(bytes, o.bytes);
+        std::swap(block, o.block);
+    }
     template <class T>
     T* as() const { return static_cast<T*>(p); }
+
+private:
+    DevBlock block;
 };
 
 // Compressed sparse rows of one edge direction.

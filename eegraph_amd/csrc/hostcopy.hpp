@@ -1,9 +1,10 @@
-// Large answers on their way to a caller's host memory.
+// Large answers on their way to a caller's host memory, and large edge lists on their way from it.
 //
 // What bounds it: hipMemcpy into pageable memory moves 256 MiB in 16 ms where the pages exist and in
 // 26 ms where the caller has just allocated them (one thread copies and takes the page faults); PCIe
 // takes 5 ms of that.  So a kernel writes an answer in slots of pinned memory, in the order and layout
 // the caller wants, and several threads copy finished slots out while the next ones are written.
+// Towards the device the threads fill the slots (192 MiB of edges: 8.2 ms as plain copies).
 #pragma once
 
 #include <algorithm>
@@ -113,6 +114,71 @@ eeg_status stage_to_host(HostRing& ring, hipStream_t s, uint32_t chunks, unsigne
     if (rc != EEG_OK) {
         stop.store(true);
         (void)hipStreamSynchronize(s);  // what is queued writes to the slots
+    }
+    for (auto& t : pool) t.join();
+    return rc;
+}
+
+// The other way: fill(i, slot) writes chunk i into its slot on one of `threads` threads, consume(i,
+// slot) queues on stream s, in order, what reads the slot.  Returns when all of it has been read.
+template <class Fill, class Consume>
+eeg_status stage_to_device(HostRing& ring, hipStream_t s, uint32_t chunks, unsigned threads, Fill fill,
+                           Consume consume) {
+    std::atomic<uint32_t> freed{0}, filled[HOST_SLOTS];  // filled: one past the chunk in the slot
+    std::atomic<unsigned> team{0};
+    std::atomic<bool> stop{false};
+    for (auto& f : filled) f.store(0, std::memory_order_relaxed);
+    auto work = [&](unsigned w) {
+        unsigned nw;
+        while (!(nw = team.load(std::memory_order_acquire))) __builtin_ia32_pause();
+        for (uint32_t i = w; i < chunks; i += nw) {
+            for (uint32_t spins = 1; i >= freed.load(std::memory_order_acquire) + HOST_SLOTS; ++spins) {
+                if (stop.load(std::memory_order_relaxed)) return;
+                if (spins % 64) __builtin_ia32_pause();
+                else std::this_thread::yield();
+            }
+            fill(i, ring.slot(i));
+            filled[i % HOST_SLOTS].store(i + 1, std::memory_order_release);
+        }
+    };
+    std::vector<std::thread> pool;
+    unsigned started = 0;
+    try {
+        pool.reserve(threads);
+        for (; started < threads; ++started) pool.emplace_back(work, started);
+    } catch (const std::exception&) {  // fewer threads, or none, do as well
+    }
+    team.store(std::max(1u, started), std::memory_order_release);
+    eeg_status rc = EEG_OK;
+    uint32_t queued = 0, done = 0;
+    while (rc == EEG_OK && done < chunks) {
+        if (!started && queued < chunks && queued < done + HOST_SLOTS) {
+            fill(queued, ring.slot(queued));
+            filled[queued % HOST_SLOTS].store(queued + 1, std::memory_order_relaxed);
+        }
+        if (queued < chunks && filled[queued % HOST_SLOTS].load(std::memory_order_acquire) == queued + 1) {
+            rc = consume(queued, ring.slot(queued));
+            if (rc == EEG_OK && hipEventRecord(ring.ev[queued % HOST_SLOTS], s) != hipSuccess)
+                rc = fail(EEG_ERR_DEVICE, "hipEventRecord failed");
+            if (rc != EEG_OK) break;
+            ++queued;
+        }
+        if (done < queued) {
+            const hipError_t e = hipEventQuery(ring.ev[done % HOST_SLOTS]);
+            if (e == hipSuccess) {
+                freed.store(++done, std::memory_order_release);
+            } else if (e != hipErrorNotReady) {
+                rc = fail(EEG_ERR_DEVICE, "copy to the device failed: %s", hipGetErrorString(e));
+                break;
+            } else {
+                (void)hipGetLastError();  // "not ready" is no error of the next launch
+            }
+        }
+        __builtin_ia32_pause();
+    }
+    if (rc != EEG_OK) {
+        stop.store(true);
+        (void)hipStreamSynchronize(s);  // what is queued reads the slots
     }
     for (auto& t : pool) t.join();
     return rc;

@@ -88,10 +88,7 @@ struct Packed {
 // of it (a hipFree and hipMalloc of 1 GiB take milliseconds).  Only for memory whose size is
 // checked where it is used.
 void carry(DevMem& from, DevMem& to, uint64_t need) {
-    if (from.p && from.bytes / 4 <= need) {
-        std::swap(from.p, to.p);
-        std::swap(from.bytes, to.bytes);
-    }
+    if (from.p && from.bytes / 4 <= need) from.swap(to);
 }
 
 std::mutex g_pack_mu;
