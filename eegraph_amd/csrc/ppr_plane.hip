@@ -6,9 +6,9 @@
 // pass over the in-edge CSR reads each source index once for all B queries and gathers one
 // B-float row per in-edge instead of B separate 4-byte words.
 //
-// Work decomposition: the in-edges of every vertex are cut into segments of at most 64; a
-// group of B lanes (one per column) sums one segment in edge order with compensated FP32
-// (TwoSum), WAVE/B segments per wavefront.  A vertex with one segment is finished at once;
+// Work decomposition: the in-edges of every vertex are cut into segments of at most 64; four
+// lanes (a quarter of the columns each) sum one segment in edge order with compensated FP32
+// (TwoSum), 16 segments per wavefront.  A vertex with one segment is finished at once;
 // the partial sums of longer vertices go to spill slots and a second pass adds them in segment
 // order; a hub's (more than PPR_HUB_SEGS segments) are first added in chunks of PPR_HUB_SEGS
 // segments by separate groups, then the chunk sums in order.  The order of every sum is fixed,
@@ -133,21 +133,27 @@ struct PlaneArgsP {
 };
 
 // Old rank of entry vertex v in column q (x0 = e_src for a fresh column, nothing read).
-template <int B>
 __device__ __forceinline__ float2 old_rank(const PlaneArgsP& a, uint32_t v, uint32_t q, uint32_t src, bool fresh) {
     return fresh ? make_float2(v == src ? 1.0f : 0.0f, 0.0f) : a.x_old[(uint64_t)v * a.S + q];
 }
 
-// New rank of entry vertex v in column q from its gathered sum; adds the L1 change to res.
-template <int B>
+// New rank (hi, lo) from its gathered sum and the old one; adds the L1 change to res and returns
+// the new contribution.
+__device__ __forceinline__ float new_rank(float damping, bool restart, uint32_t od, float2 xo, Comp sum, float* hi,
+                                          float* lo, double& res) {
+    rank_pair(restart ? 1.0f - damping : 0.0f, damping, sum, hi, lo);
+    res += fabs(((double)*hi + (double)*lo) - ((double)xo.x + (double)xo.y));
+    return od ? (*hi + *lo) / (float)od : 0.0f;
+}
+
+// ... of entry vertex v in column q, written to the planes.
 __device__ __forceinline__ void finish_col(const PlaneArgsP& a, uint32_t v, uint32_t q, uint32_t src, float2 xo,
                                            uint32_t od, Comp sum, double& res) {
     float hi, lo;
-    rank_pair(v == src ? 1.0f - a.damping : 0.0f, a.damping, sum, &hi, &lo);
+    const float c = new_rank(a.damping, v == src, od, xo, sum, &hi, &lo, res);
     const uint64_t o = (uint64_t)v * a.S + q;
     a.x_new[o] = make_float2(hi, lo);
-    a.c_new[o] = od ? (hi + lo) / (float)od : 0.0f;
-    res += fabs(((double)hi + (double)lo) - ((double)xo.x + (double)xo.y));
+    a.c_new[o] = c;
 }
 
 // Per-column FP64 residual of a workgroup: lanes q, q+B, ... of every wave, in a fixed order.
@@ -166,52 +172,120 @@ __device__ __forceinline__ void store_residual(double res, double* __restrict__ 
     }
 }
 
+// The gather: bound by the lines of the contribution rows in flight (64 B an edge at 16 columns).
+// Four lanes share a segment, a quarter of its columns each in vectors of up to four, so a
+// wavefront keeps the rows of 16 segments in flight; the quad loads four source indices at once and
+// hands them round by DPP.  (A lane per column kept 4 segments' rows in flight at 16 columns, and
+// every lane of a group loaded the same index: an iteration of 16 columns on RMAT-18 / RMAT-20 took
+// 118 / 373 us and takes 84 / 255, of 32 columns on RMAT-20 792 and 357.)
+constexpr int PQ = 4;                  // lanes per segment
+constexpr int PQ_EDGES = 4;            // rows in flight per segment
+template <int K>
+__device__ __forceinline__ uint32_t quad_lane(uint32_t x) {  // the value of lane K of the quad
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, K * 0x55, 0xf, 0xf, true);
+}
 template <int B>
 __global__ __launch_bounds__(WG) void k_pps_pull(PlaneArgsP a) {
-    constexpr int G = WAVE / B;  // segments per wavefront
-    const uint32_t lane = lane_id(), q = lane % B, grp = lane / B;
-    const uint32_t src = a.cols.src[q];
-    const bool fresh = (a.cols.fresh >> q) & 1u;
-    // a fresh column's contributions are e_src / outdeg(src): nothing is read for it
-    const uint32_t sod = (src != PPR_IDLE) ? a.outdeg[src] : 0u;
-    const float c0 = sod ? 1.0f / (float)sod : 0.0f;
-    double res = 0.0;
+    constexpr int C = B / PQ;            // columns per lane
+    constexpr int VW = C < 4 ? C : 4;    // ... in C / VW vectors, neighbouring lanes side by side
+    constexpr int G = WAVE / PQ;         // segments per wavefront
+    typedef float vec __attribute__((ext_vector_type(VW)));
+    typedef float vec2 __attribute__((ext_vector_type(2 * VW)));  // pairs of VW columns (16-byte parts)
+    const uint32_t lane = lane_id(), sub = lane % PQ, grp = lane / PQ;
+    uint32_t src[C], fresh = 0;
+    float c0[C];
+    double res[C];
+    auto col = [&](int i) { return (uint32_t)(i / VW * PQ * VW + i % VW) + sub * VW; };
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+        src[i] = a.cols.src[col(i)];
+        // a fresh column's contributions are e_src / outdeg(src): what is read for it is dropped
+        fresh |= ((a.cols.fresh >> col(i)) & 1u) << i;
+        const uint32_t sod = (src[i] != PPR_IDLE) ? a.outdeg[src[i]] : 0u;
+        c0[i] = sod ? 1.0f / (float)sod : 0.0f;
+        res[i] = 0.0;
+    }
     const uint64_t nw = (uint64_t)gridDim.x * (WG / WAVE);
     for (uint64_t w = (uint64_t)blockIdx.x * (WG / WAVE) + threadIdx.x / WAVE; w * G < a.nseg; w += nw) {
         const uint64_t t = w * G + grp;
-        if (t >= a.nseg) continue;
+        if (t >= a.nseg) continue;  // whole quads
         const uint4 dsc = a.sdesc[t];
         const uint32_t e0 = dsc.x, len = dsc.y & 0x7fffffffu, v = dsc.z;
         const bool single = (dsc.y >> 31) != 0;
-        // what finishing the vertex reads is loaded before the gathers, so its latency overlaps
-        float2 xo = make_float2(0.0f, 0.0f);
-        uint32_t od = 0;
-        if (single) {
-            xo = old_rank<B>(a, v, q, src, fresh);
-            od = a.outdeg[v];
-        }
-        Comp acc{0.0f, 0.0f};
-        // source indices of the next 8 edges are loaded while the current 8 rows are gathered
-        uint32_t u[8];
+        Comp acc[C];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) u[k] = ((uint32_t)k < len) ? a.col[e0 + k] : PPR_IDLE;
-        for (uint32_t b = 0; b < len; b += 8) {
-            float cv[8];
+        for (int i = 0; i < C; ++i) acc[i] = Comp{0.0f, 0.0f};
+        uint32_t mine = sub < len ? a.col[e0 + sub] : 0u;
+        for (uint32_t b = 0; b < len; b += PQ_EDGES) {
+            const uint32_t u[PQ_EDGES] = {quad_lane<0>(mine), quad_lane<1>(mine), quad_lane<2>(mine), quad_lane<3>(mine)};
+            vec cv[PQ_EDGES][C / VW];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                if (fresh) cv[k] = (u[k] == src) ? c0 : 0.0f;
-                else cv[k] = (u[k] != PPR_IDLE) ? a.c_old[(uint64_t)u[k] * a.S + q] : 0.0f;
+            for (int k = 0; k < PQ_EDGES; ++k)
+#pragma unroll
+                for (int j = 0; j < C / VW; ++j)  // past the last edge: row 0, dropped
+                    cv[k][j] = *reinterpret_cast<const vec*>(a.c_old + (uint64_t)u[k] * a.S + col(j * VW));
+            if (b + PQ_EDGES + sub < len) mine = a.col[e0 + b + PQ_EDGES + sub];
+            else mine = 0u;
+#pragma unroll
+            for (int k = 0; k < PQ_EDGES; ++k) {
+                if (b + k >= len) break;
+#pragma unroll
+                for (int i = 0; i < C; ++i) {
+                    float x = cv[k][i / VW][i % VW];
+                    if ((fresh >> i) & 1u) x = u[k] == src[i] ? c0[i] : 0.0f;
+                    acc[i] = comp_add(acc[i], Comp{x, 0.0f});
+                }
             }
-#pragma unroll
-            for (int k = 0; k < 8; ++k) u[k] = (b + 8 + k < len) ? a.col[e0 + b + 8 + k] : PPR_IDLE;
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                if (b + k < len) acc = comp_add(acc, Comp{cv[k], 0.0f});
         }
-        if (single) finish_col<B>(a, v, q, src, xo, od, acc, res);
-        else a.spill[(uint64_t)dsc.w * a.S + q] = make_float2(acc.s, acc.e);
+        if (single) {
+            const uint32_t od = a.outdeg[v];
+#pragma unroll
+            for (int j = 0; j < C / VW; ++j) {
+                const uint64_t o = (uint64_t)v * a.S + col(j * VW);
+                const vec2 xo = *reinterpret_cast<const vec2*>(a.x_old + o);
+                vec2 xn;
+                vec cn;
+#pragma unroll
+                for (int i = 0; i < VW; ++i) {
+                    const int f = j * VW + i;
+                    const float2 old = ((fresh >> f) & 1u) ? make_float2(v == src[f] ? 1.0f : 0.0f, 0.0f)
+                                                           : make_float2(xo[2 * i], xo[2 * i + 1]);
+                    float hi, lo;
+                    cn[i] = new_rank(a.damping, v == src[f], od, old, acc[f], &hi, &lo, res[f]);
+                    xn[2 * i] = hi;
+                    xn[2 * i + 1] = lo;
+                }
+                *reinterpret_cast<vec2*>(a.x_new + o) = xn;
+                *reinterpret_cast<vec*>(a.c_new + o) = cn;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < C / VW; ++j) {
+                vec2 p;
+#pragma unroll
+                for (int i = 0; i < VW; ++i) {
+                    p[2 * i] = acc[j * VW + i].s;
+                    p[2 * i + 1] = acc[j * VW + i].e;
+                }
+                *reinterpret_cast<vec2*>(a.spill + (uint64_t)dsc.w * a.S + col(j * VW)) = p;
+            }
+        }
     }
-    store_residual<B>(res, a.res_part);
+    // L1 change per column of the workgroup: over the segments of a wave by a fixed tree, then wave
+    // by wave
+    __shared__ double sRed[WG / WAVE][B];
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+#pragma unroll
+        for (int off = PQ; off < WAVE; off <<= 1) res[i] += __shfl_xor(res[i], off, WAVE);
+        if (lane < PQ) sRed[threadIdx.x / WAVE][col(i)] = res[i];
+    }
+    __syncthreads();
+    if (threadIdx.x < B) {
+        double t = 0;
+        for (int w = 0; w < WG / WAVE; ++w) t += sRed[w][threadIdx.x];
+        a.res_part[(uint64_t)blockIdx.x * B + threadIdx.x] = t;
+    }
 }
 
 // cnt compensated partials at p, p + stride, ... added in order.  A hub has thousands of
@@ -277,14 +351,14 @@ __global__ __launch_bounds__(WG) void k_pps_fix(PlaneArgsP a, double* res_part) 
         const uint32_t i = a.mlist[j];
         const uint32_t ns = a.sscan[i + 1] - a.sscan[i], mb = a.mbase[i];
         const uint32_t v = a.ent[i];
-        const float2 xo = old_rank<B>(a, v, q, src, fresh);
+        const float2 xo = old_rank(a, v, q, src, fresh);
         const uint32_t od = a.outdeg[v];
         // a hub's chunk sums sit every PPR_HUB_SEGS slots (k_pps_hub_chunks)
         const bool hub = a.hub_chunks && ns > PPR_HUB_SEGS;
         const uint32_t cnt = hub ? (ns + PPR_HUB_SEGS - 1) / PPR_HUB_SEGS : ns;
         const uint64_t stride = hub ? (uint64_t)PPR_HUB_SEGS * a.S : (uint64_t)a.S;
         const Comp acc = sum_slots<B>(a.spill + (uint64_t)mb * a.S + q, cnt, stride);
-        finish_col<B>(a, v, q, src, xo, od, acc, res);
+        finish_col(a, v, q, src, xo, od, acc, res);
     }
     store_residual<B>(res, res_part);
 }
@@ -436,7 +510,7 @@ eeg_status PprPlane::init(eeg_graph* g, uint32_t Bc, float d, hipStream_t s) {
     EEG_TRY(spill.alloc((size_t)t.nspill * B * 8 + 16));
     int cus = 256;
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->device);
-    grid_pull = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)cus * 8, ((uint64_t)t.nseg + 15) / 16));
+    grid_pull = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)cus * 8, ((uint64_t)t.nseg + 63) / 64));
     grid_fix = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)cus * 4, ((uint64_t)t.nmulti + 15) / 16));
     EEG_TRY(res_part.alloc((size_t)(grid_pull + grid_fix) * B * 8));
     EEG_TRY(resid.alloc((size_t)B * 8));
