@@ -944,8 +944,9 @@ __global__ void k_plane_rotate(const uint32_t* q, const Ctl* ctl, int slot,
         atomicOr((unsigned long long*)&act[threadIdx.x], sAct[threadIdx.x]);
 }
 
-// out[q * stride + i] = planes[perm[i] * B + q] for q < nq, i < count: answers in query-major,
-// original vertex order, narrow labels widened (their all-ones INF to INF).
+// Answers of vertices 0 .. count-1 of `perm` in query-major order, narrow labels widened (their
+// all-ones INF to INF): planes[perm[i] * B + q] for q < nq.  They go out in parts of `per` vertices (a
+// multiple of 64, or all), `pitch` words from part to part: rows of one part follow each other.
 //
 // Bound by memory traffic: a vertex's labels are one contiguous row and a query's answers are
 // another, so a tile of 64 vertices x 64 queries goes through LDS and both sides move whole lines
@@ -955,7 +956,8 @@ constexpr uint32_t OUT_TILE = 64;
 template <int LM>
 __global__ __launch_bounds__(WG) void k_planes_out(const uint32_t* __restrict__ planes,
                                                    const uint32_t* __restrict__ perm, uint32_t count, uint32_t B,
-                                                   uint32_t nq, uint64_t stride, uint32_t* __restrict__ out) {
+                                                   uint32_t nq, uint32_t per, uint64_t pitch,
+                                                   uint32_t* __restrict__ out) {
     constexpr uint32_t QPL = (LM == LM_W8 || LM == LM_D8) ? 4 : LM == LM_D16 ? 2 : 1;  // labels per word
     constexpr uint32_t WORDS = OUT_TILE / QPL;                                         // words per vertex
     __shared__ uint32_t sL[OUT_TILE][OUT_TILE + 1];  // [query][vertex]
@@ -978,10 +980,12 @@ __global__ __launch_bounds__(WG) void k_planes_out(const uint32_t* __restrict__ 
             }
         }
         __syncthreads();
-        const uint32_t u = threadIdx.x % OUT_TILE;
+        const uint32_t u = threadIdx.x % OUT_TILE, part = u0 / per, first = part * per;
+        const uint32_t stride = min(per, count - first);
+        uint32_t* dst = out + part * pitch + (u0 - first);
         if (u < nu)
             for (uint32_t q = threadIdx.x / OUT_TILE; q < OUT_TILE && q0 + q < nq; q += WG / OUT_TILE)
-                out[(uint64_t)(q0 + q) * stride + u0 + u] = sL[q][u];
+                dst[(uint64_t)(q0 + q) * stride + u] = sL[q][u];
         __syncthreads();
     }
 }
@@ -1581,19 +1585,19 @@ eeg_status batch_pass(eeg_graph* g, BatchWork& bw, hipStream_t s, uint32_t algo,
         if (lm == LM_D8) EEG_HIP(hipMemcpyAsync(ovq_out, bw.ovq.p, MAXW * 8, hipMemcpyDeviceToHost, s));
     }
     // answers: query-major, original vertex order
-    auto planes_out = [&](uint32_t u0, uint32_t count, uint64_t stride, uint32_t* dst) -> eeg_status {
+    auto planes_out = [&](uint32_t u0, uint32_t count, uint32_t per, uint64_t pitch, uint32_t* dst) -> eeg_status {
         const dim3 gr(std::max(1u, std::min(4096u, (count + OUT_TILE - 1) / OUT_TILE)), W);
         const uint32_t* pl = bw.planes.as<uint32_t>();
         const uint32_t* pm = g->perm.as<uint32_t>() + u0;
-        if (lm == LM_W8) k_planes_out<LM_W8><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, stride, dst);
-        else if (lm == LM_D8) k_planes_out<LM_D8><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, stride, dst);
-        else if (lm == LM_D16) k_planes_out<LM_D16><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, stride, dst);
-        else k_planes_out<LM_U32><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, stride, dst);
+        if (lm == LM_W8) k_planes_out<LM_W8><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, per, pitch, dst);
+        else if (lm == LM_D8) k_planes_out<LM_D8><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, per, pitch, dst);
+        else if (lm == LM_D16) k_planes_out<LM_D16><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, per, pitch, dst);
+        else k_planes_out<LM_U32><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, per, pitch, dst);
         EEG_HIP(hipGetLastError());
         return EEG_OK;
     };
     if (bo.out && bo.device) {
-        EEG_TRY(planes_out(0, n, n, (uint32_t*)bo.out));
+        EEG_TRY(planes_out(0, n, n, 0, (uint32_t*)bo.out));
     } else if (bo.out || bo.rows) {
         auto row = [&](uint32_t q) { return bo.rows ? bo.rows[q] : (uint32_t*)bo.out + (uint64_t)q * n; };
         const uint64_t bytes = (uint64_t)nsrc * n * 4;
@@ -1607,7 +1611,10 @@ eeg_status batch_pass(eeg_graph* g, BatchWork& bw, hipStream_t s, uint32_t algo,
             auto part = [&](uint32_t i) { return std::min(per, n - i * per); };
             EEG_TRY(stage_to_host(
                 *lent.r, s, chunks, threads, nsrc < threads,
-                [&](uint32_t i, void* slot) { return planes_out(i * per, part(i), part(i), (uint32_t*)slot); },
+                [&](uint32_t i, uint32_t count, void* slot) {
+                    return planes_out(i * per, (count - 1) * per + part(i + count - 1), per, HOST_SLOT_BYTES / 4,
+                                      (uint32_t*)slot);
+                },
                 [&](uint32_t i, const void* slot, unsigned w, unsigned nw) {
                     const uint32_t cnt = part(i);
                     const uint32_t qa = (uint32_t)((uint64_t)w * nsrc / nw), qb = (uint32_t)((uint64_t)(w + 1) * nsrc / nw);
@@ -1617,7 +1624,7 @@ eeg_status batch_pass(eeg_graph* g, BatchWork& bw, hipStream_t s, uint32_t algo,
                 }));
         } else {
             EEG_TRY(bw.rowbuf.alloc(bytes + 4));
-            EEG_TRY(planes_out(0, n, n, bw.rowbuf.as<uint32_t>()));
+            EEG_TRY(planes_out(0, n, n, 0, bw.rowbuf.as<uint32_t>()));
             if (bo.out) {
                 EEG_HIP(hipMemcpyAsync(bo.out, bw.rowbuf.p, bytes, hipMemcpyDeviceToHost, s));
             } else {

@@ -273,8 +273,17 @@ static eeg_status upload(eeg_graph* g, std::initializer_list<Upload> parts) {
     return stage_to_device(
         *lent.r, g->stream, (uint32_t)chunks.size(), host_copy_threads(total),
         [&](uint32_t i, void* slot) { memcpy(slot, chunks[i].src, chunks[i].bytes); },
-        [&](uint32_t i, const void* slot) -> eeg_status {
-            EEG_HIP(hipMemcpyAsync(chunks[i].dst, slot, chunks[i].bytes, hipMemcpyHostToDevice, g->stream));
+        [&](uint32_t i, uint32_t count, const void* slot) -> eeg_status {
+            // neighbours of one array in one copy (all but an array's last chunk fill their slots)
+            for (uint32_t k = 0; k < count;) {
+                uint32_t e = k + 1;
+                size_t bytes = chunks[i + k].bytes;
+                for (; e < count && chunks[i + e].dst == (uint8_t*)chunks[i + k].dst + (e - k) * HOST_SLOT_BYTES; ++e)
+                    bytes += chunks[i + e].bytes;
+                EEG_HIP(hipMemcpyAsync(chunks[i + k].dst, (const uint8_t*)slot + k * HOST_SLOT_BYTES, bytes,
+                                       hipMemcpyHostToDevice, g->stream));
+                k = e;
+            }
             return EEG_OK;
         });
 }
@@ -450,7 +459,9 @@ static eeg_status labels_to_host(eeg_graph* g, const void* lab, void* out, DevMe
         auto part = [&](uint32_t i) { return std::min(words, n - i * words); };
         return stage_to_host(
             *lent.r, st, chunks, host_copy_threads(bytes), true,
-            [&](uint32_t i, void* slot) { return unpermute(g, lab, slot, st, i * words, part(i)); },
+            [&](uint32_t i, uint32_t count, void* slot) {
+                return unpermute(g, lab, slot, st, i * words, (count - 1) * words + part(i + count - 1));
+            },
             [&](uint32_t i, const void* slot, unsigned, unsigned) {
                 memcpy((uint32_t*)out + (size_t)i * words, slot, (size_t)part(i) * 4);
             });

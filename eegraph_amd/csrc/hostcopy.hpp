@@ -18,10 +18,14 @@
 namespace eeg {
 
 // Slots of pinned memory and an event for each.  Rings are lent by a pool that keeps at most
-// HOST_RINGS_KEPT of them between calls (pinning 16 MiB takes about 3 ms).
-constexpr uint32_t HOST_SLOTS = 8;
+// HOST_RINGS_KEPT of them between calls (pinning 32 MiB takes milliseconds).
+constexpr uint32_t HOST_SLOTS = 16;
 constexpr size_t HOST_SLOT_BYTES = (size_t)2 << 20;
 constexpr size_t HOST_RINGS_KEPT = 2;
+// Slots, neighbours in the ring, that one launch or copy covers at most: each costs about 13 us
+// beyond its transfer (256 MiB in 128 launches 6.8 ms, in 32 5.5).  Threads take single slots.
+constexpr uint32_t HOST_GROUP = 4;
+constexpr unsigned HOST_THREADS = 8;
 struct HostRing {
     int device = 0;
     uint8_t* base = nullptr;
@@ -38,12 +42,19 @@ void give_host_ring(HostRing* r);
 constexpr uint64_t HOST_COPY_FROM = (uint64_t)8 << 20;
 inline unsigned host_copy_threads(uint64_t bytes) {
     const unsigned hw = std::thread::hardware_concurrency();
-    const unsigned most = std::max(1u, std::min(HOST_SLOTS, hw / 2));
+    const unsigned most = std::max(1u, std::min(HOST_THREADS, hw / 2));
     return (unsigned)std::min<uint64_t>(most, std::max<uint64_t>(1, bytes / (2 * HOST_SLOT_BYTES)));
 }
 
-// Runs chunks 0 .. chunks-1 through the ring: produce(i, slot) queues on stream s what fills the slot
-// with chunk i, take(i, slot, w, nw) copies share w of nw of it to where it belongs, on one of
+// Chunks that go together from `first` on, not past the ring's end.  Few chunks make small groups,
+// so that the two sides still overlap.
+inline uint32_t host_group(uint32_t first, uint32_t chunks) {
+    const uint32_t most = std::max(1u, std::min(HOST_GROUP, chunks / 8));
+    return std::min(std::min(most, chunks - first), HOST_SLOTS - first % HOST_SLOTS);
+}
+
+// Runs chunks 0 .. chunks-1 through the ring: produce(i, count, slot) queues on stream s what fills
+// the slots from `slot` on with chunks i .. i + count - 1, take(i, slot, w, nw) copies share w of nw of it to where it belongs, on one of
 // `threads` threads.  `whole`: every chunk goes to one thread (nw = 1) rather than a share of it to
 // each; what a thread touches first should be pages that no other thread touches.
 template <class Produce, class Take>
@@ -82,22 +93,27 @@ eeg_status stage_to_host(HostRing& ring, hipStream_t s, uint32_t chunks, unsigne
     eeg_status rc = EEG_OK;
     uint32_t queued = 0, seen = 0, freed = 0;
     while (rc == EEG_OK && freed < chunks) {
-        while (queued < chunks && queued < freed + HOST_SLOTS) {
-            rc = produce(queued, ring.slot(queued));
-            if (rc == EEG_OK && hipEventRecord(ring.ev[queued % HOST_SLOTS], s) != hipSuccess)
+        while (queued < chunks) {
+            const uint32_t count = host_group(queued, chunks);
+            if (queued + count > freed + HOST_SLOTS) break;
+            rc = produce(queued, count, ring.slot(queued));
+            queued += count;
+            // the event of a group is that of its last slot
+            if (rc == EEG_OK && hipEventRecord(ring.ev[(queued - 1) % HOST_SLOTS], s) != hipSuccess)
                 rc = fail(EEG_ERR_DEVICE, "hipEventRecord failed");
             if (rc != EEG_OK) break;
-            ++queued;
         }
         if (rc != EEG_OK) break;
         if (seen < queued) {
-            const hipError_t e = hipEventQuery(ring.ev[seen % HOST_SLOTS]);
+            const uint32_t count = host_group(seen, chunks);
+            const hipError_t e = hipEventQuery(ring.ev[(seen + count - 1) % HOST_SLOTS]);
             if (e == hipSuccess) {
-                if (!started) {
-                    take(seen, ring.slot(seen), 0u, 1u);
-                    left[seen % HOST_SLOTS].store(0, std::memory_order_relaxed);
+                for (uint32_t i = seen; !started && i < seen + count; ++i) {
+                    take(i, ring.slot(i), 0u, 1u);
+                    left[i % HOST_SLOTS].store(0, std::memory_order_relaxed);
                 }
-                ready.store(++seen, std::memory_order_release);
+                seen += count;
+                ready.store(seen, std::memory_order_release);
             } else if (e != hipErrorNotReady) {
                 rc = fail(EEG_ERR_DEVICE, "copy to the host failed: %s", hipGetErrorString(e));
                 break;
@@ -120,7 +136,8 @@ eeg_status stage_to_host(HostRing& ring, hipStream_t s, uint32_t chunks, unsigne
 }
 
 // The other way: fill(i, slot) writes chunk i into its slot on one of `threads` threads, consume(i,
-// slot) queues on stream s, in order, what reads the slot.  Returns when all of it has been read.
+// count, slot) queues on stream s, in order, what reads the slots from `slot` on, which hold chunks i
+// .. i + count - 1.  Returns when all of it has been read.
 template <class Fill, class Consume>
 eeg_status stage_to_device(HostRing& ring, hipStream_t s, uint32_t chunks, unsigned threads, Fill fill,
                            Consume consume) {
@@ -151,22 +168,27 @@ eeg_status stage_to_device(HostRing& ring, hipStream_t s, uint32_t chunks, unsig
     team.store(std::max(1u, started), std::memory_order_release);
     eeg_status rc = EEG_OK;
     uint32_t queued = 0, done = 0;
+    uint32_t full = 0;  // chunks seen filled, in order
     while (rc == EEG_OK && done < chunks) {
-        if (!started && queued < chunks && queued < done + HOST_SLOTS) {
-            fill(queued, ring.slot(queued));
-            filled[queued % HOST_SLOTS].store(queued + 1, std::memory_order_relaxed);
+        if (!started && full < chunks && full < done + HOST_SLOTS) {
+            fill(full, ring.slot(full));
+            filled[full % HOST_SLOTS].store(full + 1, std::memory_order_relaxed);
         }
-        if (queued < chunks && filled[queued % HOST_SLOTS].load(std::memory_order_acquire) == queued + 1) {
-            rc = consume(queued, ring.slot(queued));
-            if (rc == EEG_OK && hipEventRecord(ring.ev[queued % HOST_SLOTS], s) != hipSuccess)
+        while (full < chunks && filled[full % HOST_SLOTS].load(std::memory_order_acquire) == full + 1) ++full;
+        if (queued < chunks && full >= queued + host_group(queued, chunks)) {
+            const uint32_t count = host_group(queued, chunks);
+            rc = consume(queued, count, ring.slot(queued));
+            queued += count;
+            if (rc == EEG_OK && hipEventRecord(ring.ev[(queued - 1) % HOST_SLOTS], s) != hipSuccess)
                 rc = fail(EEG_ERR_DEVICE, "hipEventRecord failed");
             if (rc != EEG_OK) break;
-            ++queued;
         }
         if (done < queued) {
-            const hipError_t e = hipEventQuery(ring.ev[done % HOST_SLOTS]);
+            const uint32_t count = host_group(done, chunks);
+            const hipError_t e = hipEventQuery(ring.ev[(done + count - 1) % HOST_SLOTS]);
             if (e == hipSuccess) {
-                freed.store(++done, std::memory_order_release);
+                done += count;
+                freed.store(done, std::memory_order_release);
             } else if (e != hipErrorNotReady) {
                 rc = fail(EEG_ERR_DEVICE, "copy to the device failed: %s", hipGetErrorString(e));
                 break;

@@ -276,8 +276,9 @@ extern "C" eeg_status eeg_run_packed(eeg_graph* const* graphs, uint32_t ngraphs,
             const uint32_t N = u->n, chunks = (uint32_t)(((uint64_t)N + words - 1) / words);
             EEG_TRY(stage_to_host(
                 *lent.r, s, chunks, host_copy_threads(bytes), true,
-                [&](uint32_t c, void* slot) -> eeg_status {
-                    EEG_HIP(hipMemcpyAsync(slot, outd + (size_t)c * words, (size_t)std::min(words, N - c * words) * 4,
+                [&](uint32_t c, uint32_t count, void* slot) -> eeg_status {
+                    EEG_HIP(hipMemcpyAsync(slot, outd + (size_t)c * words,
+                                           (size_t)std::min<uint64_t>((uint64_t)count * words, N - c * words) * 4,
                                            hipMemcpyDeviceToHost, s));
                     return EEG_OK;
                 },
