@@ -21,6 +21,7 @@
 #include "bytes8.hpp"
 #include "frontier.hpp"
 #include "hostcopy.hpp"
+#include "progress.hpp"
 
 namespace eeg {
 namespace {
@@ -34,38 +35,11 @@ unsigned grid_n(uint64_t work, unsigned cap = 16384) {
 }
 
 
-// Replayed graphs: the per-iteration arguments come from device memory (see MsArgs).
-__device__ __forceinline__ void ms_resolve(MsArgs& a, bool finalize) {
-    if (!a.dev_it) return;
-    const uint32_t lvl = a.dev_it[0];
-    const bool odd = ((lvl - 1) & 1) != 0;  // input frontier = buffer (level-1)&1
-    a.level = lvl;
-    a.stampv = a.dev_it[1] + lvl;
-    a.launch = finalize ? 2 * lvl : 2 * lvl - 1;
-    a.qin = odd ? a.qb : a.qa;
-    a.sin = odd ? a.sb : a.sa;
-    a.qout = odd ? a.qa : a.qb;
-    a.sout = odd ? a.sa : a.sb;
-}
-__device__ __forceinline__ void plane_resolve(PlaneArgs& a) {
-    if (!a.dev_it) return;
-    const uint32_t it = a.dev_it[0];
-    const bool odd = ((it - 1) & 1) != 0;
-    a.it = it;
-    a.stampv = a.dev_it[1] + it;
-    a.qin = odd ? a.qb : a.qa;
-    a.sin = odd ? a.sb : a.sa;
-    a.qout = odd ? a.qa : a.qb;
-    a.sout = odd ? a.sa : a.sb;
-}
-
 // ---------------------------------------------------------------- multi-source BFS
 template <int K>
 // At most 168 VGPRs (3 waves per SIMD, 8 bytes of spill per lane): -9% per pass against 200
 // VGPRs and 2 waves on RMAT-24 x 256; 4 waves spilled 136 bytes.
-__global__ __launch_bounds__(WG, 3) void k_ms_push(MsArgs args) {
-    MsArgs a = args;
-    ms_resolve(a, false);
+__global__ __launch_bounds__(WG, 3) void k_ms_push(MsArgs a) {
     constexpr int VPR = WG / K, TV = TILE_EDGES / K, ROUNDS = TILE_EDGES / WG, EMAX = TV + 2;
     __shared__ uint32_t sS[EMAX];
     __shared__ uint64_t sRow[EMAX];
@@ -81,10 +55,14 @@ __global__ __launch_bounds__(WG, 3) void k_ms_push(MsArgs args) {
     const uint32_t nE = (uint32_t)(pk & 0xffffffffull), T = (uint32_t)(pk >> 32);
     const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
     if (nE == 0 || T == 0) {
-        if (lead) ctl->done = 1;
+        if (lead) {
+            ctl->done = 1;
+            publish(a.status, ctl, a.level, RUN_DONE);
+        }
         return;
     }
     if (lead) {
+        publish(a.status, ctl, a.level, RUN_GOING);
         ctl->qpack[(a.launch + 1) % 3] = 0;
         ctl->iters = a.level;
     }
@@ -255,9 +233,7 @@ __global__ __launch_bounds__(WG, 3) void k_ms_push(MsArgs args) {
 // vertices with new bits (and out-edges) as the next frontier.  A thread per candidate updates
 // the masks; the levels are then written by whole wavefronts, lane = query, one contiguous row
 // store per (candidate, word) with new bits, instead of one scattered store per new bit.
-__global__ __launch_bounds__(WG) void k_ms_finalize(MsArgs args) {
-    MsArgs a = args;
-    ms_resolve(a, true);
+__global__ __launch_bounds__(WG) void k_ms_finalize(MsArgs a) {
     __shared__ uint64_t sScan[WG / WAVE + 1];
     __shared__ unsigned long long sBase;
     __shared__ unsigned long long sAct[MAXW];
@@ -270,7 +246,10 @@ __global__ __launch_bounds__(WG) void k_ms_finalize(MsArgs args) {
     const uint32_t count = (uint32_t)(ctl->qpack[(a.launch - 1) % 3] & 0xffffffffull);
     const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
     if (count == 0) {
-        if (lead) ctl->done = 1;
+        if (lead) {
+            ctl->done = 1;
+            publish(a.status, ctl, a.level + 1, RUN_DONE);
+        }
         return;
     }
     if (lead) ctl->qpack[(a.launch + 1) % 3] = 0;
@@ -382,9 +361,7 @@ template <int K, int LM, int G>
 // RMAT-24).  Narrow labels: at most 64 VGPRs, 8 waves per SIMD (from 4-5 waves at 85-118
 // VGPRs: 25-40% faster passes on RMAT-24 x 256).
 __global__ __launch_bounds__(WG, K <= 8 ? (LM == LM_U32 ? 7 : G == WAVE ? 8 : 7) : 1) void k_plane_push_wave(
-    PlaneArgs args) {
-    PlaneArgs a = args;
-    plane_resolve(a);
+    PlaneArgs a) {
     constexpr int TV = TILE_EDGES / K, EMAX = TV + 2, NW = WG / WAVE;
     __shared__ uint32_t sS[EMAX];
     __shared__ uint64_t sRow[EMAX];
@@ -401,10 +378,14 @@ __global__ __launch_bounds__(WG, K <= 8 ? (LM == LM_U32 ? 7 : G == WAVE ? 8 : 7)
     const uint32_t nE = (uint32_t)(pk & 0xffffffffull), T = (uint32_t)(pk >> 32);
     const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
     if (nE == 0 || T == 0) {
-        if (lead) ctl->done = 1;
+        if (lead) {
+            ctl->done = 1;
+            publish(a.status, ctl, a.it, RUN_DONE);
+        }
         return;
     }
     if (lead) {
+        publish(a.status, ctl, a.it, RUN_GOING);
         ctl->qpack[(a.it + 1) % 3] = 0;
         ctl->iters = a.it;
     }
@@ -675,9 +656,7 @@ constexpr uint32_t PLANE_DENSE_FROM = 16;
 template <int K>
 // At most 168 VGPRs at K <= 8 (3 waves per SIMD instead of 2 at ~193, ~116 B of spill): -10 to -12%
 // per pass for 8 and 16 queries on RMAT-24; 4 waves were no faster than 2.
-__global__ __launch_bounds__(WG, K <= 8 ? 3 : 1) void k_plane_push(PlaneArgs args) {
-    PlaneArgs a = args;
-    plane_resolve(a);
+__global__ __launch_bounds__(WG, K <= 8 ? 3 : 1) void k_plane_push(PlaneArgs a) {
     constexpr int TV = TILE_EDGES / K, EMAX = TV + 2, NW = WG / WAVE, VPR = WG / K;
     constexpr int ROUNDS = TILE_EDGES / WG;
     __shared__ uint32_t sS[EMAX];
@@ -696,10 +675,14 @@ __global__ __launch_bounds__(WG, K <= 8 ? 3 : 1) void k_plane_push(PlaneArgs arg
     const uint32_t nE = (uint32_t)(pk & 0xffffffffull), T = (uint32_t)(pk >> 32);
     const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
     if (nE == 0 || T == 0) {
-        if (lead) ctl->done = 1;
+        if (lead) {
+            ctl->done = 1;
+            publish(a.status, ctl, a.it, RUN_DONE);
+        }
         return;
     }
     if (lead) {
+        publish(a.status, ctl, a.it, RUN_GOING);
         ctl->qpack[(a.it + 1) % 3] = 0;
         ctl->iters = a.it;
     }
@@ -907,23 +890,25 @@ __global__ __launch_bounds__(WG, K <= 8 ? 3 : 1) void k_plane_push(PlaneArgs arg
     }
 }
 
-// Vertices of the frontier just pushed forget their change masks; vertices improved this
-// iteration take theirs from nchg.  Runs over the previous frontier, then the new one.
-// With dev_it (replayed graph) the queue, slot and activity slot come from the device iteration:
-// move = 0 takes the frontier the push read, move = 1 the one it wrote.
+// Between the iterations of a batched pass, whose two mask arrays take turns: the vertices just
+// pushed (queue q, its size in Ctl slot) forget the changes they pushed, so that the array is clear
+// for the iteration after the next; dense passes build the next queue from the marks beside it.
+__global__ __launch_bounds__(COMPACT_WG) void k_plane_between(CompactArgs c, int compact, const uint32_t* __restrict__ q,
+                                                              int slot, uint64_t* __restrict__ chg, uint32_t W) {
+    if (c.ctl->done) return;
+    if (compact) compact_frontier(c);
+    const uint64_t words = (c.ctl->qpack[slot] & 0xffffffffull) * W;
+    for (uint64_t i = (uint64_t)blockIdx.x * COMPACT_WG + threadIdx.x; i < words; i += (uint64_t)gridDim.x * COMPACT_WG)
+        chg[(uint64_t)q[i / W] * W + i % W] = 0;
+}
+
+// The serving engines' form: vertices of the frontier just pushed forget their change masks (move =
+// 0), then vertices improved this iteration take theirs from nchg (move = 1).
 __global__ void k_plane_rotate(const uint32_t* q, const Ctl* ctl, int slot,
                                uint64_t* __restrict__ from, uint64_t* __restrict__ to, uint32_t W,
-                               int move, uint64_t* act, const uint32_t* dev_it, const uint32_t* qa,
-                               const uint32_t* qb, uint64_t* act_base) {
+                               int move, uint64_t* act) {
     __shared__ unsigned long long sAct[MAXW];
     if (ctl->done) return;
-    if (dev_it) {
-        const uint32_t it = dev_it[0];
-        const bool odd = ((it - 1) & 1) != 0;
-        q = move ? (odd ? qa : qb) : (odd ? qb : qa);
-        slot = move ? (int)(it % 3) : (int)((it - 1) % 3);
-        act = (move && act_base) ? act_base + (it % 4) * MAXW : nullptr;
-    }
     if (threadIdx.x < MAXW) sAct[threadIdx.x] = 0;
     __syncthreads();
     const uint32_t count = (uint32_t)(ctl->qpack[slot] & 0xffffffffull);
@@ -999,66 +984,70 @@ __global__ void k_max_u32(const uint32_t* __restrict__ a, uint64_t n, uint32_t* 
     if (lane_id() == 0 && m) atomicMax(out, m);
 }
 
-// Fills with 16-byte stores where the base allows (the planes are many GB).
-__global__ void k_fill_u32b(uint32_t* __restrict__ a, uint64_t n, uint32_t v) {
+// What a pass starts from, in one launch: up to N arrays filled, with 16-byte stores (the planes
+// are many GB; the arrays are allocations of their own, so their bases allow it), and the control
+// block cleared.
+struct StartArgs {
+    static constexpr int N = 5;
+    uint32_t* p[N];
+    uint64_t words[N];
+    uint32_t val[N];
+    Ctl* ctl;
+};
+__global__ void k_batch_start(StartArgs a) {
     const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, nt = (uint64_t)gridDim.x * blockDim.x;
-    uint64_t head = 0;
-    if (((uintptr_t)a & 15) == 0) {
-        const uint64_t n4 = n / 4;
-        uint4* a4 = reinterpret_cast<uint4*>(a);
-        for (uint64_t i = tid; i < n4; i += nt) a4[i] = make_uint4(v, v, v, v);
-        head = n4 * 4;
+#pragma unroll
+    for (int k = 0; k < StartArgs::N; ++k) {
+        if (!a.p[k]) continue;
+        const uint64_t n4 = a.words[k] / 4;
+        const uint32_t v = a.val[k];
+        uint4* p4 = reinterpret_cast<uint4*>(a.p[k]);
+        for (uint64_t i = tid; i < n4; i += nt) p4[i] = make_uint4(v, v, v, v);
+        if (tid < a.words[k] % 4) a.p[k][n4 * 4 + tid] = v;
     }
-    for (uint64_t i = head + tid; i < n; i += nt) a[i] = v;
-}
-__global__ void k_fill_u64(uint64_t* __restrict__ a, uint64_t n) {
-    const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, nt = (uint64_t)gridDim.x * blockDim.x;
-    uint64_t head = 0;
-    if (((uintptr_t)a & 15) == 0) {
-        const uint64_t n2 = n / 2;
-        ulonglong2* a2 = reinterpret_cast<ulonglong2*>(a);
-        for (uint64_t i = tid; i < n2; i += nt) a2[i] = ulonglong2{0, 0};
-        head = n2 * 2;
+    if (tid == 0) {
+        a.ctl->done = 0;
+        a.ctl->iters = 0;
+        a.ctl->err = 0;
+        for (int k = 0; k < 3; ++k) a.ctl->qpack[k] = 0;
     }
-    for (uint64_t i = head + tid; i < n; i += nt) a[i] = 0;
-}
-// dst[i] = src[idx[i]]
-__global__ void k_gather_u32(const uint32_t* __restrict__ src, const uint32_t* __restrict__ idx, uint32_t m,
-                             uint32_t* __restrict__ dst) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += gridDim.x * blockDim.x) dst[i] = src[idx[i]];
 }
 
-// Seeds: entries (vertex, query) applied on the device; the first frontier is the distinct
-// source vertices with their virtual-node prefix, computed on the host.
-__global__ void k_seed(const uint32_t* __restrict__ sv, const uint32_t* __restrict__ sq, uint32_t ns,
-                       uint64_t* __restrict__ m1, uint64_t* __restrict__ m2, uint32_t* __restrict__ lab,
-                       uint32_t R, uint32_t B, uint32_t val, int lm) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < ns; i += gridDim.x * blockDim.x) {
-        const uint64_t idx = (uint64_t)sv[i] * R + sq[i] / 64;
-        const uint64_t bit = 1ull << (sq[i] % 64);
+// Seeds of a pass, one workgroup: query i starts at the internal vertex seeds[i], its bit goes to m1
+// (and m2); the first frontier is the nf distinct sources seeds[ns ..] that have out-edges, in their
+// order.  The seeds are read from pinned host memory.
+__global__ __launch_bounds__(WG) void k_batch_seed(const uint32_t* __restrict__ seeds, uint32_t ns, uint32_t nf,
+                                                   uint64_t* __restrict__ m1, uint64_t* __restrict__ m2,
+                                                   uint32_t* __restrict__ lab, uint32_t R, uint32_t B, uint32_t val,
+                                                   int lm, const uint32_t* __restrict__ vnc, uint32_t* __restrict__ q,
+                                                   uint32_t* __restrict__ s, Ctl* ctl) {
+    __shared__ uint64_t sScan[WG / WAVE + 1];
+    const uint32_t i = threadIdx.x;  // ns and nf are at most 64 * MAXW = WG
+    if (i < ns) {
+        const uint32_t v = seeds[i];
+        const uint64_t idx = (uint64_t)v * R + i / 64, bit = 1ull << (i % 64);
         atomicOr((unsigned long long*)&m1[idx], (unsigned long long)bit);
         if (m2) atomicOr((unsigned long long*)&m2[idx], (unsigned long long)bit);
-        const uint64_t j = (uint64_t)sv[i] * B + sq[i];
+        const uint64_t j = (uint64_t)v * B + i;
         if (lm == LM_W8 || lm == LM_D8) reinterpret_cast<uint8_t*>(lab)[j] = (uint8_t)(val == INF ? 0xffu : val);
         else if (lm == LM_D16) reinterpret_cast<uint16_t*>(lab)[j] = (uint16_t)(val == INF ? 0xffffu : val);
         else lab[j] = val;
     }
-}
-
-__global__ void k_set_frontier(const uint32_t* __restrict__ fv, const uint32_t* __restrict__ fs, uint32_t nf,
-                               uint64_t packed, uint32_t* __restrict__ q, uint32_t* __restrict__ s, Ctl* ctl) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nf; i += gridDim.x * blockDim.x) {
-        q[i] = fv[i];
-        s[i] = fs[i];
+    uint32_t v = 0, nv = 0;
+    if (i < nf) {
+        v = seeds[ns + i];
+        nv = vnc[v];
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        for (int k = 0; k < 3; ++k) ctl->qpack[k] = 0;
-        ctl->qpack[0] = packed;
-        ctl->done = 0;
-        ctl->iters = 0;
-        ctl->err = 0;
+    uint64_t tot;
+    const uint64_t pre = block_excl_scan<uint64_t>(nv ? ((uint64_t)nv << 32) | 1ull : 0ull, sScan, &tot);
+    if (nv) {
+        const uint32_t at = (uint32_t)(pre & 0xffffffffull);
+        q[at] = v;
+        s[at] = (uint32_t)(pre >> 32);
     }
+    if (i == 0) ctl->qpack[0] = tot;
 }
+static_assert(64 * MAXW <= WG, "a thread per seed");
 
 // Admission of new queries between iterations (one workgroup); see launch_admit.
 __global__ __launch_bounds__(WG) void k_admit(Ctl* ctl, int in_slot, const uint32_t* __restrict__ pv,
@@ -1157,20 +1146,23 @@ struct BatchWork {
     DevMem ovq;             // 8-bit SSSP passes: queries whose distances outgrew 8 bits
     DevMem rowbuf;          // small answers on their way to the host (below HOST_COPY_FROM)
     bool d8_off = false;    // a previous 8-bit SSSP pass flagged more than a quarter of its queries
-    DevMem q[2], s[2], cand, stamp, seeds, ctl;
-    DevMem devit;           // replayed chunks: {iteration, stamp base}
+    DevMem q[2], s[2], cand, stamp, ctl;
     uint32_t epoch = 1;
-    hipGraphExec_t exec = nullptr;  // graph of one chunk and the arguments it was built with
-    std::vector<uint8_t> key;
+    // pinned: progress of the running pass, and its seeds (nothing reads or writes them once a pass has
+    // ended)
+    struct Host {
+        RunStatus status;
+        uint32_t seeds[2 * 64 * BATCH_MAXW];
+    }* host = nullptr;
     ~BatchWork() {
-        if (exec) (void)hipGraphExecDestroy(exec);
+        if (host) (void)hipHostFree(host);
     }
 };
 
 namespace {
 
-// Iterations per replayed chunk (a multiple of 2 and 3: queue ping-pong and control slots).
-constexpr uint32_t BATCH_CHUNK = 6;
+// Limits of iterations are rounded up to this many (as passes of whole chunks ran once).
+constexpr uint64_t BATCH_CHUNK = 6;
 
 // Compaction of a dense plane pass's marks into the queue the push would have written.
 CompactArgs compact_args(const PlaneArgs& a) {
@@ -1185,25 +1177,6 @@ CompactArgs compact_args(const PlaneArgs& a) {
 }
 unsigned compact_grid(uint32_t n) {
     return std::max(1u, std::min(mark_chunks(n), 1024u));
-}
-
-__global__ void k_tick_b(uint32_t* it) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *it += 1;
-}
-
-eeg_status add_node(hipGraph_t graph, hipGraphNode_t* prev, const void* fn, unsigned grid, unsigned block,
-                    void** args) {
-    hipKernelNodeParams kp{};
-    kp.func = const_cast<void*>(fn);
-    kp.gridDim = dim3(grid);
-    kp.blockDim = dim3(block);
-    kp.sharedMemBytes = 0;
-    kp.kernelParams = args;
-    kp.extra = nullptr;
-    hipGraphNode_t node = nullptr;
-    EEG_HIP(hipGraphAddKernelNode(&node, graph, *prev ? prev : nullptr, *prev ? 1 : 0, &kp));
-    *prev = node;
-    return EEG_OK;
 }
 
 // Dense plane push for K, label width lm and W mask words (rows of 16 W or 32 W narrow lane
@@ -1226,93 +1199,15 @@ const void* dense_push(uint32_t K, int lm, uint32_t W) {
     }
 }
 
-// Graph of BATCH_CHUNK iterations (BFS: push, finalize; planes: push, two rotations; each
-// followed by a counter tick), built node by node and kept until its arguments change.
-eeg_status batch_graph(BatchWork& bw, bool bfs, uint32_t K, unsigned grid, const MsArgs& ma, const PlaneArgs& pa,
-                       uint32_t nsrc, int lm, hipGraphExec_t* out) {
-    const bool dense = nsrc > PLANE_DENSE_FROM;
-    std::vector<uint8_t> key(sizeof(MsArgs) + sizeof(PlaneArgs) + 20);
-    memcpy(key.data(), &ma, sizeof(MsArgs));
-    memcpy(key.data() + sizeof(MsArgs), &pa, sizeof(PlaneArgs));
-    const uint32_t tail[5] = {bfs ? 1u : 0u, K, grid, dense ? 1u : 0u, (uint32_t)lm};
-    memcpy(key.data() + sizeof(MsArgs) + sizeof(PlaneArgs), tail, 20);
-    if (bw.exec && bw.key == key) {
-        *out = bw.exec;
-        return EEG_OK;
+// Push kernel of a plane pass with `queries` in flight.
+const void* plane_push(uint32_t K, uint32_t queries, int lm, uint32_t W) {
+    if (queries > PLANE_DENSE_FROM) return dense_push(K, lm, W);
+    switch (K) {
+        case 4: return (const void*)k_plane_push<4>;
+        case 8: return (const void*)k_plane_push<8>;
+        case 16: return (const void*)k_plane_push<16>;
+        default: return (const void*)k_plane_push<32>;
     }
-    if (bw.exec) {
-        (void)hipGraphExecDestroy(bw.exec);
-        bw.exec = nullptr;
-    }
-    hipGraph_t graph = nullptr;
-    EEG_HIP(hipGraphCreate(&graph, 0));
-    MsArgs m = ma;
-    PlaneArgs p = pa;
-    uint32_t* itp = const_cast<uint32_t*>(bfs ? ma.dev_it : pa.dev_it);
-    void* margs[] = {&m};
-    void* pargs[] = {&p};
-    void* targs[] = {&itp};
-    // rotation arguments (queue, slot and activity slot resolved on the device)
-    const uint32_t* rq = nullptr;
-    const Ctl* rctl = pa.ctl;
-    int rslot = 0;
-    uint64_t* rnone = nullptr;
-    uint64_t* rfrom1 = pa.nchg;
-    uint64_t* rto = pa.chg;
-    uint32_t rW = pa.W;
-    int move0 = 0, move1 = 1;
-    uint64_t* ract = nullptr;
-    const uint32_t* rit = pa.dev_it;
-    const uint32_t* rqa = pa.qa;
-    const uint32_t* rqb = pa.qb;
-    uint64_t* ractb = pa.act;
-    void* r0args[] = {&rq, &rctl, &rslot, &rnone, &rto, &rW, &move0, &ract, &rit, &rqa, &rqb, &ractb};
-    // sorted queues: the iteration comes from the device counter (ticked after each iteration)
-    CompactArgs cga{};
-    if (pa.mark) {
-        cga = compact_args(pa);
-        cga.qa = pa.qa;
-        cga.sa = pa.sa;
-        cga.qb = pa.qb;
-        cga.sb = pa.sb;
-        cga.dev_it = pa.dev_it;
-    }
-    void* cargs[] = {&cga};
-    void* r1args[] = {&rq, &rctl, &rslot, &rfrom1, &rto, &rW, &move1, &ract, &rit, &rqa, &rqb, &ractb};
-    const void* fpush =
-        bfs ? ((K == 4) ? (const void*)k_ms_push<4> : (K == 8) ? (const void*)k_ms_push<8>
-               : (K == 16) ? (const void*)k_ms_push<16> : (const void*)k_ms_push<32>)
-        : dense ? dense_push(K, lm, pa.W)
-                : ((K == 4) ? (const void*)k_plane_push<4> : (K == 8) ? (const void*)k_plane_push<8>
-                   : (K == 16) ? (const void*)k_plane_push<16> : (const void*)k_plane_push<32>);
-    hipGraphNode_t prev = nullptr;
-    eeg_status rc = EEG_OK;
-    for (uint32_t i = 0; i < BATCH_CHUNK && rc == EEG_OK; ++i) {
-        if (bfs) {
-            rc = add_node(graph, &prev, fpush, grid, WG, margs);
-            if (rc == EEG_OK) rc = add_node(graph, &prev, (const void*)k_ms_finalize, grid, WG, margs);
-        } else {
-            rc = add_node(graph, &prev, fpush, grid, WG, pargs);
-            if (rc == EEG_OK && pa.mark)
-                rc = add_node(graph, &prev, (const void*)k_compact_frontier, compact_grid(pa.n), COMPACT_WG, cargs);
-            if (rc == EEG_OK) rc = add_node(graph, &prev, (const void*)k_plane_rotate, 2048, WG, r0args);
-            if (rc == EEG_OK) rc = add_node(graph, &prev, (const void*)k_plane_rotate, 2048, WG, r1args);
-        }
-        if (rc == EEG_OK) rc = add_node(graph, &prev, (const void*)k_tick_b, 1, 64, targs);
-    }
-    if (rc != EEG_OK) {
-        (void)hipGraphDestroy(graph);
-        return rc;
-    }
-    const hipError_t e = hipGraphInstantiate(&bw.exec, graph, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(graph);
-    if (e != hipSuccess) {
-        bw.exec = nullptr;
-        return fail(EEG_ERR_DEVICE, "hipGraphInstantiate failed: %s", hipGetErrorString(e));
-    }
-    bw.key = key;
-    *out = bw.exec;
-    return EEG_OK;
 }
 
 }  // namespace
@@ -1400,82 +1295,56 @@ eeg_status batch_pass(eeg_graph* g, BatchWork& bw, hipStream_t s, uint32_t algo,
         bw.epoch = 1;
     }
     EEG_TRY(bw.ctl.alloc(sizeof(Ctl)));
-    EEG_TRY(bw.seeds.alloc((size_t)4 * nsrc * 4 + 16));
-    if (lm == LM_D8) {
-        EEG_TRY(bw.ovq.alloc(MAXW * 8));
-        k_fill_u64<<<1, 64, 0, s>>>(bw.ovq.as<uint64_t>(), MAXW);
-        EEG_HIP(hipGetLastError());
-    }
+    if (!bw.host)
+        EEG_HIP(hipHostMalloc((void**)&bw.host, sizeof(*bw.host), hipHostMallocMapped | hipHostMallocCoherent));
+    if (lm == LM_D8) EEG_TRY(bw.ovq.alloc(MAXW * 8));
+    const bool marks = !bfs && nsrc > PLANE_DENSE_FROM;  // dense passes: sorted queues rebuilt from marks
+    if (marks) EEG_TRY(bw.mark.alloc(mark_bytes(n)));
     Ctl* ctl = bw.ctl.as<Ctl>();
-    EEG_HIP(hipMemsetAsync(ctl, 0, sizeof(Ctl), s));
 
-    // seeds in internal ids; first frontier = distinct sources with out-edges
-    std::vector<uint32_t> sv(nsrc), sq(nsrc);
-    for (uint32_t i = 0; i < nsrc; ++i) {
-        sv[i] = g->h_perm[sources[i]];
-        sq[i] = i;
-    }
-    std::vector<uint32_t> fv(sv);
-    std::sort(fv.begin(), fv.end());
-    fv.erase(std::unique(fv.begin(), fv.end()), fv.end());
-    uint32_t* dseed = bw.seeds.as<uint32_t>();
-    // virtual-node counts of the distinct sources, gathered into the seed buffer's frontier
-    // half (overwritten below) and read back in one copy
-    std::vector<uint32_t> hvnc(fv.size());
-    EEG_HIP(hipMemcpyAsync(dseed + 2 * nsrc, fv.data(), fv.size() * 4, hipMemcpyHostToDevice, s));
-    k_gather_u32<<<grid_n(fv.size()), WG, 0, s>>>(t.vnc.as<uint32_t>(), dseed + 2 * nsrc, (uint32_t)fv.size(),
-                                                 dseed + 3 * nsrc);
-    EEG_HIP(hipGetLastError());
-    EEG_HIP(hipMemcpyAsync(hvnc.data(), dseed + 3 * nsrc, fv.size() * 4, hipMemcpyDeviceToHost, s));
-    EEG_HIP(hipStreamSynchronize(s));
-    std::vector<uint32_t> fvv, fss;
-    uint32_t acc = 0;
-    for (size_t i = 0; i < fv.size(); ++i)
-        if (hvnc[i]) {
-            fvv.push_back(fv[i]);
-            fss.push_back(acc);
-            acc += hvnc[i];
-        }
-    EEG_HIP(hipMemcpyAsync(dseed, sv.data(), nsrc * 4, hipMemcpyHostToDevice, s));
-    EEG_HIP(hipMemcpyAsync(dseed + nsrc, sq.data(), nsrc * 4, hipMemcpyHostToDevice, s));
-    if (!fvv.empty()) {
-        EEG_HIP(hipMemcpyAsync(dseed + 2 * nsrc, fvv.data(), fvv.size() * 4, hipMemcpyHostToDevice, s));
-        EEG_HIP(hipMemcpyAsync(dseed + 3 * nsrc, fss.data(), fss.size() * 4, hipMemcpyHostToDevice, s));
-    }
+    // seeds in internal ids, then the distinct ones
+    uint32_t* seeds = bw.host->seeds;
+    for (uint32_t i = 0; i < nsrc; ++i) seeds[i] = seeds[nsrc + i] = g->h_perm[sources[i]];
+    std::sort(seeds + nsrc, seeds + 2 * nsrc);
+    const uint32_t nf = (uint32_t)(std::unique(seeds + nsrc, seeds + 2 * nsrc) - (seeds + nsrc));
     uint64_t* rec = bw.m1.as<uint64_t>();
-    k_fill_u64<<<grid_n(nrec), WG, 0, s>>>(rec, nrec);
-    if (!bfs) k_fill_u64<<<grid_n(nw), WG, 0, s>>>(bw.m3.as<uint64_t>(), nw);
     // every label unreached: 0 (widest), INF or all ones (narrow INF) for distances; nb is a
     // multiple of 64, so the narrow planes are whole 32-bit words
     const uint32_t unreached = widest ? 0u : (lm == LM_U32 ? INF : 0xffffffffu);
-    k_fill_u32b<<<grid_n(nb * lbytes / 4), WG, 0, s>>>(bw.planes.as<uint32_t>(), nb * lbytes / 4, unreached);
-    EEG_HIP(hipGetLastError());
+    StartArgs sa{};
+    sa.ctl = ctl;
+    int na = 0;
+    auto fill = [&](void* p, uint64_t bytes, uint32_t val) {
+        sa.p[na] = static_cast<uint32_t*>(p);
+        sa.words[na] = bytes / 4;
+        sa.val[na++] = val;
+    };
+    fill(bw.planes.p, nb * lbytes, unreached);
+    fill(rec, nrec * 8, 0u);
+    if (!bfs) fill(bw.m3.p, nw * 8, 0u);
+    if (marks) fill(bw.mark.p, mark_bytes(n), 0u);
+    if (lm == LM_D8) fill(bw.ovq.p, MAXW * 8, 0u);
+    k_batch_start<<<grid_n(nb * lbytes / 16), WG, 0, s>>>(sa);
     // BFS: seen and visit get the source bits, level 0.  Planes: chg gets them.
-    k_seed<<<grid_n(nsrc), WG, 0, s>>>(dseed, dseed + nsrc, nsrc, rec, bfs ? rec + 2 * W : nullptr,
-                                       bw.planes.as<uint32_t>(), R, B, widest ? INF : 0u, lm);
-    k_set_frontier<<<grid_n(fvv.size() ? fvv.size() : 1), WG, 0, s>>>(
-        dseed + 2 * nsrc, dseed + 3 * nsrc, (uint32_t)fvv.size(),
-        ((unsigned long long)acc << 32) | (unsigned long long)fvv.size(), bw.q[0].as<uint32_t>(),
-        bw.s[0].as<uint32_t>(), ctl);
+    k_batch_seed<<<1, WG, 0, s>>>(seeds, nsrc, nf, rec, bfs ? rec + 2 * W : nullptr, bw.planes.as<uint32_t>(), R, B,
+                                  widest ? INF : 0u, lm, t.vnc.as<uint32_t>(), bw.q[0].as<uint32_t>(),
+                                  bw.s[0].as<uint32_t>(), ctl);
     EEG_HIP(hipGetLastError());
 
     const int cus = cu_count_b(g->device);
     // 48: 4-5% faster 32-bit planes than 24; narrow planes (8 waves per SIMD) 3-4% faster at 96
     // than at 48 (RMAT-24 x 256)
-    const unsigned grid = (unsigned)cus * (o.wgs_per_cu ? o.wgs_per_cu : (lm == LM_U32 ? 48 : 96));
+    // (no more than a small graph has tiles; the dense push cuts them down to four virtual nodes)
+    const uint64_t tiles = bfs ? std::max<uint64_t>((t.P * K + TILE_EDGES - 1) / TILE_EDGES, ((uint64_t)n + WG - 1) / WG)
+                           : nsrc > PLANE_DENSE_FROM ? (t.P + WG / WAVE - 1) / (WG / WAVE)
+                                                     : (t.P * K + TILE_EDGES - 1) / TILE_EDGES;
+    const unsigned grid = (unsigned)std::max<uint64_t>(
+        1, std::min<uint64_t>(tiles, (uint64_t)cus * (o.wgs_per_cu ? o.wgs_per_cu : (lm == LM_U32 ? 48 : 96))));
     const uint32_t base = bw.epoch;
-    hipEvent_t e0, e1;
-    EEG_HIP(hipEventCreate(&e0));
-    EEG_HIP(hipEventCreate(&e1));
-    EEG_HIP(hipEventRecord(e0, s));
     Ctl hc{};
-    uint32_t launches = 0, level = 0;
     const uint32_t max_iters = o.max_iters ? o.max_iters : n + 2;
-    // BFS: one level = push + finalize; planes: one iteration = push + two mask rotations.
-    // Chunks of 8 run ahead of the host's look at the control block.
     const uint32_t qcap = n + 1;
-    // argument blocks shared by every iteration; the per-iteration fields are set per launch,
-    // or derived on the device when a graph of BATCH_CHUNK iterations is replayed
+    // argument blocks shared by every iteration; the per-iteration fields are set per launch
     MsArgs ma{};
     PlaneArgs pa{};
     if (bfs) {
@@ -1511,75 +1380,67 @@ eeg_status batch_pass(eeg_graph* g, BatchWork& bw, hipStream_t s, uint32_t algo,
         pa.qcap = qcap;
         pa.widest = widest ? 1 : 0;
         pa.ovq = lm == LM_D8 ? bw.ovq.as<uint64_t>() : nullptr;
-        if (nsrc > PLANE_DENSE_FROM) {  // dense passes: sorted queues rebuilt from marks
-            EEG_TRY(bw.mark.alloc(mark_bytes(n)));
-            k_fill_u32b<<<grid_n(mark_bytes(n) / 4), WG, 0, s>>>(bw.mark.as<uint32_t>(), mark_bytes(n) / 4, 0u);
-            EEG_HIP(hipGetLastError());
+        if (marks) {
             pa.mark = bw.mark.as<uint8_t>();
             pa.cmark = chunk_marks(bw.mark.p, n);
         }
     }
-    const bool replay = !o.timing;
-    hipGraphExec_t exec = nullptr;
-    if (replay) {
-        EEG_TRY(bw.devit.alloc(8));
-        uint32_t* dit = bw.devit.as<uint32_t>();
-        k_fill_u32b<<<1, 64, 0, s>>>(dit, 1, 1u);
-        k_fill_u32b<<<1, 64, 0, s>>>(dit + 1, 1, base);
+    ma.status = pa.status = &bw.host->status;
+    const void* push = bfs ? nullptr : plane_push(K, nsrc, lm, W);
+    const unsigned grid_between =
+        std::max(marks ? compact_grid(n) : 1u, (unsigned)std::min<uint64_t>(512, (nw + COMPACT_WG - 1) / COMPACT_WG));
+    // A level of BFS is a push and a finalize; an iteration of planes a push and what comes between it
+    // and the next.  (Replayed graphs of six iterations, with their counter and the two rotations of
+    // the masks, took three and four or five launches, ran up to six iterations past the end and were
+    // built anew for new arguments.)
+    auto launch = [&](uint32_t j) -> eeg_status {
+        const int cur = (int)((j - 1) & 1);
+        uint32_t *qin = bw.q[cur].as<uint32_t>(), *sin = bw.s[cur].as<uint32_t>();
+        uint32_t *qout = bw.q[cur ^ 1].as<uint32_t>(), *sout = bw.s[cur ^ 1].as<uint32_t>();
+        if (bfs) {
+            ma.level = j;
+            ma.stampv = base + j;
+            ma.qin = qin;
+            ma.sin = sin;
+            ma.qout = qout;
+            ma.sout = sout;
+            return launch_ms_level(ma, K, grid, s);
+        }
+        pa.it = j;
+        pa.stampv = base + j;
+        pa.qin = qin;
+        pa.sin = sin;
+        pa.qout = qout;
+        pa.sout = sout;
+        void* args[] = {&pa};
+        EEG_HIP(hipLaunchKernel(push, dim3(grid), dim3(WG), args, 0, s));
+        CompactArgs ca = compact_args(pa);
+        ca.qa = ca.qb = qout;
+        ca.sa = ca.sb = sout;
+        ca.it = j;
+        k_plane_between<<<grid_between, COMPACT_WG, 0, s>>>(ca, marks ? 1 : 0, qin, (int)((j - 1) % 3), pa.chg, W);
         EEG_HIP(hipGetLastError());
-        ma.dev_it = pa.dev_it = dit;
-        ma.qa = pa.qa = bw.q[0].as<uint32_t>();
-        ma.sa = pa.sa = bw.s[0].as<uint32_t>();
-        ma.qb = pa.qb = bw.q[1].as<uint32_t>();
-        ma.sb = pa.sb = bw.s[1].as<uint32_t>();
-        EEG_TRY(batch_graph(bw, bfs, K, grid, ma, pa, nsrc, lm, &exec));
-    }
-    uint32_t j = 1;
-    while (true) {
-        if (replay) {
-            EEG_HIP(hipGraphLaunch(exec, s));
-            j += BATCH_CHUNK;
-            launches += BATCH_CHUNK;
-        }
-        const uint32_t chunk = replay ? 0 : 8;
-        for (uint32_t c = 0; c < chunk; ++c, ++j, ++launches) {
-            const int cur = (int)((j - 1) & 1);
-            if (bfs) {
-                MsArgs a = ma;
-                a.level = j;
-                a.stampv = base + j;
-                a.qin = bw.q[cur].as<uint32_t>();
-                a.sin = bw.s[cur].as<uint32_t>();
-                a.qout = bw.q[cur ^ 1].as<uint32_t>();
-                a.sout = bw.s[cur ^ 1].as<uint32_t>();
-                EEG_TRY(launch_ms_level(a, K, grid, s));
-            } else {
-                PlaneArgs a = pa;
-                a.it = j;
-                a.stampv = base + j;
-                a.qin = bw.q[cur].as<uint32_t>();
-                a.sin = bw.s[cur].as<uint32_t>();
-                a.qout = bw.q[cur ^ 1].as<uint32_t>();
-                a.sout = bw.s[cur ^ 1].as<uint32_t>();
-                EEG_TRY(launch_plane_iteration(a, K, grid, s, nsrc, lm));
-            }
-        }
-        EEG_HIP(hipMemcpyAsync(&hc, ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s));
+        std::swap(pa.chg, pa.nchg);
+        return EEG_OK;
+    };
+    reset_status(&bw.host->status);
+    uint32_t j = 1, state = RUN_GOING;
+    const uint64_t limit = ((uint64_t)max_iters + 16 + BATCH_CHUNK - 1) / BATCH_CHUNK * BATCH_CHUNK;
+    const eeg_status ran = run_ahead(s, &bw.host->status, limit, &j, &state, launch);
+    bw.epoch = base + j + 2;
+    if (ran != EEG_OK) return ran;
+    if (state == RUN_DONE) {
+        hc.iters = (uint32_t)(bw.host->status.word >> 8) - 1;
+    } else {
         EEG_HIP(hipStreamSynchronize(s));
+        EEG_HIP(hipMemcpy(&hc, ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
         if (hc.err == PLANE_ERR_NARROW && lm != LM_U32) {  // distances outgrew the labels
-            bw.epoch = base + j + 2;
-            (void)hipEventDestroy(e0);
-            (void)hipEventDestroy(e1);
             *overflow = true;
             return EEG_OK;
         }
         if (hc.err) return fail(EEG_ERR_DEVICE, "batched frontier overflow (err=%u)", hc.err);
-        if (hc.done) break;
-        level = hc.iters;
-        if (j > max_iters + 16) return fail(EEG_ERR_NOT_CONVERGED, "batched traversal did not converge");
+        if (!hc.done) return fail(EEG_ERR_NOT_CONVERGED, "batched traversal did not converge");
     }
-    EEG_HIP(hipEventRecord(e1, s));
-    bw.epoch = base + j + 2;
     if (ovq_out) {
         for (uint32_t i = 0; i < MAXW; ++i) ovq_out[i] = 0;
         if (lm == LM_D8) EEG_HIP(hipMemcpyAsync(ovq_out, bw.ovq.p, MAXW * 8, hipMemcpyDeviceToHost, s));
@@ -1637,15 +1498,10 @@ eeg_status batch_pass(eeg_graph* g, BatchWork& bw, hipStream_t s, uint32_t algo,
         }
     }
     EEG_HIP(hipStreamSynchronize(s));
-    float ms = 0;
-    EEG_HIP(hipEventElapsedTime(&ms, e0, e1));
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    (void)level;
     if (st) {
         st->iterations = hc.iters;
-        st->launches = launches;
-        st->ms_traversal = ms;
+        st->launches = j - 1;
+        st->ms_traversal = run_ms(&bw.host->status, g->device);
         st->ms_total = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_host0).count();
         st->label_bits = bfs ? 0u : (uint32_t)(8 * lbytes);
     }
@@ -1798,26 +1654,13 @@ eeg_status launch_ms_level(MsArgs a, uint32_t K, unsigned grid, hipStream_t s) {
     return EEG_OK;
 }
 
-eeg_status launch_plane_iteration(PlaneArgs a, uint32_t K, unsigned grid, hipStream_t s, uint32_t in_flight, int lm) {
+eeg_status launch_plane_iteration(PlaneArgs a, uint32_t K, unsigned grid, hipStream_t s, uint32_t in_flight) {
     void* args[] = {&a};
-    const void* fn = (K == 4) ? (const void*)k_plane_push<4> : (K == 8) ? (const void*)k_plane_push<8>
-                     : (K == 16) ? (const void*)k_plane_push<16> : (const void*)k_plane_push<32>;
-    if (in_flight > PLANE_DENSE_FROM) fn = dense_push(K, lm, a.W);
-    EEG_HIP(hipLaunchKernel(fn, dim3(grid), dim3(WG), args, 0, s));
-    if (a.mark) {  // sorted queue: the push only marked vertices
-        CompactArgs ca = compact_args(a);
-        ca.qa = ca.qb = a.qout;
-        ca.sa = ca.sb = a.sout;
-        ca.it = a.it;
-        void* cargs[] = {&ca};
-        EEG_HIP(hipLaunchKernel((const void*)k_compact_frontier, dim3(compact_grid(a.n)), dim3(COMPACT_WG), cargs, 0, s));
-    }
+    EEG_HIP(hipLaunchKernel(plane_push(K, in_flight, LM_U32, a.W), dim3(grid), dim3(WG), args, 0, s));
     // forget the pushed frontier's masks, then move this iteration's improvements in
-    k_plane_rotate<<<2048, WG, 0, s>>>(a.qin, a.ctl, (int)((a.it - 1) % 3), nullptr, a.chg, a.W, 0, nullptr,
-                                        nullptr, nullptr, nullptr, nullptr);
+    k_plane_rotate<<<2048, WG, 0, s>>>(a.qin, a.ctl, (int)((a.it - 1) % 3), nullptr, a.chg, a.W, 0, nullptr);
     k_plane_rotate<<<2048, WG, 0, s>>>(a.qout, a.ctl, (int)(a.it % 3), a.nchg, a.chg, a.W, 1,
-                                        a.act ? a.act + (a.it % 4) * MAXW : nullptr, nullptr, nullptr, nullptr,
-                                        nullptr);
+                                       a.act ? a.act + (a.it % 4) * MAXW : nullptr);
     EEG_HIP(hipGetLastError());
     return EEG_OK;
 }

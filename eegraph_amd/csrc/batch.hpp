@@ -10,8 +10,7 @@ namespace eeg {
 
 constexpr uint32_t BATCH_MAXW = 4;  // up to 256 queries per traversal (4 x 64-bit words)
 
-// State of multi-source passes (label planes, masks, queues, the replayed graph of a chunk);
-// one per graph handle for eeg_run_batch, one per serving lane that batches its queries.
+// State of multi-source passes (label planes, masks, queues); one per graph handle for eeg_run_batch, one per serving lane that batches its queries.
 struct BatchWork;
 std::shared_ptr<BatchWork> make_batch_work();
 // BFS/SSSP/SSWP from up to 256 sources in one pass (narrow labels as eeg_run_batch chooses
@@ -52,10 +51,7 @@ struct MsArgs {
     uint32_t launch;       // launch index (slot rotation)
     uint32_t level;        // level being discovered by this push (1-based)
     uint32_t stampv;
-    // replayed graph: level = dev_it[0], stamp base = dev_it[1]; launch, stampv and the queue
-    // ping-pong over (qa, sa) / (qb, sb) are derived from them
-    const uint32_t* dev_it;
-    uint32_t *qa, *sa, *qb, *sb;
+    RunStatus* status;     // pinned: progress for the host (null: none)
 };
 
 // Batched SSSP / SSWP over vertex-major label planes.
@@ -80,10 +76,9 @@ struct PlaneArgs {
     uint32_t it;
     uint32_t stampv;
     int widest;           // 0: SSSP (min, +w), 1: SSWP (max, min(.,w))
-    const uint32_t* dev_it;  // replayed graph, as in MsArgs
-    uint32_t *qa, *sa, *qb, *sb;
+    RunStatus* status;    // pinned: progress for the host (null: none)
     uint8_t* mark;        // dense passes of eeg_run_batch: improved vertices are marked and
-    uint8_t* cmark;       // k_compact_frontier builds the next queue in vertex order (null: the
+    uint8_t* cmark;       // compact_frontier builds the next queue in vertex order (null: the
                           // push appends to the queue itself)
     uint64_t* ovq;        // 8-bit distance passes: W words, queries to answer again wider
 };
@@ -92,11 +87,9 @@ struct PlaneArgs {
 eeg_status launch_ms_level(MsArgs a, uint32_t K, unsigned grid, hipStream_t s);
 // One plane iteration: push, then the two change-mask rotations.  `in_flight` (queries being
 // traversed) picks the push variant: one wavefront per virtual node with lane = query for
-// many, a two-pass kernel with K lanes per virtual node for few.
-// `lm` is the label width of the dense push (0: 32-bit labels, lane = query; narrow widths
-// only with the planes of eeg_run_batch).
-eeg_status launch_plane_iteration(PlaneArgs a, uint32_t K, unsigned grid, hipStream_t s, uint32_t in_flight,
-                                  int lm = 0);
+// many, a two-pass kernel with K lanes per virtual node for few.  32-bit labels, pushed queues
+// (the passes of eeg_run_batch launch their own).
+eeg_status launch_plane_iteration(PlaneArgs a, uint32_t K, unsigned grid, hipStream_t s, uint32_t in_flight);
 
 // Admission between iterations (one workgroup): pairs (pv[i], pc[i]) = (internal source,
 // column) get label `val`; their column bit is ORed into m_always, and into m_edges when the

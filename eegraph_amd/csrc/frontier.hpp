@@ -1,6 +1,6 @@
 // Sorted frontier queues, shared by the single-query traversals (relax.hip) and the batched
 // plane passes (batch.hip): a kernel that improved a vertex marks it (a byte per vertex and a byte
-// per 16384 vertices), and k_compact_frontier turns the marks into the next queue in vertex order.
+// per 16384 vertices), and compact_frontier turns the marks into the next queue in vertex order.
 //
 // Marks are bytes written by plain stores because atomics are performed past the L2 at about 24 G/s
 // whatever they do: as bits set with atomicOr they were half of the atomics of a traversal
@@ -38,7 +38,7 @@ __device__ __forceinline__ void set_mark(uint8_t* mark, uint8_t* cmark, uint32_t
 // Sorted frontier: the vertices that iteration `it` marked, with out-edges, as the next queue
 // (buffer it & 1, Ctl slot it % 3), in ascending id order within each block's 16384-vertex
 // chunk; chunks take their queue ranges in the order their atomic lands.  Marks are cleared as
-// they are read.  One thread per 16 vertices; replayed graphs resolve `it` from dev_it.
+// they are read.  One thread per 16 vertices.
 struct CompactArgs {
     uint8_t* mark;
     uint8_t* cmark;
@@ -48,17 +48,15 @@ struct CompactArgs {
     uint32_t *qa, *sa, *qb, *sb;  // queue buffers 0 and 1
     uint32_t cap;
     uint32_t it;
-    const uint32_t* dev_it;
-    uint32_t it_off;
 };
 
 // four bytes of 0 or 1 -> four bits
 __device__ __forceinline__ uint32_t mark_bits(uint32_t x) { return (x * 0x10204080u) >> 28; }
 
-__global__ __launch_bounds__(COMPACT_WG) void k_compact_frontier(CompactArgs a) {
-    const uint32_t it = a.dev_it ? *a.dev_it + a.it_off : a.it;
+// Every thread of the grid (COMPACT_WG a workgroup) calls it.
+__device__ __forceinline__ void compact_frontier(const CompactArgs& a) {
+    const uint32_t it = a.it;
     Ctl* ctl = a.ctl;
-    if (ctl->done) return;
     uint32_t* qout = (it & 1u) ? a.qb : a.qa;
     uint32_t* sout = (it & 1u) ? a.sb : a.sa;
     const int slot = (int)(it % 3u);

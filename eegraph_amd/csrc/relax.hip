@@ -25,6 +25,7 @@
 
 #include "engine.hpp"
 #include "frontier.hpp"
+#include "progress.hpp"
 
 namespace eeg {
 namespace {
@@ -68,18 +69,6 @@ struct RelaxArgs {
     uint32_t tbase;
     uint32_t all_first;      // iteration 1 runs every tile (CC: every vertex starts active)
 };
-
-// Progress of a run as its iterations start, written to pinned memory by one thread.  The words
-// are independent (the host waits for each on its own), so relaxed stores do.
-enum RunState : uint32_t { RUN_GOING = 0, RUN_DONE = 1, RUN_ERROR = 2 };
-__device__ __forceinline__ void publish(RunStatus* st, const Ctl* ctl, uint32_t it, uint32_t state) {
-    if (!st) return;
-    const unsigned long long now = (unsigned long long)wall_clock64();
-    if (it == 1) __hip_atomic_store(&st->t0, now, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    if (state == RUN_DONE) __hip_atomic_store(&st->t1, now, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    if (ctl->err) state = RUN_ERROR;
-    __hip_atomic_store(&st->word, ((unsigned long long)it << 8) | state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
 
 // BS threads per workgroup (256, 512 or 1024): a tile keeps TILE_EDGES edge slots, so a larger
 // workgroup runs fewer rounds of one edge per lane.
@@ -396,6 +385,11 @@ __global__ __launch_bounds__(BS) void k_relax(RelaxArgs a) {
     }
 }
 
+__global__ __launch_bounds__(COMPACT_WG) void k_compact_frontier(CompactArgs a) {
+    if (a.ctl->done) return;
+    compact_frontier(a);
+}
+
 // ---------------------------------------------------------------- initialisation
 // Initial labels (src/eegraph.cu:38-49 BFS/SSSP, :1549-1560 SSWP, :544-553 CC): the host
 // picks the values; CC passes the original ids, so components end labelled by their minimum
@@ -612,13 +606,6 @@ int cu_count(int device) {
     return c;
 }
 
-// Ticks of the device clock (wall_clock64) per millisecond.
-double clock_khz(int device) {
-    int khz = 0;
-    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) != hipSuccess || khz <= 0) khz = 100000;
-    return (double)khz;
-}
-
 }  // namespace
 
 namespace {
@@ -640,11 +627,6 @@ eeg_status ensure_tiles(Tigr& t, uint32_t K, hipStream_t s) {
     t.tiles_built = true;
     return EEG_OK;
 }
-
-// Iterations queued beyond the one that the device is known to have started: enough that it never
-// waits for the host (an iteration takes 9 us or more, seeing it start and queueing the next about
-// 8), and what is left to run dry after the last one is short.
-constexpr uint32_t RUN_AHEAD = 2;
 
 // Iterations launched for a limit of max_iters (>= 1): the fixpoint must be seen among them.  Whole
 // chunks, of 6 after the first iteration for queues, of 2, 4, 8, 8, ... for sweeps.
@@ -897,12 +879,7 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
         return EEG_OK;
     };
 
-    // (nothing of an earlier run writes the status any more: a run ends when its last status is
-    // seen, or with its stream synchronised)
-    volatile RunStatus* vs = w.status;
-    vs->word = 0;
-    vs->t0 = 0;
-    vs->t1 = 0;
+    reset_status(w.status);
     uint32_t it = 1;
     eeg_status rc = EEG_OK;
     Ctl hc{};
@@ -930,36 +907,17 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
         }
         hc = w.host_ctl[0];
     } else {
-        // The device reports each iteration as it starts; the host keeps RUN_AHEAD iterations
-        // queued beyond it and stops with the one that finds nothing to do.  (Replayed graphs of
+        // (Replayed graphs of
         // six iterations, polled by copies of the control block, ran up to 12 launches of ~4.5 us
         // past the end and took ~0.3 ms to instantiate: RMAT-14 SSSP 360 -> 240 us a call, RMAT-22
         // BFS 855 -> 753, first call 1189 -> 987; in-place SSWP, whose launches had events
         // between them, 1624 -> 1445.)
         const uint64_t limit = launch_limit(mode == M_QUEUE, max_iters);
         uint32_t state = RUN_GOING;
-        uint64_t started = 0;
-        for (uint32_t spins = 1;; ++spins) {
-            while (it <= limit && it <= started + RUN_AHEAD) EEG_TRY(launch(it++));
-            const unsigned long long word = vs->word;
-            state = (uint32_t)(word & 0xff);
-            if (state != RUN_GOING) break;
-            if (word >> 8 != started) {
-                started = word >> 8;
-                spins = 0;
-                continue;
-            }
-            if ((spins & 0x3fff) == 0) {  // a device error ends the wait; so does the last iteration
-                const hipError_t e = hipStreamQuery(s);
-                if (e == hipSuccess && it > limit && vs->word == word) break;
-                if (e != hipSuccess && e != hipErrorNotReady)
-                    return fail(EEG_ERR_DEVICE, "traversal failed: %s", hipGetErrorString(e));
-            }
-            __builtin_ia32_pause();
-        }
+        EEG_TRY(run_ahead(s, w.status, limit, &it, &state, launch));
         if (state == RUN_DONE && !ra.count_stats) {
             hc.done = 1;
-            hc.iters = (uint32_t)(vs->word >> 8) - 1;
+            hc.iters = (uint32_t)(w.status->word >> 8) - 1;
         } else {
             EEG_HIP(hipStreamSynchronize(s));
             EEG_HIP(hipMemcpy(&hc, ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
@@ -972,11 +930,9 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
     if (sorted && hc.done && !hc.err) w.marks_clear = true;
 
     if (st) {
-        // device clock from the start of the first iteration to the one that found nothing to do
-        while (hc.done && !vs->t1) __builtin_ia32_pause();
         st->iterations = hc.iters;
         st->launches = it - 1;
-        st->ms_traversal = hc.done ? (double)(vs->t1 - vs->t0) / clock_khz(g->device) : 0.0;
+        st->ms_traversal = hc.done ? run_ms(w.status, g->device) : 0.0;
         st->edges_relaxed = hc.stat[2];
         st->vnodes_processed = hc.stat[1];
         st->vertices_touched = hc.stat[0];
