@@ -792,7 +792,9 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
     const uint32_t wpc_queue = o.wgs_per_cu ? o.wgs_per_cu : std::max(1u, 24u / per);
     const unsigned grid_static =
         (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(static_tiles, (uint64_t)cus * wpc_static));
-    const unsigned grid_queue = (unsigned)cus * wpc_queue;
+    // a frontier has no more tiles than the graph (workgroups without one still take their turn: 6144
+    // of them on RMAT-14, which has 190 tiles)
+    const unsigned grid_queue = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(static_tiles, (uint64_t)cus * wpc_queue));
     KernelFn kfn = pick_kernel(alg, K, mode, block);
 
     RelaxArgs ra{};
