@@ -628,6 +628,8 @@ eeg_status ensure_tiles(Tigr& t, uint32_t K, hipStream_t s) {
     return EEG_OK;
 }
 
+constexpr uint32_t SORTED_FROM = 1u << 19;  // see run_traversal
+
 // Iterations launched for a limit of max_iters (>= 1): the fixpoint must be seen among them.  Whole
 // chunks, of 6 after the first iteration for queues, of 2, 4, 8, 8, ... for sweeps.
 uint64_t launch_limit(bool queue, uint64_t max_iters) {
@@ -654,7 +656,12 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
         default: return fail(EEG_ERR_INVALID_ARG, "unknown variant %u", o.variant);
     }
     if (o.frontier > EEG_FRONTIER_COMPACT) return fail(EEG_ERR_INVALID_ARG, "unknown frontier kind %u", o.frontier);
-    const bool sorted = mode == M_QUEUE && o.frontier == EEG_FRONTIER_SORTED;
+    const bool by_default = mode == M_QUEUE && o.frontier == EEG_FRONTIER_SORTED;
+    // Below SORTED_FROM vertices the sorted queue's second launch costs more than its order gives: the
+    // queue is pushed by the relaxations there (device time sorted / pushed, us: RMAT-14 SSSP 137 / 104,
+    // RMAT-16 213 / 164, RMAT-18 347 / 322, RMAT-20 571 / 579; grids of 60 k, 250 k and 1 M vertices 760 /
+    // 592, 891 / 778 and 1388 / 1535).
+    const bool sorted = by_default && g->n >= SORTED_FROM;
     const int alg = (int)algo;  // EEG_BFS..EEG_CC map onto A_BFS..A_CC
     if ((alg == A_SSSP || alg == A_SSWP) && !g->weighted)
         return fail(EEG_ERR_INVALID_ARG, "SSSP/SSWP need a weighted graph");
@@ -664,7 +671,7 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
     // limits iterations, names a frontier kind other than the default or sweeps every virtual
     // node propagates labels (device time of that against this: RMAT-22 1.9 / 0.21 ms,
     // 4096^2 grid 29 / 2.6 ms)
-    if (alg == A_CC && (sorted || mode == M_ASYNC) && !o.collect_activity && !o.count_work && !o.timing && !o.max_iters)
+    if (alg == A_CC && (by_default || mode == M_ASYNC) && !o.collect_activity && !o.count_work && !o.timing && !o.max_iters)
         return run_components(g, st, w, s);
     if (alg == A_CC) EEG_TRY(ensure_sym(g));
     Csr& c = (alg == A_CC) ? g->sym : g->out;

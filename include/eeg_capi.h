@@ -77,8 +77,10 @@ typedef enum eeg_variant {
 typedef enum eeg_frontier_kind {
     EEG_FRONTIER_SORTED = 0,  /* (default) vertex queue in ascending id order per 16384-vertex
                                  block, built from marks (a byte per vertex) after every
-                                 iteration; eeg_run_device_noalloc runs EEG_FRONTIER_COMPACT
-                                 for it (same answers; the marks would need memory) */
+                                 iteration; graphs of fewer than 2^19 vertices, where that
+                                 launch costs more than the order gives, and
+                                 eeg_run_device_noalloc (the marks would need memory) run
+                                 EEG_FRONTIER_COMPACT for it (same answers) */
     EEG_FRONTIER_FLAGS = 1,   /* per-vertex flag scan over every virtual node */
     EEG_FRONTIER_COMPACT = 2  /* vertex queue in the order vertices improve (ballot/prefix
                                  compaction per tile, dedup stamps) */
