@@ -1144,7 +1144,8 @@ struct BatchWork {
     DevMem mark;            // dense plane passes: vertices improved this iteration (frontier.hpp)
     int64_t wmax = -1;      // largest edge weight of the graph (-1: not measured yet)
     DevMem ovq;             // 8-bit SSSP passes: queries whose distances outgrew 8 bits
-    DevMem rowbuf;          // small answers on their way to the host (below HOST_COPY_FROM)
+    DevMem rowbuf;          // answers on their way to the host (below HOST_COPY_FROM)
+    HostMem small;          // ... small ones
     bool d8_off = false;    // a previous 8-bit SSSP pass flagged more than a quarter of its queries
     DevMem q[2], s[2], cand, stamp, ctl;
     uint32_t epoch = 1;
@@ -1483,6 +1484,12 @@ eeg_status batch_pass(eeg_graph* g, BatchWork& bw, hipStream_t s, uint32_t algo,
                         if (uint32_t* dst = row(q))
                             memcpy(dst + (size_t)i * per, (const uint32_t*)slot + (size_t)q * cnt, (size_t)cnt * 4);
                 }));
+        } else if (bytes <= HOST_SMALL) {
+            EEG_TRY(bw.small.alloc(bytes));
+            EEG_TRY(planes_out(0, n, n, 0, bw.small.as<uint32_t>()));
+            EEG_HIP(hipStreamSynchronize(s));
+            for (uint32_t q = 0; q < nsrc; ++q)
+                if (uint32_t* dst = row(q)) memcpy(dst, bw.small.as<uint32_t>() + (size_t)q * n, (size_t)n * 4);
         } else {
             EEG_TRY(bw.rowbuf.alloc(bytes + 4));
             EEG_TRY(planes_out(0, n, n, 0, bw.rowbuf.as<uint32_t>()));

@@ -450,8 +450,16 @@ extern "C" eeg_status eeg_csr_export_derived(eeg_graph* g, uint32_t which, uint6
 }
 
 // Labels in internal order to `out`, n words of host memory, in original order.
-static eeg_status labels_to_host(eeg_graph* g, const void* lab, void* out, DevMem& buf, hipStream_t st) {
+static eeg_status labels_to_host(eeg_graph* g, Work& w, void* out, hipStream_t st) {
     const size_t bytes = (size_t)g->n * 4;
+    const void* lab = w.lab.p;
+    if (bytes <= HOST_SMALL) {
+        EEG_TRY(w.small.alloc(bytes));
+        EEG_TRY(unpermute(g, lab, w.small.p, st, 0, g->n));
+        EEG_HIP(hipStreamSynchronize(st));
+        memcpy(out, w.small.p, bytes);
+        return EEG_OK;
+    }
     LentRing lent(g->device, bytes >= HOST_COPY_FROM);
     if (lent.r) {
         constexpr uint32_t words = HOST_SLOT_BYTES / 4;
@@ -466,9 +474,9 @@ static eeg_status labels_to_host(eeg_graph* g, const void* lab, void* out, DevMe
                 memcpy((uint32_t*)out + (size_t)i * words, slot, (size_t)part(i) * 4);
             });
     }
-    EEG_TRY(buf.alloc(bytes + 4));
-    EEG_TRY(unpermute(g, lab, buf.p, st, 0, g->n));
-    EEG_HIP(hipMemcpyAsync(out, buf.p, bytes, hipMemcpyDeviceToHost, st));
+    EEG_TRY(w.out.alloc(bytes + 4));
+    EEG_TRY(unpermute(g, lab, w.out.p, st, 0, g->n));
+    EEG_HIP(hipMemcpyAsync(out, w.out.p, bytes, hipMemcpyDeviceToHost, st));
     EEG_HIP(hipStreamSynchronize(st));
     return EEG_OK;
 }
@@ -513,7 +521,7 @@ static eeg_status run_common(eeg_graph* g, uint32_t algo, uint32_t source, const
             EEG_TRY(unpermute(g, g->work.lab.p, out, us, 0, g->n));
             EEG_HIP(hipStreamSynchronize(us));
         } else {
-            EEG_TRY(labels_to_host(g, g->work.lab.p, out, g->work.out, g->stream));
+            EEG_TRY(labels_to_host(g, g->work, out, g->stream));
         }
     }
     st->ms_total = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();

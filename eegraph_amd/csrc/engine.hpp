@@ -77,6 +77,30 @@ private:
     DevBlock block;
 };
 
+// Owning pinned host memory that kernels write (answers of at most HOST_SMALL bytes: a kernel's own
+// stores and a memcpy save the runtime's copy, ~30 us a call).
+constexpr size_t HOST_SMALL = (size_t)1 << 20;
+struct HostMem {
+    void* p = nullptr;
+    size_t bytes = 0;
+    HostMem() = default;
+    HostMem(const HostMem&) = delete;
+    HostMem& operator=(const HostMem&) = delete;
+    ~HostMem() {
+        if (p) (void)hipHostFree(p);
+    }
+    eeg_status alloc(size_t n) {
+        if (p && bytes >= n) return EEG_OK;
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        EEG_HIP(hipHostMalloc(&p, n, hipHostMallocDefault));
+        bytes = n;
+        return EEG_OK;
+    }
+    template <class T>
+    T* as() const { return static_cast<T*>(p); }
+};
+
 // Compressed sparse rows of one edge direction.
 struct Csr {
     uint32_t n = 0;
@@ -149,6 +173,7 @@ struct RunStatus {
 struct Work {
     DevMem lab;         // u32[n] (or f32 ranks), internal vertex order
     DevMem out;         // u32[n]: result in original vertex order before a host copy
+    HostMem small;      // ... a small one
     DevMem q[2], s[2];  // frontier queues: entry vertex ids and vnode prefix
     DevMem stamp;       // u32[n] iteration stamps for queue dedup
     DevMem flag;        // u32[n] iteration stamps for flag-scan frontiers
