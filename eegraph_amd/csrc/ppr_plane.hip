@@ -513,12 +513,11 @@ eeg_status PprPlane::init(eeg_graph* g, uint32_t Bc, float d, hipStream_t s) {
     grid_pull = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)cus * 8, ((uint64_t)t.nseg + 63) / 64));
     grid_fix = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)cus * 4, ((uint64_t)t.nmulti + 15) / 16));
     EEG_TRY(res_part.alloc((size_t)(grid_pull + grid_fix) * B * 8));
-    EEG_TRY(resid.alloc((size_t)B * 8));
     EEG_HIP(hipStreamSynchronize(s));
     return EEG_OK;
 }
 
-eeg_status PprPlane::iterate(eeg_graph* g, uint32_t j, const PprCols& cols, hipStream_t s, uint32_t W) {
+eeg_status PprPlane::iterate(eeg_graph* g, uint32_t j, const PprCols& cols, hipStream_t s, double* resid, uint32_t W) {
     if (W == 0) W = B;
     if ((W != 8 && W != 16 && W != 32) || W > B) return fail(EEG_ERR_INVALID_ARG, "pass width %u of %u columns", W, B);
     for (uint32_t q = W; q < B; ++q)
@@ -562,7 +561,7 @@ eeg_status PprPlane::iterate(eeg_graph* g, uint32_t j, const PprCols& cols, hipS
         if (t.nhub) k_pps_hub_chunks<32><<<grid_hub, WG, 0, s>>>(a.spill, t.hubs.as<uint4>(), t.nhub, t.nhubch, B);
         k_pps_fix<32><<<grid_fix, WG, 0, s>>>(a, fix_part);
     }
-    k_pps_reduce<<<W, WG, 0, s>>>(res_part.as<double>(), grid_pull + grid_fix, W, resid.as<double>());
+    k_pps_reduce<<<W, WG, 0, s>>>(res_part.as<double>(), grid_pull + grid_fix, W, resid);
     EEG_HIP(hipGetLastError());
     return EEG_OK;
 }
@@ -609,6 +608,11 @@ eeg_status run_ppr_batch(eeg_graph* g, const uint32_t* sources, uint32_t nsrc, c
     hipStream_t s = g->stream;
     DevMem dout;
     if (out_host) EEG_TRY(dout.alloc((size_t)n * 4 + 4));
+    // L1 changes in pinned memory: the host sees an iteration's by their arrival (a copy and a
+    // synchronisation took ~20 us of the 50 of an RMAT-14 iteration)
+    EEG_TRY(g->work.small.alloc(4096));
+    volatile uint64_t* arrived = g->work.small.as<uint64_t>();
+    constexpr uint64_t NOT_YET = ~0ull;  // no kernel writes this NaN
     std::vector<double> hres(B);
     hipEvent_t e0, e1;
     EEG_HIP(hipEventCreate(&e0));
@@ -633,9 +637,22 @@ eeg_status run_ppr_batch(eeg_graph* g, const uint32_t* sources, uint32_t nsrc, c
         }
         // columns are refilled lowest first, so a pass needs only the width of the busy ones
         // (a pass of 8 or 16 columns costs about 0.3 or 0.6 of one of 32)
-        EEG_TRY(pl.iterate(g, j, cols, s, pl.width_for(cols)));
-        EEG_HIP(hipMemcpyAsync(hres.data(), pl.resid.p, (size_t)B * 8, hipMemcpyDeviceToHost, s));
-        EEG_HIP(hipStreamSynchronize(s));
+        const uint32_t W = pl.width_for(cols);
+        for (uint32_t q = 0; q < W; ++q) arrived[q] = NOT_YET;
+        EEG_TRY(pl.iterate(g, j, cols, s, g->work.small.as<double>(), W));
+        for (uint32_t q = 0; q < W; ++q) {
+            for (uint32_t spins = 1; arrived[q] == NOT_YET; ++spins) {
+                if ((spins & 0x3fff) == 0) {  // a device error ends the wait
+                    const hipError_t e = hipStreamQuery(s);
+                    if (e != hipSuccess && e != hipErrorNotReady)
+                        return fail(EEG_ERR_DEVICE, "PPR planes: %s", hipGetErrorString(e));
+                    (void)hipGetLastError();  // "not ready" is no error of the next launch
+                }
+                __builtin_ia32_pause();
+            }
+            const uint64_t bits = arrived[q];
+            memcpy(&hres[q], &bits, 8);
+        }
         ++total_iters;
         cols.fresh = 0;
         for (uint32_t q = 0; q < B; ++q) {

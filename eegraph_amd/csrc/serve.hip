@@ -643,12 +643,8 @@ void PprEngine::loop() {
             PprCols cols = cur;
             cols.fresh = fresh;
             // columns are taken lowest first: the pass covers only up to the highest busy one
-            rc = pl.iterate(g, it, cols, st, pl.width_for(cols));
-            if (rc == EEG_OK &&
-                (hipMemcpyAsync(hres + (it % 4) * 32, pl.resid.p, (size_t)ncols * 8, hipMemcpyDeviceToHost, st) !=
-                     hipSuccess ||
-                 hipEventRecord(ev[it % 4], st) != hipSuccess))
-                rc = EEG_ERR_DEVICE;
+            rc = pl.iterate(g, it, cols, st, hres + (it % 4) * 32, pl.width_for(cols));
+            if (rc == EEG_OK && hipEventRecord(ev[it % 4], st) != hipSuccess) rc = EEG_ERR_DEVICE;
             if (rc == EEG_OK) inflight.push_back(it++);
         }
         if (rc != EEG_OK) {
