@@ -46,7 +46,8 @@ size_t block_size(size_t n) {
     return (n + step - 1) / step * step;
 }
 std::mutex g_blocks_mu;
-std::vector<DevBlock> g_blocks;  // oldest first
+// oldest first; never destroyed (handles may go while the process ends)
+std::vector<DevBlock>& g_blocks = *new std::vector<DevBlock>();
 size_t g_blocks_bytes = 0;
 
 bool find_block(size_t size, int device, DevBlock* out) {
@@ -120,7 +121,7 @@ HostRing::~HostRing() {
 
 namespace {
 std::mutex g_rings_mu;
-std::vector<HostRing*> g_rings;  // idle; what is left at the end goes with the process
+std::vector<HostRing*>& g_rings = *new std::vector<HostRing*>();  // idle; never destroyed, as above
 }  // namespace
 
 HostRing* take_host_ring(int device) {
