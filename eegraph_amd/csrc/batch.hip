@@ -938,15 +938,20 @@ __global__ void k_plane_rotate(const uint32_t* q, const Ctl* ctl, int slot,
 // (each lane taking one label from its own vertex's row read every line up to 32 times: 256 answers
 // of 2^18 vertices in 1.31 ms).  The answers usually go over PCIe, to pinned memory.
 constexpr uint32_t OUT_TILE = 64;
+struct WantedQueries {  // a bit per query; the others are left out
+    uint64_t w[MAXW];
+};
 template <int LM>
 __global__ __launch_bounds__(WG) void k_planes_out(const uint32_t* __restrict__ planes,
                                                    const uint32_t* __restrict__ perm, uint32_t count, uint32_t B,
                                                    uint32_t nq, uint32_t per, uint64_t pitch,
-                                                   uint32_t* __restrict__ out) {
+                                                   WantedQueries want, uint32_t* __restrict__ out) {
     constexpr uint32_t QPL = (LM == LM_W8 || LM == LM_D8) ? 4 : LM == LM_D16 ? 2 : 1;  // labels per word
     constexpr uint32_t WORDS = OUT_TILE / QPL;                                         // words per vertex
     __shared__ uint32_t sL[OUT_TILE][OUT_TILE + 1];  // [query][vertex]
     const uint32_t q0 = blockIdx.y * OUT_TILE;
+    const uint64_t wanted = want.w[blockIdx.y];
+    if (!wanted) return;
     for (uint32_t u0 = blockIdx.x * OUT_TILE; u0 < count; u0 += gridDim.x * OUT_TILE) {
         const uint32_t nu = min(OUT_TILE, count - u0);
         for (uint32_t i = threadIdx.x; i < nu * WORDS; i += WG) {
@@ -970,7 +975,7 @@ __global__ __launch_bounds__(WG) void k_planes_out(const uint32_t* __restrict__ 
         uint32_t* dst = out + part * pitch + (u0 - first);
         if (u < nu)
             for (uint32_t q = threadIdx.x / OUT_TILE; q < OUT_TILE && q0 + q < nq; q += WG / OUT_TILE)
-                dst[(uint64_t)(q0 + q) * stride + u] = sL[q][u];
+                if ((wanted >> q) & 1ull) dst[(uint64_t)(q0 + q) * stride + u] = sL[q][u];
         __syncthreads();
     }
 }
@@ -1447,20 +1452,27 @@ eeg_status batch_pass(eeg_graph* g, BatchWork& bw, hipStream_t s, uint32_t algo,
         if (lm == LM_D8) EEG_HIP(hipMemcpyAsync(ovq_out, bw.ovq.p, MAXW * 8, hipMemcpyDeviceToHost, s));
     }
     // answers: query-major, original vertex order
+    WantedQueries want{};
+    bool any = false;
+    for (uint32_t q = 0; q < nsrc; ++q)
+        if (bo.out || (bo.rows && bo.rows[q])) {
+            want.w[q / 64] |= 1ull << (q % 64);
+            any = true;
+        }
     auto planes_out = [&](uint32_t u0, uint32_t count, uint32_t per, uint64_t pitch, uint32_t* dst) -> eeg_status {
         const dim3 gr(std::max(1u, std::min(4096u, (count + OUT_TILE - 1) / OUT_TILE)), W);
         const uint32_t* pl = bw.planes.as<uint32_t>();
         const uint32_t* pm = g->perm.as<uint32_t>() + u0;
-        if (lm == LM_W8) k_planes_out<LM_W8><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, per, pitch, dst);
-        else if (lm == LM_D8) k_planes_out<LM_D8><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, per, pitch, dst);
-        else if (lm == LM_D16) k_planes_out<LM_D16><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, per, pitch, dst);
-        else k_planes_out<LM_U32><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, per, pitch, dst);
+        if (lm == LM_W8) k_planes_out<LM_W8><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, per, pitch, want, dst);
+        else if (lm == LM_D8) k_planes_out<LM_D8><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, per, pitch, want, dst);
+        else if (lm == LM_D16) k_planes_out<LM_D16><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, per, pitch, want, dst);
+        else k_planes_out<LM_U32><<<gr, WG, 0, s>>>(pl, pm, count, B, nsrc, per, pitch, want, dst);
         EEG_HIP(hipGetLastError());
         return EEG_OK;
     };
     if (bo.out && bo.device) {
         EEG_TRY(planes_out(0, n, n, 0, (uint32_t*)bo.out));
-    } else if (bo.out || bo.rows) {
+    } else if (any) {
         auto row = [&](uint32_t q) { return bo.rows ? bo.rows[q] : (uint32_t*)bo.out + (uint64_t)q * n; };
         const uint64_t bytes = (uint64_t)nsrc * n * 4;
         LentRing lent(g->device, bytes >= HOST_COPY_FROM);

@@ -56,6 +56,7 @@ eeg_status run_ahead(hipStream_t s, RunStatus* status, uint64_t limit, uint32_t*
             if (e == hipSuccess && *it > limit && vs->word == word) return EEG_OK;
             if (e != hipSuccess && e != hipErrorNotReady)
                 return fail(EEG_ERR_DEVICE, "traversal failed: %s", hipGetErrorString(e));
+            (void)hipGetLastError();  // "not ready" is no error of the next launch
         }
         __builtin_ia32_pause();
     }
