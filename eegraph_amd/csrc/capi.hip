@@ -11,6 +11,7 @@
 #include "engine.hpp"
 #include "hostcopy.hpp"
 #include "ppr_plane.hpp"
+#include "upload_chunks.hpp"
 
 namespace eeg {
 
@@ -250,11 +251,6 @@ extern "C" eeg_status eeg_graph_create_device(const uint32_t* d_src, const uint3
 }
 
 // Host arrays to device memory on the graph's stream, finished on return.
-struct Upload {
-    void* dst;
-    const void* src;
-    size_t bytes;
-};
 static eeg_status upload(eeg_graph* g, std::initializer_list<Upload> parts) {
     size_t total = 0;
     for (const Upload& u : parts) total += u.bytes;
@@ -265,26 +261,20 @@ static eeg_status upload(eeg_graph* g, std::initializer_list<Upload> parts) {
         EEG_HIP(hipStreamSynchronize(g->stream));
         return EEG_OK;
     }
-    // slots hold runs of one array each
-    std::vector<Upload> chunks;
-    chunks.reserve(total / HOST_SLOT_BYTES + parts.size());
-    for (const Upload& u : parts)
-        for (size_t o = 0; o < u.bytes; o += HOST_SLOT_BYTES)
-            chunks.push_back(Upload{(uint8_t*)u.dst + o, (const uint8_t*)u.src + o, std::min(HOST_SLOT_BYTES, u.bytes - o)});
+    const UploadChunks chunks{parts.begin(), parts.size(), HOST_SLOT_BYTES};
     return stage_to_device(
-        *lent.r, g->stream, (uint32_t)chunks.size(), host_copy_threads(total),
-        [&](uint32_t i, void* slot) { memcpy(slot, chunks[i].src, chunks[i].bytes); },
+        *lent.r, g->stream, chunks.count(), host_copy_threads(total),
+        [&](uint32_t i, void* slot) {
+            const Upload c = chunks[i];
+            memcpy(slot, c.src, c.bytes);
+        },
         [&](uint32_t i, uint32_t count, const void* slot) -> eeg_status {
-            // neighbours of one array in one copy (all but an array's last chunk fill their slots)
-            for (uint32_t k = 0; k < count;) {
-                uint32_t e = k + 1;
-                size_t bytes = chunks[i + k].bytes;
-                for (; e < count && chunks[i + e].dst == (uint8_t*)chunks[i + k].dst + (e - k) * HOST_SLOT_BYTES; ++e)
-                    bytes += chunks[i + e].bytes;
-                EEG_HIP(hipMemcpyAsync(chunks[i + k].dst, (const uint8_t*)slot + k * HOST_SLOT_BYTES, bytes,
-                                       hipMemcpyHostToDevice, g->stream));
-                k = e;
-            }
+            hipError_t e = hipSuccess;
+            chunks.runs(i, count, [&](void* dst, size_t off, size_t bytes) {
+                e = hipMemcpyAsync(dst, (const uint8_t*)slot + off, bytes, hipMemcpyHostToDevice, g->stream);
+                return e == hipSuccess;
+            });
+            EEG_HIP(e);
             return EEG_OK;
         });
 }
