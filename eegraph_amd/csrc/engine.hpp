@@ -93,7 +93,7 @@ struct HostMem {
         if (p && bytes >= n) return EEG_OK;
         if (p) (void)hipHostFree(p);
         p = nullptr;
-        EEG_HIP(hipHostMalloc(&p, n, hipHostMallocDefault));
+        EEG_HIP(hipHostMalloc(&p, n, hipHostMallocMapped | hipHostMallocCoherent));
         bytes = n;
         return EEG_OK;
     }

@@ -27,6 +27,7 @@
 #include "compensated.hpp"
 #include "ppr_plane.hpp"
 #include "scan.hpp"
+#include "wait_word.hpp"
 
 namespace eeg {
 namespace {
@@ -388,7 +389,9 @@ __global__ __launch_bounds__(WG) void k_pps_reduce(const double* __restrict__ pa
     if (threadIdx.x == 0) {
         double r = 0;
         for (int w = 0; w < WG / WAVE; ++w) r += s[w];
-        resid[blockIdx.x] = r;
+        // the host may wait for the word itself, so it goes out at system scope
+        __hip_atomic_store(reinterpret_cast<unsigned long long*>(resid) + blockIdx.x,
+                           (unsigned long long)__double_as_longlong(r), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -613,6 +616,15 @@ eeg_status run_ppr_batch(eeg_graph* g, const uint32_t* sources, uint32_t nsrc, c
     EEG_TRY(g->work.small.alloc(4096));
     volatile uint64_t* arrived = g->work.small.as<uint64_t>();
     constexpr uint64_t NOT_YET = ~0ull;  // no kernel writes this NaN
+    hipError_t failed = hipSuccess;
+    auto stream_state = [&] {
+        const hipError_t e = hipStreamQuery(s);
+        if (e == hipSuccess) return Queue::DRAINED;
+        (void)hipGetLastError();  // "not ready" is no error of the next launch
+        if (e == hipErrorNotReady) return Queue::BUSY;
+        failed = e;
+        return Queue::FAILED;
+    };
     std::vector<double> hres(B);
     hipEvent_t e0, e1;
     EEG_HIP(hipEventCreate(&e0));
@@ -641,15 +653,9 @@ eeg_status run_ppr_batch(eeg_graph* g, const uint32_t* sources, uint32_t nsrc, c
         for (uint32_t q = 0; q < W; ++q) arrived[q] = NOT_YET;
         EEG_TRY(pl.iterate(g, j, cols, s, g->work.small.as<double>(), W));
         for (uint32_t q = 0; q < W; ++q) {
-            for (uint32_t spins = 1; arrived[q] == NOT_YET; ++spins) {
-                if ((spins & 0x3fff) == 0) {  // a device error ends the wait
-                    const hipError_t e = hipStreamQuery(s);
-                    if (e != hipSuccess && e != hipErrorNotReady)
-                        return fail(EEG_ERR_DEVICE, "PPR planes: %s", hipGetErrorString(e));
-                    (void)hipGetLastError();  // "not ready" is no error of the next launch
-                }
-                __builtin_ia32_pause();
-            }
+            if (!wait_word(&arrived[q], NOT_YET, stream_state))
+                return fail(EEG_ERR_DEVICE, "PPR planes: %s",
+                            failed != hipSuccess ? hipGetErrorString(failed) : "an iteration left no residual");
             const uint64_t bits = arrived[q];
             memcpy(&hres[q], &bits, 8);
         }
