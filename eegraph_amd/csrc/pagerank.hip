@@ -308,10 +308,10 @@ __global__ __launch_bounds__(WG) void k_pr_fix(PullArgs a, const uint32_t* __res
     }
 }
 
-// Vertices without in-edges hold their teleport term from the first iteration on.
+// Vertices without in-edges hold their teleport term from the first iteration on.  In place the old
+// and the new ranks are the same memory, so the old one is read first and the pointers may alias.
 __global__ void k_pr_isolated(const uint64_t* __restrict__ in_row, const uint32_t* __restrict__ outdeg,
-                              uint32_t n, const float* __restrict__ x_old, const float* __restrict__ xl_old,
-                              float* __restrict__ x_new, float* __restrict__ xl_new,
+                              uint32_t n, const float* x_old, const float* xl_old, float* x_new, float* xl_new,
                               float* __restrict__ c_new, float base0, uint32_t pers, float pers_base,
                               double* res_part, const Ctl* ctl) {
     __shared__ double sRed[WG / WAVE];
@@ -321,11 +321,12 @@ __global__ void k_pr_isolated(const uint64_t* __restrict__ in_row, const uint32_
          v += (uint64_t)gridDim.x * blockDim.x) {
         if (in_row[v + 1] != in_row[v]) continue;
         const float base = (v == pers) ? pers_base : base0;
+        const double xo = (double)x_old[v] + (double)xl_old[v];
         x_new[v] = base;
         xl_new[v] = 0.0f;
         const uint32_t d = outdeg[v];
         c_new[v] = d ? base / (float)d : 0.0f;
-        res += fabs((double)base - ((double)x_old[v] + (double)xl_old[v]));
+        res += fabs((double)base - xo);
     }
     res = wave_sum(res);
     if (lane_id() == 0) sRed[threadIdx.x / WAVE] = res;
