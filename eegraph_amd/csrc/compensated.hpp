@@ -54,26 +54,15 @@ __device__ __forceinline__ Comp group_sum_first_lane(float x) {
 
 // New rank base + d * sum kept as an FP32 pair (hi, lo): the product d*s is split exactly with
 // an FMA, base + d*s with TwoSum, and the small terms folded into lo.  The pair carries ~46
-// bits, so the iteration settles on an exact fixed point instead of cycling by one FP32 ulp.
+// bits.  No contraction: the compiler would put d*s into an FMA with the base, whose TwoSum error
+// then holds the rounding error of the product that pe adds again.
 __device__ __forceinline__ void rank_pair(float base, float d, Comp sum, float* hi, float* lo) {
-    const float p = d * sum.s;
-    const float pe = fmaf(d, sum.s, -p);
-    const Comp q = two_sum(base, p);
-    const float small = q.e + (pe + d * sum.e);
-    const float h = q.s + small;            // fast two-sum: |q.s| >= |small|
-    *hi = h;
-    *lo = small - (h - q.s);
-}
-
-// The same with the product kept apart: contracted into an FMA with the base (as the compiler may
-// in rank_pair), d * s already carries the rounding error that pe adds again.
-__device__ __forceinline__ void rank_pair_split(float base, float d, Comp sum, float* hi, float* lo) {
 #pragma clang fp contract(off)
     const float p = d * sum.s;
     const float pe = fmaf(d, sum.s, -p);
     const Comp q = two_sum(base, p);
     const float small = q.e + (pe + d * sum.e);
-    const float h = q.s + small;
+    const float h = q.s + small;            // fast two-sum: |q.s| >= |small|
     *hi = h;
     *lo = small - (h - q.s);
 }

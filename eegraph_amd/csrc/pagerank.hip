@@ -651,7 +651,7 @@ __device__ __forceinline__ void finish_row(const FinishArgs& f, uint32_t v, Comp
     const double xo = (double)a.x_old[v] + (double)a.xl_old[v];
     const uint32_t d = a.outdeg[v];
     float hi, lo;
-    rank_pair_split(v == a.pers ? a.pers_base : a.base, a.damping, sum, &hi, &lo);
+    rank_pair(v == a.pers ? a.pers_base : a.base, a.damping, sum, &hi, &lo);
     a.x_new[v] = hi;
     a.xl_new[v] = lo;
     const double x = (double)hi + (double)lo;
