@@ -15,6 +15,14 @@
 // so results do not depend on the schedule.
 // Each column's L1 change is accumulated in FP64 per lane and reduced in a fixed order.
 //
+// A contribution rounded to one float holds the ranks a few ulps off their fixed point, and where the
+// paths have a period (grids, bipartite graphs) the phases of the iteration settle at different points:
+// the L1 change then stays near 1e-7 for good (16 of 28 restart vertices on grids of 3600 .. 60,000
+// vertices, 184 of 200 random bipartite graphs of up to 10).  So where the change falls too slowly,
+// each contribution's rounding error is added to the vertex's next contribution, as in the streamed
+// single query, until the stop.  The errors are a plane of their own, written and read only for such
+// columns (Feed below).
+//
 // Columns are independent: a column may start (fresh: x0 = e_s, nothing read from the planes)
 // at any iteration while others continue, which the serving loop uses to admit queries between
 // iterations.
@@ -110,6 +118,21 @@ __global__ void k_seg_desc(const uint64_t* __restrict__ row, const uint32_t* __r
     }
 }
 
+// Rounding errors of a column are fed back from an iteration on whose L1 change r follows
+// - r <= FEED_FROM / (1 - d): what single floats leave adds up to some 2^-24 / (1 - d),
+// - r > (d + (1 - d) / 4) * the change before: it falls by d or more but for rounding,
+// while r > FEED_TO; below, they are dropped, and the iteration settles on a fixed point for smaller
+// stops.  (CPU runs: grids and bipartite graphs, d = 0.5 .. 0.99, meet the 1e-7 stop at most a few
+// iterations after FP64 does; RMAT graphs are left alone.)
+constexpr double FEED_FROM = 1.5e-7, FEED_TO = 5e-8;
+enum Feed : uint32_t { FEED_WRITE = 1, FEED_READ = 2 };  // what an iteration does with the errors
+// Of a column, left by an iteration for the next one.
+struct PprColState {
+    double last;    // L1 change
+    uint32_t feed;  // Feed bits
+    uint32_t pad;
+};
+
 struct PlaneArgsP {
     const uint64_t* row;     // in-edge CSR
     const uint32_t* col;
@@ -129,6 +152,8 @@ struct PlaneArgsP {
     float damping;
     PprCols cols;
     uint32_t hub_chunks;     // 1: hubs' spill slots hold chunk sums every PPR_HUB_SEGS slots
+    float* err;              // rounding errors of the last contributions (null: not fed back)
+    const PprColState* col_state;  // of every column (that of a fresh one is its predecessor's)
     uint32_t S;              // row stride of the planes and spill slots (columns allocated);
                              // a pass of B <= S columns reads and writes the first B of a row
 };
@@ -138,22 +163,40 @@ __device__ __forceinline__ float2 old_rank(const PlaneArgsP& a, uint32_t v, uint
     return fresh ? make_float2(v == src ? 1.0f : 0.0f, 0.0f) : a.x_old[(uint64_t)v * a.S + q];
 }
 
-// New rank (hi, lo) from its gathered sum and the old one; adds the L1 change to res and returns
-// the new contribution.
-__device__ __forceinline__ float new_rank(float damping, bool restart, uint32_t od, float2 xo, Comp sum, float* hi,
-                                          float* lo, double& res) {
+// New rank (hi, lo) from its gathered sum and the old one; adds the L1 change to res.
+__device__ __forceinline__ void new_rank(float damping, bool restart, float2 xo, Comp sum, float* hi, float* lo,
+                                         double& res) {
     rank_pair(restart ? 1.0f - damping : 0.0f, damping, sum, hi, lo);
     res += fabs(((double)*hi + (double)*lo) - ((double)xo.x + (double)xo.y));
-    return od ? (*hi + *lo) / (float)od : 0.0f;
+}
+// The contribution of a rank to each out-neighbour.
+__device__ __forceinline__ float contribution(float hi, float lo, uint32_t od) {
+    return od ? (hi + lo) / (float)od : 0.0f;
+}
+// The contribution c with the last rounding error *e added; *e receives the error of the sum.  What c
+// itself lost is the remainder of its division (an FMA gives it exactly).
+__device__ __forceinline__ float fed_contribution(float c, float hi, float lo, uint32_t od, float* e) {
+    if (!od) return 0.0f;  // (nothing gathers it)
+    const float d = (float)od;
+    const float t = (fmaf(-c, d, hi) + lo) * __builtin_amdgcn_rcpf(d) + *e;
+    const float f = c + t;  // fast two-sum: |c| >= |t|, a few roundings of it
+    *e = t - (f - c);
+    return f;
 }
 
-// ... of entry vertex v in column q, written to the planes.
+// Column q of entry vertex v: rank and contribution into the planes.
 __device__ __forceinline__ void finish_col(const PlaneArgsP& a, uint32_t v, uint32_t q, uint32_t src, float2 xo,
-                                           uint32_t od, Comp sum, double& res) {
+                                           uint32_t od, Comp sum, uint32_t feed, double& res) {
     float hi, lo;
-    const float c = new_rank(a.damping, v == src, od, xo, sum, &hi, &lo, res);
+    new_rank(a.damping, v == src, xo, sum, &hi, &lo, res);
     const uint64_t o = (uint64_t)v * a.S + q;
     a.x_new[o] = make_float2(hi, lo);
+    float c = contribution(hi, lo, od);
+    if (feed & FEED_WRITE) {
+        float e = (feed & FEED_READ) ? a.err[o] : 0.0f;
+        c = fed_contribution(c, hi, lo, od, &e);
+        a.err[o] = e;
+    }
     a.c_new[o] = c;
 }
 
@@ -193,7 +236,7 @@ __global__ __launch_bounds__(WG) void k_pps_pull(PlaneArgsP a) {
     typedef float vec __attribute__((ext_vector_type(VW)));
     typedef float vec2 __attribute__((ext_vector_type(2 * VW)));  // pairs of VW columns (16-byte parts)
     const uint32_t lane = lane_id(), sub = lane % PQ, grp = lane / PQ;
-    uint32_t src[C], fresh = 0;
+    uint32_t src[C], fresh = 0, wr = 0, rd = 0;  // bits: fresh, errors written, errors read
     float c0[C];
     double res[C];
     auto col = [&](int i) { return (uint32_t)(i / VW * PQ * VW + i % VW) + sub * VW; };
@@ -201,7 +244,10 @@ __global__ __launch_bounds__(WG) void k_pps_pull(PlaneArgsP a) {
     for (int i = 0; i < C; ++i) {
         src[i] = a.cols.src[col(i)];
         // a fresh column's contributions are e_src / outdeg(src): what is read for it is dropped
-        fresh |= ((a.cols.fresh >> col(i)) & 1u) << i;
+        const uint32_t fr = (a.cols.fresh >> col(i)) & 1u, fd = a.err && !fr ? a.col_state[col(i)].feed : 0u;
+        fresh |= fr << i;
+        wr |= (fd & FEED_WRITE ? 1u : 0u) << i;
+        rd |= (fd & FEED_READ ? 1u : 0u) << i;
         const uint32_t sod = (src[i] != PPR_IDLE) ? a.outdeg[src[i]] : 0u;
         c0[i] = sod ? 1.0f / (float)sod : 0.0f;
         res[i] = 0.0;
@@ -252,11 +298,26 @@ __global__ __launch_bounds__(WG) void k_pps_pull(PlaneArgsP a) {
                     const float2 old = ((fresh >> f) & 1u) ? make_float2(v == src[f] ? 1.0f : 0.0f, 0.0f)
                                                            : make_float2(xo[2 * i], xo[2 * i + 1]);
                     float hi, lo;
-                    cn[i] = new_rank(a.damping, v == src[f], od, old, acc[f], &hi, &lo, res[f]);
+                    new_rank(a.damping, v == src[f], old, acc[f], &hi, &lo, res[f]);
+                    cn[i] = contribution(hi, lo, od);
                     xn[2 * i] = hi;
                     xn[2 * i + 1] = lo;
                 }
                 *reinterpret_cast<vec2*>(a.x_new + o) = xn;
+                if ((wr >> (j * VW)) & ((1u << VW) - 1)) {
+                    vec* ep = reinterpret_cast<vec*>(a.err + o);
+                    const vec eo = *ep;
+                    vec en;
+#pragma unroll
+                    for (int i = 0; i < VW; ++i) {
+                        const int f = j * VW + i;
+                        float e = ((rd >> f) & 1u) ? eo[i] : 0.0f;
+                        const float c = fed_contribution(cn[i], xn[2 * i], xn[2 * i + 1], od, &e);
+                        if ((wr >> f) & 1u) cn[i] = c;
+                        en[i] = e;
+                    }
+                    *ep = en;
+                }
                 *reinterpret_cast<vec*>(a.c_new + o) = cn;
             }
         } else {
@@ -344,6 +405,7 @@ __global__ __launch_bounds__(WG) void k_pps_fix(PlaneArgsP a, double* res_part) 
     const uint32_t lane = lane_id(), q = lane % B, grp = lane / B;
     const uint32_t src = a.cols.src[q];
     const bool fresh = (a.cols.fresh >> q) & 1u;
+    const uint32_t feed = a.err && !fresh ? a.col_state[q].feed : 0u;
     double res = 0.0;
     const uint64_t nw = (uint64_t)gridDim.x * (WG / WAVE);
     for (uint64_t w = (uint64_t)blockIdx.x * (WG / WAVE) + threadIdx.x / WAVE; w * G < a.nmulti; w += nw) {
@@ -359,7 +421,7 @@ __global__ __launch_bounds__(WG) void k_pps_fix(PlaneArgsP a, double* res_part) 
         const uint32_t cnt = hub ? (ns + PPR_HUB_SEGS - 1) / PPR_HUB_SEGS : ns;
         const uint64_t stride = hub ? (uint64_t)PPR_HUB_SEGS * a.S : (uint64_t)a.S;
         const Comp acc = sum_slots<B>(a.spill + (uint64_t)mb * a.S + q, cnt, stride);
-        finish_col(a, v, q, src, xo, od, acc, res);
+        finish_col(a, v, q, src, xo, od, acc, feed, res);
     }
     store_residual<B>(res, res_part);
 }
@@ -368,8 +430,10 @@ __global__ __launch_bounds__(WG) void k_pps_fix(PlaneArgsP a, double* res_part) 
 // and added in index order, then a fixed tree.  Bound by the latency of its loads, so four are in
 // flight per thread and the columns run side by side (3072 partials x 16 columns: 59 us as one
 // workgroup with a load at a time, 9 us as this).
+// Decides as well what the next iteration does with the column's rounding errors (feed).
 __global__ __launch_bounds__(WG) void k_pps_reduce(const double* __restrict__ part, uint32_t nparts, uint32_t W,
-                                                   double* __restrict__ resid) {
+                                                   double* __restrict__ resid, double damping, uint32_t fresh,
+                                                   PprColState* __restrict__ col_state) {
     __shared__ double s[WG / WAVE];
     const double* p = part + blockIdx.x;
     double t = 0;
@@ -392,6 +456,12 @@ __global__ __launch_bounds__(WG) void k_pps_reduce(const double* __restrict__ pa
         // the host may wait for the word itself, so it goes out at system scope
         __hip_atomic_store(reinterpret_cast<unsigned long long*>(resid) + blockIdx.x,
                            (unsigned long long)__double_as_longlong(r), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        PprColState& c = col_state[blockIdx.x];
+        const bool first = (fresh >> blockIdx.x) & 1u, fed = !first && (c.feed & FEED_WRITE);
+        const bool slow = !first && r > (damping + 0.25 * (1.0 - damping)) * c.last;
+        const bool on = r > FEED_TO && r <= FEED_FROM / (1.0 - damping) && (fed || slow);
+        c.feed = on ? FEED_WRITE | (fed ? FEED_READ : 0u) : 0u;
+        c.last = r;
     }
 }
 
@@ -495,7 +565,7 @@ eeg_status ensure_ppr_seg(eeg_graph* g) {
 }
 
 size_t PprPlane::bytes_for(uint32_t n, uint32_t B, uint32_t nspill) {
-    return (size_t)n * B * 4 * 6 + (size_t)nspill * B * 8 + (size_t)B * 8 * 4096;
+    return (size_t)n * B * 4 * 7 + (size_t)nspill * B * 8 + (size_t)B * 8 * 4096;
 }
 
 eeg_status PprPlane::init(eeg_graph* g, uint32_t Bc, float d, hipStream_t s) {
@@ -511,11 +581,14 @@ eeg_status PprPlane::init(eeg_graph* g, uint32_t Bc, float d, hipStream_t s) {
         for (DevMem* m : {&c[k], &x[k]}) EEG_HIP(hipMemsetAsync(m->p, 0, m->bytes, s));
     }
     EEG_TRY(spill.alloc((size_t)t.nspill * B * 8 + 16));
+    EEG_TRY(col_state.alloc(32 * sizeof(PprColState)));
+    EEG_HIP(hipMemsetAsync(col_state.p, 0, 32 * sizeof(PprColState), s));
     int cus = 256;
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->device);
     grid_pull = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)cus * 8, ((uint64_t)t.nseg + 63) / 64));
     grid_fix = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)cus * 4, ((uint64_t)t.nmulti + 15) / 16));
     EEG_TRY(res_part.alloc((size_t)(grid_pull + grid_fix) * B * 8));
+    if (err.alloc(plane) != EEG_OK) clear_error();  // without it errors are not fed back
     EEG_HIP(hipStreamSynchronize(s));
     return EEG_OK;
 }
@@ -547,6 +620,8 @@ eeg_status PprPlane::iterate(eeg_graph* g, uint32_t j, const PprCols& cols, hipS
     a.damping = damping;
     a.cols = cols;
     a.hub_chunks = t.nhub ? 1u : 0u;
+    a.err = err.as<float>();
+    a.col_state = col_state.as<PprColState>();
     a.S = B;
     // residual partials and the reduction are W columns wide
     double* fix_part = res_part.as<double>() + (size_t)grid_pull * W;
@@ -564,7 +639,8 @@ eeg_status PprPlane::iterate(eeg_graph* g, uint32_t j, const PprCols& cols, hipS
         if (t.nhub) k_pps_hub_chunks<32><<<grid_hub, WG, 0, s>>>(a.spill, t.hubs.as<uint4>(), t.nhub, t.nhubch, B);
         k_pps_fix<32><<<grid_fix, WG, 0, s>>>(a, fix_part);
     }
-    k_pps_reduce<<<W, WG, 0, s>>>(res_part.as<double>(), grid_pull + grid_fix, W, resid);
+    k_pps_reduce<<<W, WG, 0, s>>>(res_part.as<double>(), grid_pull + grid_fix, W, resid,
+                                  (double)damping, cols.fresh, col_state.as<PprColState>());
     EEG_HIP(hipGetLastError());
     return EEG_OK;
 }
@@ -595,7 +671,7 @@ eeg_status PprPlane::extract(eeg_graph* g, uint32_t j, uint32_t q, uint32_t src,
 
 // Batched PPR (eeg_run_batch): up to B columns in flight; every column iterates from e_src
 // until its own L1 change drops below epsilon, is read out and takes the next source, so each
-// answer is the single-query iteration's, summed in a fixed order.
+// answer is the single-query iteration's within its stop, summed in a fixed order.
 eeg_status run_ppr_batch(eeg_graph* g, const uint32_t* sources, uint32_t nsrc, const eeg_opts& o, float* out_host,
                          eeg_stats* st) {
     const float d = o.damping > 0 ? o.damping : 0.85f;

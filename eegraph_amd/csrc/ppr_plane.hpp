@@ -30,6 +30,8 @@ struct PprPlane {
     float damping = 0.85f;
     DevMem c[2];                // n x B contributions x/outdeg
     DevMem x[2];                // n x B ranks as compensated pairs (hi, lo)
+    DevMem err;                 // n x B rounding errors of the contributions (may be absent)
+    DevMem col_state;           // PprColState of every column
     DevMem spill;               // nspill x B float2
     DevMem res_part;            // (grid_pull + grid_fix) x B doubles
     unsigned grid_pull = 0, grid_fix = 0;
