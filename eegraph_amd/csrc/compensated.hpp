@@ -67,4 +67,34 @@ __device__ __forceinline__ void rank_pair(float base, float d, Comp sum, float* 
     *lo = small - (h - q.s);
 }
 
+// The contribution of a rank to each out-neighbour.
+__device__ __forceinline__ float contribution(float hi, float lo, uint32_t od) {
+    return od ? (hi + lo) / (float)od : 0.0f;
+}
+// The contribution c with the last rounding error *e added; *e receives the error of the sum.  What c
+// itself lost is the remainder of its division (an FMA gives it exactly).
+__device__ __forceinline__ float fed_contribution(float c, float hi, float lo, uint32_t od, float* e) {
+    if (!od) return 0.0f;  // (nothing gathers it)
+    const float d = (float)od;
+    const float t = (fmaf(-c, d, hi) + lo) * __builtin_amdgcn_rcpf(d) + *e;
+    const float f = c + t;  // fast two-sum: |c| >= |t|, a few roundings of it
+    *e = t - (f - c);
+    return f;
+}
+
+// Rounding errors of contributions are fed back from an iteration on whose L1 change r follows
+// - r <= FEED_FROM / (1 - d): what single floats leave adds up to some 2^-24 / (1 - d),
+// - r > (d + (1 - d) / 4) * the change before (`last`): it falls by d or more but for rounding,
+// while r > FEED_TO; below, they are dropped, and the iteration settles on a fixed point for smaller
+// stops.  (CPU runs: grids and bipartite graphs, d = 0.5 .. 0.99, meet the 1e-7 stop at most a few
+// iterations after FP64 does; RMAT graphs are left alone.)
+constexpr double FEED_FROM = 1.5e-7, FEED_TO = 5e-8;
+enum Feed : uint32_t { FEED_WRITE = 1, FEED_READ = 2 };  // what an iteration does with the errors
+// Feed bits of the next iteration; `was`: of the one that ended.
+__device__ __forceinline__ uint32_t next_feed(double r, double last, double d, uint32_t was) {
+    const bool slow = r > (d + 0.25 * (1.0 - d)) * last;
+    if (!(r > FEED_TO && r <= FEED_FROM / (1.0 - d) && ((was & FEED_WRITE) || slow))) return 0u;
+    return FEED_WRITE | ((was & FEED_WRITE) ? FEED_READ : 0u);
+}
+
 }  // namespace eeg

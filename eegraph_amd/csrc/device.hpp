@@ -140,7 +140,9 @@ struct Ctl {
     unsigned long long stat[4];    // entries staged, vnodes pushed, edges relaxed, updates
     double residual[4];            // PR: L1 residual of the last iterations (slot i&3)
     double mass;                   // PR delta push / PPR: residual mass still unpushed
-    double pad2[3];
+    uint32_t feed;                 // PR pull: Feed bits of the next iteration (compensated.hpp)
+    uint32_t pad1;
+    double pad2[2];
 };
 
 }  // namespace eeg

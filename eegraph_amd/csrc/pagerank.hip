@@ -58,16 +58,23 @@ struct PullArgs {
     float pers_base;         // its teleport term, 1-d
     uint32_t strided;        // in place: workgroup b takes tiles b, b + grid, ... (see k_pr_pull)
     const uint32_t* tstart;  // first entry of each tile (vlist position)
+    float* cerr;             // per vertex: rounding error of its last contribution (null: dropped)
 };
 
 // New rank of v from its gathered sum; xo = old rank (hi + lo), d = out-degree.
 __device__ __forceinline__ void finish_vertex(const PullArgs& a, uint32_t v, Comp sum, double xo, uint32_t d,
-                                              double& res) {
+                                              uint32_t feed, double& res) {
     float hi, lo;
     rank_pair(v == a.pers ? a.pers_base : a.base, a.damping, sum, &hi, &lo);
     a.x_new[v] = hi;
     a.xl_new[v] = lo;
-    a.c_new[v] = d ? (hi + lo) / (float)d : 0.0f;
+    float c = contribution(hi, lo, d);
+    if (feed & FEED_WRITE) {
+        float e = (feed & FEED_READ) ? a.cerr[v] : 0.0f;
+        c = fed_contribution(c, hi, lo, d, &e);
+        a.cerr[v] = e;
+    }
+    a.c_new[v] = c;
     res += fabs(((double)hi + (double)lo) - xo);
 }
 
@@ -96,6 +103,7 @@ __global__ __launch_bounds__(WG, K >= 8 ? 8 : 4) void k_pr_pull(PullArgs a) {
     __shared__ double sRed[WG / WAVE];
 
     if (a.ctl->done) return;
+    const uint32_t feed = a.cerr ? a.ctl->feed : 0u;
     double res = 0.0;
     const uint32_t T = a.P, nE = a.nz;
     const uint32_t ntiles = (T + TV - 1) / TV;
@@ -185,7 +193,7 @@ __global__ __launch_bounds__(WG, K >= 8 ? 8 : 4) void k_pr_pull(PullArgs a) {
                 const bool continues = sS[k + 1] > t1;
                 if (!started_before && !continues) {
                     const float2 xo = sXo[k];
-                    finish_vertex(a, a.vlist[e_start + k], acc, (double)xo.x + (double)xo.y, sOd[k], res);
+                    finish_vertex(a, a.vlist[e_start + k], acc, (double)xo.x + (double)xo.y, sOd[k], feed, res);
                 } else if (started_before) {
                     a.spill[2 * tile] = make_float2(acc.s, acc.e);      // head
                 } else {
@@ -261,6 +269,7 @@ __global__ __launch_bounds__(WG) void k_pr_fix(PullArgs a, const uint32_t* __res
                                                uint32_t TV, double* res_part) {
     __shared__ double sRed[WG / WAVE];
     if (a.ctl->done) return;
+    const uint32_t feed = a.cerr ? a.ctl->feed : 0u;
     double res = 0.0;
     for (uint32_t i = blockIdx.x * WG + threadIdx.x; i < nspan; i += gridDim.x * WG) {
         const uint32_t pos = span[i];
@@ -273,7 +282,7 @@ __global__ __launch_bounds__(WG) void k_pr_fix(PullArgs a, const uint32_t* __res
             acc = comp_add(acc, Comp{h.x, h.y});
         }
         const uint32_t v = a.vlist[pos];
-        finish_vertex(a, v, acc, (double)a.x_old[v] + (double)a.xl_old[v], a.outdeg[v], res);
+        finish_vertex(a, v, acc, (double)a.x_old[v] + (double)a.xl_old[v], a.outdeg[v], feed, res);
     }
     const int lane = (int)lane_id();
     const uint32_t nw = gridDim.x * (WG / WAVE);
@@ -295,7 +304,7 @@ __global__ __launch_bounds__(WG) void k_pr_fix(PullArgs a, const uint32_t* __res
         }
         if (lane == 0) {
             const uint32_t v = a.vlist[pos];
-            finish_vertex(a, v, acc, (double)a.x_old[v] + (double)a.xl_old[v], a.outdeg[v], res);
+            finish_vertex(a, v, acc, (double)a.x_old[v] + (double)a.xl_old[v], a.outdeg[v], feed, res);
         }
     }
     res = wave_sum(res);
@@ -343,7 +352,7 @@ __global__ void k_pr_isolated(const uint64_t* __restrict__ in_row, const uint32_
 // a tree), so the residual is deterministic.
 constexpr int RED_WG = 1024;
 __global__ __launch_bounds__(RED_WG) void k_pr_reduce(const double* __restrict__ part, uint32_t nparts, Ctl* ctl,
-                                                      uint32_t it, double eps) {
+                                                      uint32_t it, double eps, double damping) {
     __shared__ double sRed[RED_WG];
     if (ctl->done) return;
     // strided per thread, four loads in flight, added in index order (the same sum as one at
@@ -365,6 +374,7 @@ __global__ __launch_bounds__(RED_WG) void k_pr_reduce(const double* __restrict__
         __syncthreads();
     }
     if (threadIdx.x == 0) {
+        ctl->feed = next_feed(sRed[0], ctl->residual[(it - 1) & 3], damping, ctl->feed);
         ctl->residual[it & 3] = sRed[0];
         ctl->iters = it;
         if (sRed[0] < eps) ctl->done = 1;
@@ -912,7 +922,11 @@ eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_
     }
     EEG_TRY(w.spill.alloc((size_t)(ntiles + 1) * 2 * sizeof(float2)));
     if (stream) EEG_TRY(w.psum.alloc((size_t)ps.nz * sizeof(float2)));
-    if (stream && !pairs) EEG_TRY(w.cerr.alloc((size_t)n * 4));
+    if (!pairs) {
+        const eeg_status got = w.cerr.alloc((size_t)n * 4);
+        if (stream) EEG_TRY(got);
+        else if (got != EEG_OK) clear_error();  // the pull does without
+    }
     // vertices whose virtual nodes cross a tile boundary (finished by k_pr_fix)
     const DevMem& span = t.span;
     const uint32_t nshort = t.nspan, nlong = t.nspan_long;
@@ -964,6 +978,7 @@ eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_
     pa.pers_base = 1.0f - d;
     pa.strided = inplace ? 1u : 0u;
     pa.tstart = t.prstart.as<uint32_t>();
+    pa.cerr = stream ? nullptr : w.cerr.as<float>();
     double* red = w.red.as<double>();
     auto pull_fn = (K == 4) ? k_pr_pull<4> : (K == 8) ? k_pr_pull<8> : (K == 16) ? k_pr_pull<16> : k_pr_pull<32>;
 
@@ -1045,7 +1060,7 @@ eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_
             EEG_HIP(hipMemsetAsync(red + grid_pull + grid_fix, 0, grid_iso * sizeof(double), s));
         }
         // (the streamed gather sums the residual at the start of the next iteration)
-        if (!stream) k_pr_reduce<<<1, RED_WG, 0, s>>>(red, nparts, ctl, it, eps);
+        if (!stream) k_pr_reduce<<<1, RED_WG, 0, s>>>(red, nparts, ctl, it, eps, (double)d);
         EEG_HIP(hipGetLastError());
         if (recorded.size() <= it) recorded.resize((size_t)it + 64, 0);
         recorded[it] = (rec || o.timing) ? 1 : 0;

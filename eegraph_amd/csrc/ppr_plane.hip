@@ -118,14 +118,6 @@ __global__ void k_seg_desc(const uint64_t* __restrict__ row, const uint32_t* __r
     }
 }
 
-// Rounding errors of a column are fed back from an iteration on whose L1 change r follows
-// - r <= FEED_FROM / (1 - d): what single floats leave adds up to some 2^-24 / (1 - d),
-// - r > (d + (1 - d) / 4) * the change before: it falls by d or more but for rounding,
-// while r > FEED_TO; below, they are dropped, and the iteration settles on a fixed point for smaller
-// stops.  (CPU runs: grids and bipartite graphs, d = 0.5 .. 0.99, meet the 1e-7 stop at most a few
-// iterations after FP64 does; RMAT graphs are left alone.)
-constexpr double FEED_FROM = 1.5e-7, FEED_TO = 5e-8;
-enum Feed : uint32_t { FEED_WRITE = 1, FEED_READ = 2 };  // what an iteration does with the errors
 // Of a column, left by an iteration for the next one.
 struct PprColState {
     double last;    // L1 change
@@ -169,21 +161,6 @@ __device__ __forceinline__ void new_rank(float damping, bool restart, float2 xo,
     rank_pair(restart ? 1.0f - damping : 0.0f, damping, sum, hi, lo);
     res += fabs(((double)*hi + (double)*lo) - ((double)xo.x + (double)xo.y));
 }
-// The contribution of a rank to each out-neighbour.
-__device__ __forceinline__ float contribution(float hi, float lo, uint32_t od) {
-    return od ? (hi + lo) / (float)od : 0.0f;
-}
-// The contribution c with the last rounding error *e added; *e receives the error of the sum.  What c
-// itself lost is the remainder of its division (an FMA gives it exactly).
-__device__ __forceinline__ float fed_contribution(float c, float hi, float lo, uint32_t od, float* e) {
-    if (!od) return 0.0f;  // (nothing gathers it)
-    const float d = (float)od;
-    const float t = (fmaf(-c, d, hi) + lo) * __builtin_amdgcn_rcpf(d) + *e;
-    const float f = c + t;  // fast two-sum: |c| >= |t|, a few roundings of it
-    *e = t - (f - c);
-    return f;
-}
-
 // Column q of entry vertex v: rank and contribution into the planes.
 __device__ __forceinline__ void finish_col(const PlaneArgsP& a, uint32_t v, uint32_t q, uint32_t src, float2 xo,
                                            uint32_t od, Comp sum, uint32_t feed, double& res) {
@@ -457,10 +434,8 @@ __global__ __launch_bounds__(WG) void k_pps_reduce(const double* __restrict__ pa
         __hip_atomic_store(reinterpret_cast<unsigned long long*>(resid) + blockIdx.x,
                            (unsigned long long)__double_as_longlong(r), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         PprColState& c = col_state[blockIdx.x];
-        const bool first = (fresh >> blockIdx.x) & 1u, fed = !first && (c.feed & FEED_WRITE);
-        const bool slow = !first && r > (damping + 0.25 * (1.0 - damping)) * c.last;
-        const bool on = r > FEED_TO && r <= FEED_FROM / (1.0 - damping) && (fed || slow);
-        c.feed = on ? FEED_WRITE | (fed ? FEED_READ : 0u) : 0u;
+        const bool first = (fresh >> blockIdx.x) & 1u;
+        c.feed = next_feed(r, first ? r : c.last, damping, first ? 0u : c.feed);
         c.last = r;
     }
 }

@@ -1,4 +1,4 @@
-"""PageRank where paths have a period (grids, bipartite graphs): every form of the sync iteration meets
+"""PageRank where paths have a period (grids, bipartite graphs): every form of the iteration meets
 its 1e-7 stop, as soon as the FP64 iteration does, and holds the right ranks.  Sizes lie on both sides of
 the 19,456 vertices up to which single queries carry contributions as pairs.
 
@@ -62,6 +62,15 @@ def test_single(case):
     check(x, st["iterations"], ref("pr"))
     for src, r in zip(srcs[:4], ppr):
         x, st = g.run("ppr", int(src), variant="sync_push_dd")
+        check(x, st["iterations"], r)
+
+
+def test_in_place(case):
+    n, g, srcs, ref, ppr = case
+    x, st = g.run("pr", 0, variant="async_push_dd")
+    check(x, st["iterations"], ref("pr"))
+    for src, r in zip(srcs[:6], ppr):
+        x, st = g.run("ppr", int(src), variant="async_push_dd")
         check(x, st["iterations"], r)
 
 
