@@ -1167,8 +1167,9 @@ struct BatchWork {
 
 namespace {
 
-// Limits of iterations are rounded up to this many (as passes of whole chunks ran once).
-constexpr uint64_t BATCH_CHUNK = 6;
+// Limits of iterations are rounded up to this many (as passes of whole chunks ran once), or with timing
+// to the second.
+constexpr uint64_t BATCH_CHUNK = 6, BATCH_CHUNK_TIMED = 8;
 
 // Compaction of a dense plane pass's marks into the queue the push would have written.
 CompactArgs compact_args(const PlaneArgs& a) {
@@ -1431,7 +1432,8 @@ eeg_status batch_pass(eeg_graph* g, BatchWork& bw, hipStream_t s, uint32_t algo,
     };
     reset_status(&bw.host->status);
     uint32_t j = 1, state = RUN_GOING;
-    const uint64_t limit = ((uint64_t)max_iters + 16 + BATCH_CHUNK - 1) / BATCH_CHUNK * BATCH_CHUNK;
+    const uint64_t chunk = o.timing ? BATCH_CHUNK_TIMED : BATCH_CHUNK;
+    const uint64_t limit = ((uint64_t)max_iters + 16 + chunk - 1) / chunk * chunk;
     const eeg_status ran = run_ahead(s, &bw.host->status, limit, &j, &state, launch);
     bw.epoch = base + j + 2;
     if (ran != EEG_OK) return ran;

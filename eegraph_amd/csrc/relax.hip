@@ -631,9 +631,10 @@ eeg_status ensure_tiles(Tigr& t, uint32_t K, hipStream_t s) {
 constexpr uint32_t SORTED_FROM = 1u << 19;  // see run_traversal
 
 // Iterations launched for a limit of max_iters (>= 1): the fixpoint must be seen among them.  Whole
-// chunks, of 6 after the first iteration for queues, of 2, 4, 8, 8, ... for sweeps.
-uint64_t launch_limit(bool queue, uint64_t max_iters) {
-    if (queue) return max_iters < 8 ? 7 : 1 + 6 * ((max_iters - 2) / 6 + 1);
+// chunks, of 6 after the first iteration for queues, of 2, 4, 8, 8, ... for sweeps and for queues whose
+// launches are timed.
+uint64_t launch_limit(bool by_six, uint64_t max_iters) {
+    if (by_six) return max_iters < 8 ? 7 : 1 + 6 * ((max_iters - 2) / 6 + 1);
     return max_iters < 7 ? 6 : 6 + 8 * ((max_iters + 1) / 8);
 }
 
@@ -921,7 +922,7 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
         // past the end and took ~0.3 ms to instantiate: RMAT-14 SSSP 360 -> 240 us a call, RMAT-22
         // BFS 855 -> 753, first call 1189 -> 987; in-place SSWP, whose launches had events
         // between them, 1624 -> 1445.)
-        const uint64_t limit = launch_limit(mode == M_QUEUE, max_iters);
+        const uint64_t limit = launch_limit(mode == M_QUEUE && !o.timing, max_iters);
         uint32_t state = RUN_GOING;
         EEG_TRY(run_ahead(s, w.status, limit, &it, &state, launch));
         if (state == RUN_DONE && !ra.count_stats) {
