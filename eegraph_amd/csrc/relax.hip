@@ -722,7 +722,10 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
     if (mode == M_ASYNC) EEG_TRY(w.vnpush.alloc((size_t)t.P * 4 + 4));
 
     // ---- labels, control block and first frontier
-    const uint32_t base = w.epoch;  // iteration it uses stamp base + it
+    // Iteration it uses stamp base + it.  All of them are taken at once, so that a run that ends early
+    // with an error leaves none to be used again; one that ends well gives back the rest.
+    const uint32_t base = w.epoch;
+    w.epoch = (uint32_t)std::min<uint64_t>((uint64_t)base + max_iters + 200, 0xfffffff0ull);
     const bool seeded = (alg != A_CC);
     Ctl* ctl = w.ctl.as<Ctl>();
     {
@@ -924,7 +927,11 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
         // between them, 1624 -> 1445.)
         const uint64_t limit = launch_limit(mode == M_QUEUE && !o.timing, max_iters);
         uint32_t state = RUN_GOING;
-        EEG_TRY(run_ahead(s, w.status, limit, &it, &state, launch));
+        const eeg_status ran = run_ahead(s, w.status, limit, &it, &state, launch);
+        if (ran != EEG_OK) {  // iterations queued so far still report to the status
+            (void)hipStreamSynchronize(s);
+            return ran;
+        }
         if (state == RUN_DONE && !ra.count_stats) {
             hc.done = 1;
             hc.iters = (uint32_t)(w.status->word >> 8) - 1;
