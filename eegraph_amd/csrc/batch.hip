@@ -1436,7 +1436,10 @@ eeg_status batch_pass(eeg_graph* g, BatchWork& bw, hipStream_t s, uint32_t algo,
     const uint64_t limit = ((uint64_t)max_iters + 16 + chunk - 1) / chunk * chunk;
     const eeg_status ran = run_ahead(s, &bw.host->status, limit, &j, &state, launch);
     bw.epoch = base + j + 2;
-    if (ran != EEG_OK) return ran;
+    if (ran != EEG_OK) {  // iterations queued so far still report to the status
+        (void)hipStreamSynchronize(s);
+        return ran;
+    }
     if (state == RUN_DONE) {
         hc.iters = (uint32_t)(bw.host->status.word >> 8) - 1;
     } else {
