@@ -69,8 +69,8 @@ inline double clock_khz(int device) {
     return (double)khz;
 }
 
-// Device time of a finished run, from the start of its first iteration to the one that found nothing
-// to do.
+// Device time of a run, from the start of its first iteration to the one that found nothing to do, or
+// to the end of the last one admitted.
 inline double run_ms(const RunStatus* status, int device) {
     const volatile RunStatus* vs = status;
     while (!vs->t1) __builtin_ia32_pause();

@@ -390,6 +390,11 @@ __global__ __launch_bounds__(COMPACT_WG) void k_compact_frontier(CompactArgs a) 
     compact_frontier(a);
 }
 
+// Behind the last iteration that a limit admits: the end of a run that has not found its own.
+__global__ void k_run_end(RunStatus* st) {
+    if (threadIdx.x == 0 && st->t1 == 0) st->t1 = (unsigned long long)wall_clock64();
+}
+
 // ---------------------------------------------------------------- initialisation
 // Initial labels (src/eegraph.cu:38-49 BFS/SSSP, :1549-1560 SSWP, :544-553 CC): the host
 // picks the values; CC passes the original ids, so components end labelled by their minimum
@@ -914,6 +919,8 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
             else activity.push_back((uint32_t)(h.stat[3] - upd_before));
             upd_before = h.stat[3];
             if (++it > max_iters) {
+                k_run_end<<<1, 64, 0, s>>>(w.status);
+                EEG_HIP(hipStreamSynchronize(s));
                 rc = fail(EEG_ERR_NOT_CONVERGED, "no fixpoint after %u iterations", max_iters);
                 break;
             }
@@ -927,7 +934,11 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
         // between them, 1624 -> 1445.)
         const uint64_t limit = launch_limit(mode == M_QUEUE && !o.timing, max_iters);
         uint32_t state = RUN_GOING;
-        const eeg_status ran = run_ahead(s, w.status, limit, &it, &state, launch);
+        const eeg_status ran = run_ahead(s, w.status, limit, &it, &state, [&](uint32_t i) -> eeg_status {
+            EEG_TRY(launch(i));
+            if (i == limit) k_run_end<<<1, 64, 0, s>>>(w.status);
+            return EEG_OK;
+        });
         if (ran != EEG_OK) {  // iterations queued so far still report to the status
             (void)hipStreamSynchronize(s);
             return ran;
@@ -949,7 +960,7 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
     if (st) {
         st->iterations = hc.iters;
         st->launches = it - 1;
-        st->ms_traversal = hc.done ? run_ms(w.status, g->device) : 0.0;
+        st->ms_traversal = (hc.done || w.status->t1) ? run_ms(w.status, g->device) : 0.0;
         st->edges_relaxed = hc.stat[2];
         st->vnodes_processed = hc.stat[1];
         st->vertices_touched = hc.stat[0];

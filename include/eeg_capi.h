@@ -124,7 +124,10 @@ typedef struct eeg_opts {
 typedef struct eeg_stats {
     uint32_t iterations;        /* sweeps / frontier rounds that did work */
     uint32_t launches;          /* relaxation kernels launched (includes no-op overshoot) */
-    double ms_traversal;        /* device events: first relaxation kernel -> converged */
+    double ms_traversal;        /* device time from the first relaxation kernel to the fixpoint, or to
+                                   the last iteration that a limit admits: the device clock as the
+                                   kernels read it (BFS, SSSP, SSWP, batches of them), device events
+                                   (PageRank, union-find) */
     double ms_total;            /* host wall clock: label init + traversal + copy-out */
     double ms_kernel_sum;       /* sum of per-launch relaxation kernel times (opts.timing) */
     uint32_t kernels_timed;     /* number of launches summed in ms_kernel_sum */

@@ -3,10 +3,13 @@ every launch timed; batched levels rounded up to 6, or 8 with timing), and that 
 stopped answers the next one as if nothing had been.
 
 Along the path 0 -> 1 -> .. -> L a BFS from 0 takes L iterations and one more that finds nothing."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import eegraph_amd as eg
+import eegraph_amd._lib as L
 import oracle_py as O
 
 pytestmark = pytest.mark.gpu
@@ -73,3 +76,16 @@ def test_a_stopped_handle_answers_again(n, variant, frontier):
                 assert np.array_equal(out, ref), (alg, max_iters)
                 if n < 100:
                     break
+
+
+@pytest.mark.parametrize("n", SIZES)
+@pytest.mark.parametrize("variant,frontier,activity", [("sync_push_dd", "sorted", 0), ("sync_push_dd", "compact", 1),
+                                                       ("sync_push_dd", "flags", 0), ("sync_push_dd", "sorted", 1)])
+def test_a_stopped_run_reports_its_time(n, variant, frontier, activity):
+    with path(n, 40) as g:
+        out, st = np.empty(n, np.uint32), L.Stats()
+        o = eg.make_opts(variant=variant, frontier=frontier, max_iters=3, collect_activity=bool(activity))
+        rc = L.lib.eeg_run(g.handle, L.BFS, 0, C.byref(o), out.ctypes.data, C.byref(st))
+        assert rc == L.ERR_NOT_CONVERGED
+        assert 0 < st.ms_traversal <= st.ms_total
+        assert out[0] == 0 and out[3] == 3 and out[39] == eg.DIST_INFINITY
