@@ -1501,13 +1501,12 @@ eeg_status batch_pass(eeg_graph* g, BatchWork& bw, hipStream_t s, uint32_t algo,
                         if (uint32_t* dst = row(q))
                             memcpy(dst + (size_t)i * per, (const uint32_t*)slot + (size_t)q * cnt, (size_t)cnt * 4);
                 }));
-        } else if (bytes <= HOST_SMALL) {
-            EEG_TRY(bw.small.alloc(bytes));
+        } else if (bytes <= HOST_SMALL && bw.small.alloc(bytes)) {
             EEG_TRY(planes_out(0, n, n, 0, bw.small.as<uint32_t>()));
             EEG_HIP(hipStreamSynchronize(s));
             for (uint32_t q = 0; q < nsrc; ++q)
                 if (uint32_t* dst = row(q)) memcpy(dst, bw.small.as<uint32_t>() + (size_t)q * n, (size_t)n * 4);
-        } else {
+        } else {  // (or no pinned memory)
             EEG_TRY(bw.rowbuf.alloc(bytes + 4));
             EEG_TRY(planes_out(0, n, n, 0, bw.rowbuf.as<uint32_t>()));
             if (bo.out) {

@@ -444,8 +444,7 @@ extern "C" eeg_status eeg_csr_export_derived(eeg_graph* g, uint32_t which, uint6
 static eeg_status labels_to_host(eeg_graph* g, Work& w, void* out, hipStream_t st) {
     const size_t bytes = (size_t)g->n * 4;
     const void* lab = w.lab.p;
-    if (bytes <= HOST_SMALL) {
-        EEG_TRY(w.small.alloc(bytes));
+    if (bytes <= HOST_SMALL && w.small.alloc(bytes)) {
         EEG_TRY(unpermute(g, lab, w.small.p, st, 0, g->n));
         EEG_HIP(hipStreamSynchronize(st));
         memcpy(out, w.small.p, bytes);

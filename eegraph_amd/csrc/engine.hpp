@@ -78,7 +78,8 @@ private:
 };
 
 // Owning pinned host memory that kernels write (answers of at most HOST_SMALL bytes: a kernel's own
-// stores and a memcpy save the runtime's copy, ~30 us a call).
+// stores and a memcpy save the runtime's copy, ~30 us a call).  Where none can be had the callers fall
+// back on device memory and that copy.
 constexpr size_t HOST_SMALL = (size_t)1 << 20;
 struct HostMem {
     void* p = nullptr;
@@ -89,13 +90,15 @@ struct HostMem {
     ~HostMem() {
         if (p) (void)hipHostFree(p);
     }
-    eeg_status alloc(size_t n) {
-        if (p && bytes >= n) return EEG_OK;
+    bool alloc(size_t n) {  // false: none to be had (no error is recorded)
+        if (p && bytes >= n) return true;
         if (p) (void)hipHostFree(p);
-        p = nullptr;
-        EEG_HIP(hipHostMalloc(&p, n, hipHostMallocMapped | hipHostMallocCoherent));
         bytes = n;
-        return EEG_OK;
+        if (hipHostMalloc(&p, n, hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess) return true;
+        (void)hipGetLastError();
+        p = nullptr;
+        bytes = 0;
+        return false;
     }
     template <class T>
     T* as() const { return static_cast<T*>(p); }

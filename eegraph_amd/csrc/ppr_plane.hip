@@ -663,8 +663,12 @@ eeg_status run_ppr_batch(eeg_graph* g, const uint32_t* sources, uint32_t nsrc, c
     DevMem dout;
     if (out_host) EEG_TRY(dout.alloc((size_t)n * 4 + 4));
     // L1 changes in pinned memory: the host sees an iteration's by their arrival (a copy and a
-    // synchronisation took ~20 us of the 50 of an RMAT-14 iteration)
-    EEG_TRY(g->work.small.alloc(4096));
+    // synchronisation took ~20 us of the 50 of an RMAT-14 iteration), or where none can be pinned in
+    // device memory, copied
+    DevMem dres;
+    const bool pinned = g->work.small.alloc(4096);
+    if (!pinned) EEG_TRY(dres.alloc((size_t)B * 8));
+    double* resid = pinned ? g->work.small.as<double>() : dres.as<double>();
     volatile uint64_t* arrived = g->work.small.as<uint64_t>();
     constexpr uint64_t NOT_YET = ~0ull;  // no kernel writes this NaN
     hipError_t failed = hipSuccess;
@@ -701,9 +705,13 @@ eeg_status run_ppr_batch(eeg_graph* g, const uint32_t* sources, uint32_t nsrc, c
         // columns are refilled lowest first, so a pass needs only the width of the busy ones
         // (a pass of 8 or 16 columns costs about 0.3 or 0.6 of one of 32)
         const uint32_t W = pl.width_for(cols);
-        for (uint32_t q = 0; q < W; ++q) arrived[q] = NOT_YET;
-        EEG_TRY(pl.iterate(g, j, cols, s, g->work.small.as<double>(), W));
-        for (uint32_t q = 0; q < W; ++q) {
+        for (uint32_t q = 0; pinned && q < W; ++q) arrived[q] = NOT_YET;
+        EEG_TRY(pl.iterate(g, j, cols, s, resid, W));
+        if (!pinned) {
+            EEG_HIP(hipMemcpyAsync(hres.data(), resid, (size_t)W * 8, hipMemcpyDeviceToHost, s));
+            EEG_HIP(hipStreamSynchronize(s));
+        }
+        for (uint32_t q = 0; pinned && q < W; ++q) {
             if (!wait_word(&arrived[q], NOT_YET, stream_state))
                 return fail(EEG_ERR_DEVICE, "PPR planes: %s",
                             failed != hipSuccess ? hipGetErrorString(failed) : "an iteration left no residual");
