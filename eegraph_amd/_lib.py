@@ -126,6 +126,7 @@ _sig("eeg_graph_create_device", C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, u64
 _sig("eeg_graph_create_rmat", C.c_int, u32, u32, C.c_double, C.c_double, C.c_double, u64, u32,
      u32, C.c_int, P(C.c_void_p))
 _sig("eeg_graph_destroy", C.c_int, C.c_void_p)
+_sig("eeg_trim", C.c_int, P(u64))
 _sig("eeg_graph_get_info", C.c_int, C.c_void_p, P(GraphInfo))
 _sig("eeg_graph_prepare", C.c_int, C.c_void_p, u32, u32)
 _sig("eeg_tigr_export", C.c_int, C.c_void_p, u32, C.c_void_p, C.c_void_p, C.c_void_p, P(u64))
@@ -151,7 +152,7 @@ _sig("eeg_energy_read", C.c_int, C.c_int, P(C.c_double), P(u64))
 EXPORTS = [
     "eeg_strerror", "eeg_last_error", "eeg_device_count", "eeg_gen_rmat", "eeg_gen_grid_size",
     "eeg_gen_grid", "eeg_load_edgelist", "eeg_save_edgelist", "eeg_edgelist_free",
-    "eeg_graph_create", "eeg_graph_create_device", "eeg_graph_create_rmat", "eeg_graph_destroy",
+    "eeg_graph_create", "eeg_graph_create_device", "eeg_graph_create_rmat", "eeg_graph_destroy", "eeg_trim",
     "eeg_graph_get_info", "eeg_graph_prepare", "eeg_tigr_export", "eeg_csr_export",
     "eeg_csr_export_derived", "eeg_run",
     "eeg_run_device", "eeg_run_device_noalloc", "eeg_run_batch", "eeg_run_packed", "eeg_autotune", "eeg_server_create",

@@ -24,6 +24,14 @@ def device_count():
     return c.value
 
 
+def trim():
+    """Gives the memory that the library keeps for later calls (freed device blocks, at most 1 GiB,
+    and idle pinned buffers) back to the device and the host; returns its bytes."""
+    b = C.c_uint64(0)
+    L.check(L.lib.eeg_trim(C.byref(b)), "eeg_trim")
+    return b.value
+
+
 def gen_rmat(scale, edge_factor, a=0.57, b=0.19, c=0.19, seed=1, wmin=1, wmax=64,
              weights=True, threads=0):
     """RMAT edge list (src, dst, w) of edge_factor << scale edges, counter-based."""

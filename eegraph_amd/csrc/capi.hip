@@ -62,21 +62,25 @@ bool find_block(size_t size, int device, DevBlock* out) {
         }
     return false;
 }
-// Frees kept blocks, oldest first, until at most `keep` bytes are left.
-void drop_blocks(size_t keep) {
+// Frees kept blocks, oldest first, until at most `keep` bytes are left; bytes freed.
+uint64_t drop_blocks(size_t keep) {
+    uint64_t freed = 0;
     while (true) {
         DevBlock b;
         {
             std::lock_guard<std::mutex> lk(g_blocks_mu);
-            if (g_blocks.empty() || g_blocks_bytes <= keep) return;
+            if (g_blocks.empty() || g_blocks_bytes <= keep) return freed;
             b = g_blocks.front();
             g_blocks.erase(g_blocks.begin());
             g_blocks_bytes -= b.size;
         }
         (void)hipFree(b.p);
+        freed += b.size;
     }
 }
 }  // namespace
+
+uint64_t drop_dev_blocks() { return drop_blocks(0); }
 
 hipError_t take_dev_block(size_t bytes, DevBlock* out) {
     DevBlock b;
@@ -163,6 +167,19 @@ void give_host_ring(HostRing* r) {
     }
     delete r;
 }
+
+namespace {
+// Frees the idle rings; their bytes.
+uint64_t drop_host_rings() {
+    std::vector<HostRing*> idle;
+    {
+        std::lock_guard<std::mutex> lk(g_rings_mu);
+        idle.swap(g_rings);
+    }
+    for (HostRing* r : idle) delete r;
+    return (uint64_t)idle.size() * HOST_SLOTS * HOST_SLOT_BYTES;
+}
+}  // namespace
 
 // The owner has synchronised the stream: no record of these events is pending here.
 Work::~Work() {
@@ -350,6 +367,17 @@ extern "C" eeg_status eeg_graph_destroy(eeg_graph* g) {
     DeviceGuard dg;
     (void)hipSetDevice(g->device);
     delete g;
+    // where memory is short, whoever closes a graph wants it back
+    size_t avail = 0, total = 0;
+    if (hipMemGetInfo(&avail, &total) != hipSuccess) (void)hipGetLastError();
+    else if (avail < total / 8) (void)drop_dev_blocks();
+    return EEG_OK;
+}
+
+extern "C" eeg_status eeg_trim(uint64_t* freed_bytes) {
+    clear_error();
+    const uint64_t freed = drop_dev_blocks() + drop_host_rings();
+    if (freed_bytes) *freed_bytes = freed;
     return EEG_OK;
 }
 

@@ -28,7 +28,9 @@ namespace eeg {
 // most DEV_KEPT_MAX in all, and handed out again (a hipFree of 64 MiB takes 0.33 ms and a hipMalloc
 // 0.07; building a graph of 16.8 M edges, one query and the end of the handle spent 9 of 21 ms in
 // them).  Freeing waits for the device, as hipFree does, so a block handed out again has no users
-// on any stream.  When memory runs out, what is kept is freed and the request repeated.
+// on any stream.  When memory runs out, what is kept is freed and the request repeated.  For other
+// users of the card it is given back by eeg_trim, and when a handle is closed while the card has less
+// than an eighth of its memory free.
 constexpr size_t DEV_BLOCK_MAX = (size_t)256 << 20;
 constexpr size_t DEV_KEPT_MAX = (size_t)1 << 30;
 struct DevBlock {
@@ -38,6 +40,7 @@ struct DevBlock {
 };
 hipError_t take_dev_block(size_t bytes, DevBlock* out);
 void free_dev_block(const DevBlock& b);
+uint64_t drop_dev_blocks();  // frees everything kept (its bytes)
 
 // Owning device allocation.
 struct DevMem {

@@ -959,6 +959,7 @@ extern "C" eeg_status eeg_server_create(eeg_graph* g, const eeg_server_cfg* cfg,
     srv->discard = (c.flags & EEG_SERVER_DISCARD_LABELS) != 0;
     srv->t0 = Clock::now();
     const uint32_t n = g->n;
+    (void)drop_dev_blocks();  // budgets are shares of the free memory
     if (c.label_budget_bytes == 0) {
         size_t fr = 0, tot = 0;
         EEG_HIP(hipMemGetInfo(&fr, &tot));

@@ -215,7 +215,15 @@ eeg_status eeg_graph_create_device(const uint32_t* d_src, const uint32_t* d_dst,
 eeg_status eeg_graph_create_rmat(uint32_t scale, uint32_t edge_factor, double a, double b,
                                  double c, uint64_t seed, uint32_t wmin, uint32_t wmax,
                                  int device, eeg_graph** out);
+/* The handle's memory is free for this library at once.  For other users of the card: freed device
+ * blocks of up to 256 MiB, 1 GiB of them in all, stay with the library for the next handles and runs,
+ * and up to two pinned host buffers of 32 MiB.  They are given back by eeg_trim, when a request of the
+ * library's own runs out of memory, and (device blocks) when a handle is destroyed while less than an
+ * eighth of the card's memory is free. */
 eeg_status eeg_graph_destroy(eeg_graph* g);
+/* Frees the memory kept for later calls, on every device; *freed_bytes (may be NULL): how much.  Waits
+ * for the devices concerned.  Handles and runs in progress are not touched. */
+eeg_status eeg_trim(uint64_t* freed_bytes);
 eeg_status eeg_graph_get_info(const eeg_graph* g, eeg_graph_info* info);
 
 /* Builds derived device tables ahead of time so traversals do not pay for them:
