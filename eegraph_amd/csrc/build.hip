@@ -394,8 +394,6 @@ eeg_status build_csr_from_device_edges(eeg_graph* g, const uint32_t* d_src, cons
         EEG_HIP(hipMemsetAsync(orow.p, 0, ((size_t)n + 1) * 8, st));
     }
     if (m >= 1ull << 28) vin.release();  // (waits; 8 B an edge, which the rows below take again)
-    EEG_TRY(c.col.alloc(m * 4));
-    if (d_w) EEG_TRY(c.w.alloc(m * 4));
     DevMem key, kout, ids, tmpn, shift;
     unsigned long long stats[2] = {0, 0};
     g->h_perm.resize(n);
@@ -421,6 +419,14 @@ eeg_status build_csr_from_device_edges(eeg_graph* g, const uint32_t* d_src, cons
     }
     EEG_TRY(scan_exclusive(NewDegLoad{orow.as<uint64_t>(), g->inv.as<uint32_t>(), n}, RowStore{c.row.as<uint64_t>()},
                            (uint64_t)n + 1, st, nullptr));
+    // (last, so that nothing is asked for after it)
+    if (c.col.alloc(m * 4) != EEG_OK || (d_w && c.w.alloc(m * 4) != EEG_OK)) {
+        vin.release();  // short of memory: what the sorts needed goes first
+        tmp.release();
+        clear_error();
+        EEG_TRY(c.col.alloc(m * 4));
+        if (d_w) EEG_TRY(c.w.alloc(m * 4));
+    }
     if (m) {
         k_row_shift<<<grid_for(n), WG, 0, st>>>(g->perm.as<uint32_t>(), orow.as<uint64_t>(), c.rowp(), n,
                                                 shift.as<int64_t>());

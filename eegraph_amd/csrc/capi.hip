@@ -38,29 +38,29 @@ eeg_status Work::progress() {
 
 // ---------------------------------------------------------------- device blocks (DevMem)
 namespace {
-// Blocks of one size are interchangeable, so sizes are rounded up to an eighth of the power of two
-// below (12.5% at most).
-size_t block_size(size_t n) {
-    if (n > DEV_BLOCK_MAX) return n;
-    if (n <= 4096) return 4096;
-    const size_t step = ((size_t)1 << (63 - __builtin_clzll(n))) / 8;
-    return (n + step - 1) / step * step;
-}
+// Whole pages are asked for and no more, so that a card that is nearly full holds as much as without
+// kept blocks; a request takes a kept block that is up to an eighth larger.
+size_t block_size(size_t n) { return (n + 4095) / 4096 * 4096; }
 std::mutex g_blocks_mu;
 // oldest first; never destroyed (handles may go while the process ends)
 std::vector<DevBlock>& g_blocks = *new std::vector<DevBlock>();
 size_t g_blocks_bytes = 0;
 
+// The smallest kept block that will do; of two alike the one freed last.
 bool find_block(size_t size, int device, DevBlock* out) {
     std::lock_guard<std::mutex> lk(g_blocks_mu);
-    for (size_t i = g_blocks.size(); i-- > 0;)
-        if (g_blocks[i].size == size && g_blocks[i].device == device) {
-            *out = g_blocks[i];
-            g_blocks.erase(g_blocks.begin() + (ptrdiff_t)i);
-            g_blocks_bytes -= size;
-            return true;
-        }
-    return false;
+    size_t best = g_blocks.size();
+    for (size_t i = g_blocks.size(); i-- > 0;) {
+        const DevBlock& b = g_blocks[i];
+        if (b.device == device && b.size >= size && b.size <= size + size / 8 &&
+            (best == g_blocks.size() || b.size < g_blocks[best].size))
+            best = i;
+    }
+    if (best == g_blocks.size()) return false;
+    *out = g_blocks[best];
+    g_blocks.erase(g_blocks.begin() + (ptrdiff_t)best);
+    g_blocks_bytes -= out->size;
+    return true;
 }
 // Frees kept blocks, oldest first, until at most `keep` bytes are left; bytes freed.
 uint64_t drop_blocks(size_t keep) {

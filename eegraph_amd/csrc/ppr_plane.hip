@@ -563,9 +563,12 @@ eeg_status PprPlane::init(eeg_graph* g, uint32_t Bc, float d, hipStream_t s) {
     grid_pull = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)cus * 8, ((uint64_t)t.nseg + 63) / 64));
     grid_fix = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)cus * 4, ((uint64_t)t.nmulti + 15) / 16));
     EEG_TRY(res_part.alloc((size_t)(grid_pull + grid_fix) * B * 8));
-    if (err.alloc(plane) != EEG_OK) clear_error();  // without it errors are not fed back
     EEG_HIP(hipStreamSynchronize(s));
     return EEG_OK;
+}
+
+void PprPlane::take_err() {
+    if (err.alloc((size_t)n * B * 4 + 16) != EEG_OK) clear_error();
 }
 
 eeg_status PprPlane::iterate(eeg_graph* g, uint32_t j, const PprCols& cols, hipStream_t s, double* resid, uint32_t W) {
@@ -662,6 +665,7 @@ eeg_status run_ppr_batch(eeg_graph* g, const uint32_t* sources, uint32_t nsrc, c
     hipStream_t s = g->stream;
     DevMem dout;
     if (out_host) EEG_TRY(dout.alloc((size_t)n * 4 + 4));
+    pl.take_err();
     // L1 changes in pinned memory: the host sees an iteration's by their arrival (a copy and a
     // synchronisation took ~20 us of the 50 of an RMAT-14 iteration), or where none can be pinned in
     // device memory, copied

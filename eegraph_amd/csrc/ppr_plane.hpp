@@ -37,6 +37,7 @@ struct PprPlane {
     unsigned grid_pull = 0, grid_fix = 0;
     static size_t bytes_for(uint32_t n, uint32_t B, uint32_t nspill);
     eeg_status init(eeg_graph* g, uint32_t B, float damping, hipStream_t s);
+    void take_err();  // the plane of errors, once everything else is there; does without if it must
     // one Jacobi iteration for every column; resid (pinned memory, or any that kernels can write)
     // receives each column's L1 change, its last launch writes it.  W (8, 16 or 32, at most B; 0 = B)
     // columns per pass: columns W.. must be idle, the pass reads and writes the first W of every

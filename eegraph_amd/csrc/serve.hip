@@ -592,6 +592,7 @@ eeg_status PprEngine::init(eeg_graph* g, uint32_t B, float damping) {
     for (auto& e : ev) EEG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     EEG_HIP(hipHostMalloc((void**)&hres, 4 * 32 * sizeof(double), hipHostMallocMapped | hipHostMallocCoherent));
     EEG_TRY(pl.init(g, B, damping, st));
+    pl.take_err();
     for (uint32_t q = 0; q < 32; ++q) cur.src[q] = PPR_IDLE;
     cur.fresh = 0;
     col.assign(ncols, nullptr);

@@ -1,0 +1,137 @@
+"""Calls on a card that is nearly full.  A child process runs them with a hipMalloc that refuses what goes
+past a budget (preloaded beside whatever is preloaded already): a call that fits some budget fits every
+larger one, with the same answer, and needs no more than its comment says."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SHIM = r"""
+#define _GNU_SOURCE
+#include <dlfcn.h>
+#include <pthread.h>
+#include <stddef.h>
+size_t budget = (size_t)-1;
+static size_t live;
+static struct { void* p; size_t n; } blocks[65536];
+static pthread_mutex_t mu = PTHREAD_MUTEX_INITIALIZER;
+static void* hip(const char* f) { /* the runtime that libeegraph.so has loaded, which is in no global scope */
+    void* h = dlopen("libamdhip64.so.7", RTLD_LAZY | RTLD_NOLOAD);
+    return h ? dlsym(h, f) : NULL;
+}
+int hipMalloc(void** p, size_t n) {
+    static int (*next)(void**, size_t);
+    int rc = 2; /* hipErrorOutOfMemory */
+    if (!next) next = (int (*)(void**, size_t))hip("hipMalloc");
+    if (!next) return 1;
+    pthread_mutex_lock(&mu);
+    if (n <= budget && live <= budget - n) rc = next(p, n);
+    for (int i = 0; rc == 0 && i < 65536; ++i)
+        if (!blocks[i].p) {
+            blocks[i].p = *p;
+            blocks[i].n = n;
+            live += n;
+            break;
+        }
+    pthread_mutex_unlock(&mu);
+    return rc;
+}
+int hipFree(void* p) {
+    static int (*next)(void*);
+    if (!next) next = (int (*)(void*))hip("hipFree");
+    if (!next) return 1;
+    pthread_mutex_lock(&mu);
+    for (int i = 0; p && i < 65536; ++i)
+        if (blocks[i].p == p) {
+            live -= blocks[i].n;
+            blocks[i].p = NULL;
+            break;
+        }
+    pthread_mutex_unlock(&mu);
+    return next(p);
+}
+"""
+
+CHILD = r"""
+import ctypes, sys
+sys.path.insert(0, sys.argv[1])
+import numpy as np
+import eegraph_amd as eg
+from eegraph_amd import _lib as L
+
+budget = ctypes.c_size_t.in_dll(ctypes.CDLL(sys.argv[2]), "budget")
+ALL, MIB = (1 << 64) - 1, 1 << 20
+n, m = 200_000, 3_200_000
+rng = np.random.default_rng(1)
+s, d, w = (rng.integers(lo, hi, m).astype(np.uint32) for lo, hi in ((0, n), (0, n), (1, 60)))
+
+def graph():
+    return eg.Graph.from_edges(s, d, w, n=n)
+
+# least budget (bytes) of a call on a new handle; `tables`: built beforehand, without a budget
+def least(name, call, tables=0, lo=8, hi=260):
+    want = None
+    if call:
+        with graph() as g:
+            if tables: g.prepare(8, tables)
+            want = call(g)
+    def fits(mib):
+        g = None
+        try:
+            if call:
+                g = graph()
+                if tables: g.prepare(8, tables)
+            eg.trim()
+            budget.value = int(mib * MIB)
+            if call:
+                got = call(g)
+                assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (name, mib)
+            else:
+                g = graph()
+            return True
+        except eg.EEGError as e:
+            assert "out of memory" in str(e), (name, mib, e)
+            return False
+        finally:
+            budget.value = ALL
+            if g: g.close()
+
+    ok = [fits(mib) for mib in range(lo, hi, 2)]
+    first = ok.index(True)
+    top = lo + 2 * first
+    assert all(ok[first:]), (name, [lo + 2 * i for i in range(first, len(ok)) if not ok[i]])
+    step = 1.0  # from the step of the sweep down to an eighth of a MiB
+    while step >= 0.125:
+        if fits(top - step): top -= step
+        step /= 2
+    print(name, top, "MiB", flush=True)
+    return top * MIB
+
+# the edge list, the sorted sources, two lists of values and the sort's own copy: 44 bytes an edge
+assert least("create", None) <= 44 * m + 64 * n
+# planes of 32 columns (24 bytes a vertex and column) beside the graph (16 bytes an edge, and the sort
+# that builds the in-edges; 64 bytes a vertex)
+assert least("ppr batch", lambda g: g.run_batch("ppr", np.arange(20))[0]) <= 24 * 32 * n + 16 * m + 64 * n
+least("sssp", lambda g: g.run("sssp", 1)[0])
+least("sssp batch", lambda g: g.run_batch("sssp", np.arange(20))[0])
+print("done")
+"""
+
+
+@pytest.mark.skipif(not shutil.which("gcc"), reason="needs gcc")
+def test_within_a_budget(tmp_path):
+    (tmp_path / "shim.c").write_text(SHIM)
+    (tmp_path / "child.py").write_text(CHILD)
+    so = str(tmp_path / "shim.so")
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", str(tmp_path / "shim.c"), "-o", so, "-ldl", "-lpthread"], check=True)
+    env = dict(os.environ, LD_PRELOAD=":".join(x for x in (os.environ.get("LD_PRELOAD"), so) if x))
+    r = subprocess.run([sys.executable, "-u", str(tmp_path / "child.py"), ROOT, so], env=env, capture_output=True,
+                       text=True, timeout=110)
+    assert r.returncode == 0, r.stdout + r.stderr[-2000:]
+    assert "done" in r.stdout
