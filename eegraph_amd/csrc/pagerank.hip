@@ -853,30 +853,30 @@ eeg_status ensure_pr_span(eeg_graph* g, uint32_t K, bool inplace) {
             EEG_HIP(hipGetLastError());
         }
     }
+    // (the pull's tables are small; their memory is taken first, so that it can always run)
+    const uint32_t TV = PR_TILE / K;
+    const uint64_t ntiles = (t.P + TV - 1) / TV;
+    const uint32_t cap = (uint32_t)ntiles + 1;
+    EEG_TRY(t.span.alloc((size_t)cap * 4 + 8));  // and two counters
+    EEG_TRY(t.prstart.alloc((size_t)ntiles * 4 + 4));
     if (!inplace) {
         EEG_TRY(ensure_pr_stream(g, K));
         if (g->prstream.built) return EEG_OK;
     }
     if (t.span_built) return EEG_OK;
-    const uint32_t TV = PR_TILE / K;
-    const uint64_t ntiles = (t.P + TV - 1) / TV;
     hipStream_t s = g->stream;
-    DevMem cnt;
-    const uint32_t cap = (uint32_t)ntiles + 1;
-    EEG_TRY(t.span.alloc((size_t)cap * 4));
-    EEG_TRY(cnt.alloc(8));
-    EEG_HIP(hipMemsetAsync(cnt.p, 0, 8, s));
-    EEG_TRY(t.prstart.alloc((size_t)ntiles * 4 + 4));
+    uint32_t* cnt = t.span.as<uint32_t>() + cap;
+    EEG_HIP(hipMemsetAsync(cnt, 0, 8, s));
     if (t.nz) {
         k_list_spanning<<<std::max(1u, std::min(8192u, (t.nz + WG - 1) / WG)), WG, 0, s>>>(
-            t.vscan.as<uint32_t>(), t.nz, TV, cap, t.span.as<uint32_t>(), cnt.as<uint32_t>());
+            t.vscan.as<uint32_t>(), t.nz, TV, cap, t.span.as<uint32_t>(), cnt);
         EEG_HIP(hipGetLastError());
         k_tile_starts<<<std::max<uint64_t>(1, std::min<uint64_t>(4096, (ntiles + WG - 1) / WG)), WG, 0, s>>>(
             t.vscan.as<uint32_t>(), t.nz, TV, (uint32_t)ntiles, t.prstart.as<uint32_t>());
         EEG_HIP(hipGetLastError());
     }
     uint32_t ns[2] = {0, 0};
-    EEG_HIP(hipMemcpyAsync(ns, cnt.p, 8, hipMemcpyDeviceToHost, s));
+    EEG_HIP(hipMemcpyAsync(ns, cnt, 8, hipMemcpyDeviceToHost, s));
     EEG_HIP(hipStreamSynchronize(s));
     if ((uint64_t)ns[0] + ns[1] > cap) return fail(EEG_ERR_DEVICE, "PageRank span list overflow");
     t.nspan = ns[0];
@@ -905,28 +905,57 @@ eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_
     Work& w = wk ? *wk : g->work;
     EEG_TRY(ensure_in(g));
     EEG_TRY(ensure_tigr(g, g->in, g->tin, K));
-    EEG_TRY(ensure_pr_span(g, K, inplace));
     const Tigr& t = g->tin[k_index(K)];
     const PrStream& ps = g->prstream;
-    const bool stream = !inplace && ps.built;
-    const bool pairs = stream && n <= PS_PAIRS;
     const uint32_t TV = PR_TILE / K;
-    const uint64_t ntiles = stream ? ps.ntiles : (t.P + TV - 1) / TV;
+    const uint64_t pull_tiles = (t.P + TV - 1) / TV;
+    int cus = 256;
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->device);
+    // workgroups per CU: more than stay resident (8), so tiles are handed out as workgroups
+    // finish; 48 for the Jacobi gather, 24 in place (whose sweep count also depends on it)
+    const uint32_t wpc = o.wgs_per_cu ? o.wgs_per_cu : (inplace ? 24u : 48u);
+    const unsigned grid_pull = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(pull_tiles, (uint64_t)cus * wpc));
+    const unsigned grid_iso = std::max(1u, std::min(4096u, (n + WG - 1) / WG));
+    constexpr unsigned FIX_WGS = 1024;
 
-    EEG_TRY(w.ctl.alloc(sizeof(Ctl)));
-    if (!w.host_ctl) EEG_HIP(hipHostMalloc((void**)&w.host_ctl, 2 * sizeof(Ctl), hipHostMallocDefault));
-    for (int i = 0; i < 2; ++i) {
-        EEG_TRY(w.fx[i].alloc((size_t)n * 4 + 4));
-        EEG_TRY(w.fc[i].alloc((size_t)n * (pairs ? 8 : 4) + 8));
-        EEG_TRY(w.fl[i].alloc((size_t)n * 4 + 4));
+    // What the pull needs comes first: the streamed gather's tables and buffers take memory that is
+    // left over, and where there is too little of it the pull runs.
+    auto pull_state = [&]() -> eeg_status {
+        EEG_TRY(w.ctl.alloc(sizeof(Ctl)));
+        if (!w.host_ctl) EEG_HIP(hipHostMalloc((void**)&w.host_ctl, 2 * sizeof(Ctl), hipHostMallocDefault));
+        for (int i = 0; i < 2; ++i) {
+            EEG_TRY(w.fx[i].alloc((size_t)n * 4 + 4));
+            EEG_TRY(w.fc[i].alloc((size_t)n * (n <= PS_PAIRS ? 8 : 4) + 8));
+            EEG_TRY(w.fl[i].alloc((size_t)n * 4 + 4));
+        }
+        EEG_TRY(w.spill.alloc((size_t)(pull_tiles + 1) * 2 * sizeof(float2)));
+        EEG_TRY(w.red.alloc((size_t)std::max(grid_pull + FIX_WGS + grid_iso, PS_PARTS) * sizeof(double)));
+        return w.lab.alloc((size_t)n * 4 + 4);
+    };
+    EEG_TRY(pull_state());
+    EEG_TRY(ensure_pr_span(g, K, inplace));
+    bool stream = !inplace && ps.built;
+    if (stream) {
+        auto stream_state = [&]() -> eeg_status {
+            EEG_TRY(w.spill.alloc((size_t)(ps.ntiles + 1) * 2 * sizeof(float2)));
+            EEG_TRY(w.psum.alloc((size_t)ps.nz * sizeof(float2)));
+            return n > PS_PAIRS ? w.cerr.alloc((size_t)n * 4) : EEG_OK;
+        };
+        const eeg_status got = stream_state();
+        if (got == EEG_ERR_OOM) {
+            clear_error();
+            stream = false;
+            EEG_TRY(pull_state());
+            std::unique_lock<std::mutex> lk(g->mu, std::defer_lock);
+            if (wk) lk.lock();  // (otherwise the caller holds it)
+            EEG_TRY(ensure_pr_span(g, K, true));
+        } else {
+            EEG_TRY(got);
+        }
     }
-    EEG_TRY(w.spill.alloc((size_t)(ntiles + 1) * 2 * sizeof(float2)));
-    if (stream) EEG_TRY(w.psum.alloc((size_t)ps.nz * sizeof(float2)));
-    if (!pairs) {
-        const eeg_status got = w.cerr.alloc((size_t)n * 4);
-        if (stream) EEG_TRY(got);
-        else if (got != EEG_OK) clear_error();  // the pull does without
-    }
+    const bool pairs = stream && n <= PS_PAIRS;
+    const uint64_t ntiles = stream ? ps.ntiles : pull_tiles;
+    if (!stream && w.cerr.alloc((size_t)n * 4) != EEG_OK) clear_error();  // the pull does without
     // vertices whose virtual nodes cross a tile boundary (finished by k_pr_fix)
     const DevMem& span = t.span;
     const uint32_t nshort = t.nspan, nlong = t.nspan_long;
@@ -934,14 +963,7 @@ eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_
     const uint32_t* span_long = span.as<uint32_t>() + (t.span_cap - nlong);
     // the fix-up order only matters within a vertex, so the list order is irrelevant
 
-    int cus = 256;
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->device);
-    // workgroups per CU: more than stay resident (8), so tiles are handed out as workgroups
-    // finish; 48 for the Jacobi gather, 24 in place (whose sweep count also depends on it)
-    const uint32_t wpc = o.wgs_per_cu ? o.wgs_per_cu : (inplace ? 24u : 48u);
-    const unsigned grid_pull = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(ntiles, (uint64_t)cus * wpc));
-    const unsigned grid_fix = std::max(1u, std::min(1024u, std::max((nshort + WG - 1) / WG, (nlong + 3) / 4)));
-    const unsigned grid_iso = std::max(1u, std::min(4096u, (n + WG - 1) / WG));
+    const unsigned grid_fix = std::max(1u, std::min(FIX_WGS, std::max((nshort + WG - 1) / WG, (nlong + 3) / 4)));
     // streamed gather: its LDS admits one workgroup of 1024 threads per CU, which keeps its hubs
     // for all its tiles; a given wgs_per_cu counts 256-thread workgroups, so more take turns (a
     // serving lane leaves gaps for others).  At least 4 tiles per workgroup, and no more hubs
@@ -950,7 +972,6 @@ eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_
         1, std::min<uint64_t>((ntiles + 3) / 4, (uint64_t)cus * (o.wgs_per_cu ? (o.wgs_per_cu + 3) / 4 : 1)));
     const unsigned grid_finish = std::max(1u, std::min(PS_PARTS, (n + WG - 1) / WG));
     const uint32_t nparts = stream ? grid_finish : grid_pull + grid_fix + grid_iso;
-    EEG_TRY(w.red.alloc((size_t)nparts * sizeof(double)));
     EEG_HIP(hipMemsetAsync(w.red.p, 0, (size_t)nparts * sizeof(double), s));
 
     Ctl* ctl = w.ctl.as<Ctl>();
@@ -1136,7 +1157,6 @@ eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_
     if (rc == EEG_OK && !hc.done)
         rc = fail(EEG_ERR_NOT_CONVERGED, "PageRank residual above %g after %u iterations", eps, max_iters);
     // result: the buffer written by the last iteration, copied into the label slot
-    EEG_TRY(w.lab.alloc((size_t)n * 4 + 4));
     const int fb = inplace ? 0 : (int)(iters & 1);
     k_pr_output<<<grid_iso, WG, 0, s>>>(w.fx[fb].as<float>(), w.fl[fb].as<float>(), n, w.lab.as<float>());
     EEG_HIP(hipGetLastError());

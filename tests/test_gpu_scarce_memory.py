@@ -120,6 +120,20 @@ assert least("create", None) <= 44 * m + 64 * n
 assert least("ppr batch", lambda g: g.run_batch("ppr", np.arange(20))[0]) <= 24 * 32 * n + 16 * m + 64 * n
 least("sssp", lambda g: g.run("sssp", 1)[0])
 least("sssp batch", lambda g: g.run_batch("sssp", np.arange(20))[0])
+# PageRank with its tables at hand: the streamed gather where it fits, else the pull, which needs what
+# the in-place sweeps need (their ranks differ in the last bits, so each is held against its own)
+SLACK = 1e-6  # two forms of the sum, each within 2^-24 * (1 + 2 / (1 - 0.85)) of the exact iteration
+def ranks(variant):
+    def call(g):
+        x = g.run("pr", 0, variant=variant)[0]
+        assert np.abs(x.astype(np.float64) - exact).sum() < 2 * SLACK + 1e-7 * 0.85 / 0.15
+        return x * 0
+    return call
+with graph() as g:
+    exact = g.run("pr", 0, epsilon=1e-9)[0].astype(np.float64)
+tables = L.PREP_TRANSPOSE | L.PREP_TIGR
+in_place = least("pr, in place", ranks("async_push_dd"), tables)
+assert least("pr", ranks("sync_push_dd"), tables) <= in_place
 print("done")
 """
 
