@@ -84,15 +84,36 @@ __global__ void k_cc_init(const uint64_t* __restrict__ row, const uint32_t* __re
     }
 }
 
-// Every vertex points at its root (no links run beside it, so plain stores do).
+// Root of v, which v points at afterwards (no links run beside it, so roots stay roots).  Mostly a step
+// or two away.  Where first edges form a long chain (a wheel whose rim is listed first: a vertex a step,
+// although all vertices have a neighbour in common) the lanes on it jump: each stores how far it has got
+// and reads on from there past the caches, so that the distance doubles with every step of the lanes
+// that are under way.  The lanes above them come later, so a thread takes one vertex and the grid is as
+// large as the graph.  Device time on wheels of 2^20 / 2^22 vertices, walking only, with a grid of 8192
+// workgroups: 3.8 / 162 ms; now 0.27 / 0.75 (label propagation 0.19 / 0.68).  Walks up to CC_STEPS are
+// cheaper in the caches: jumping after 64 steps costs the 2048^2 grid 0.61 ms, after 128 0.55 as without.
+constexpr int CC_STEPS = 128;
+__device__ __forceinline__ uint32_t cc_settle(uint32_t* parent, uint32_t v) {
+    const uint32_t p = parent[v];
+    uint32_t r = p, g = parent[r];
+    for (int k = 0; k < CC_STEPS && g != r; ++k) {
+        r = g;
+        g = parent[r];
+    }
+    while (g != r) {
+        r = g;
+        __hip_atomic_store(&parent[v], r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        g = __hip_atomic_load(&parent[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (r != p) parent[v] = r;
+    return r;
+}
+
+// Every vertex points at its root.
 __global__ void k_cc_compress(uint32_t* parent, uint32_t n) {
     for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n;
-         v += (uint64_t)gridDim.x * blockDim.x) {
-        const uint32_t p = parent[v];
-        uint32_t r = p, g;
-        while ((g = parent[r]) != r) r = g;
-        if (r != p) parent[v] = r;
-    }
+         v += (uint64_t)gridDim.x * blockDim.x)
+        (void)cc_settle(parent, (uint32_t)v);
 }
 
 // First edges: the larger of two roots below the smaller.  Plain stores: of two links of the same
@@ -273,11 +294,7 @@ __global__ void k_cc_min(uint32_t* parent, uint32_t n, const uint32_t* __restric
         const uint64_t v = b + threadIdx.x;
         uint32_t r = 0xffffffffu, id = 0xffffffffu;
         if (v < n) {
-            const uint32_t p = parent[v];
-            uint32_t g;
-            r = p;
-            while ((g = parent[r]) != r) r = g;
-            if (r != p) parent[v] = r;
+            r = cc_settle(parent, (uint32_t)v);
             if (r != v) id = inv[v];
         }
         const uint32_t r0 = __builtin_amdgcn_readfirstlane(r);
@@ -318,16 +335,16 @@ eeg_status run_components(eeg_graph* g, eeg_stats* st, Work& w, hipStream_t s) {
     EEG_TRY(w.event(0, &e0));
     EEG_TRY(w.event(1, &e1));
     EEG_HIP(hipEventRecord(e0, s));
-    const unsigned gn = cc_grid(n);
+    const unsigned gn = cc_grid(n), gv = cc_grid(n, 0x7fffffffu);
     uint32_t launches = 3;
     k_cc_init<<<gn, WG, 0, s>>>(c.rowp(), c.colp(), n, inv, parent, minid, ctl);
     if (c.m) {
-        k_cc_compress<<<gn, WG, 0, s>>>(parent, n);
+        k_cc_compress<<<gv, WG, 0, s>>>(parent, n);
         k_cc_hook_first<<<gn, WG, 0, s>>>(c.rowp(), c.colp(), n, parent);
-        k_cc_compress<<<gn, WG, 0, s>>>(parent, n);
+        k_cc_compress<<<gv, WG, 0, s>>>(parent, n);
         k_cc_sample<<<1, CC_SAMPLE, 0, s>>>(c.colp(), c.m, parent, giant);
         k_cc_link_first<<<gn, WG, 0, s>>>(c.rowp(), c.colp(), n, parent, giant);
-        k_cc_compress<<<gn, WG, 0, s>>>(parent, n);
+        k_cc_compress<<<gv, WG, 0, s>>>(parent, n);
         if (sym) {
             k_cc_collect<<<gn, WG, 0, s>>>(c.rowp(), n, parent, giant, w.q[1].as<uint32_t>(), w.s[1].as<uint32_t>(), ctl);
             k_cc_link_queue<<<2048, WG, 0, s>>>(c.rowp(), c.colp(), w.q[1].as<uint32_t>(), w.s[1].as<uint32_t>(), ctl, parent);
@@ -338,7 +355,7 @@ eeg_status run_components(eeg_graph* g, eeg_stats* st, Work& w, hipStream_t s) {
         }
         launches += 8;
     }
-    k_cc_min<<<gn, WG, 0, s>>>(parent, n, inv, minid);
+    k_cc_min<<<gv, WG, 0, s>>>(parent, n, inv, minid);
     k_cc_label<<<gn, WG, 0, s>>>(parent, n, minid, w.lab.as<uint32_t>());
     EEG_HIP(hipGetLastError());
     EEG_HIP(hipEventRecord(e1, s));
