@@ -35,6 +35,25 @@ def test_labels(n, sym):
         assert np.array_equal(out, O.wcc(n, s, d)), k
 
 
+@pytest.mark.parametrize("sym", [False, True])
+@pytest.mark.parametrize("leaves", [1, 2, 3, 4, 65, 66, 67, 129, 1000])
+def test_forests(leaves, sym):
+    """Beside a giant component, trees whose hubs have around the two edges that are linked first, and the
+    64 more that a wave takes at once; joined in pairs by their last leaves."""
+    rng = np.random.default_rng(leaves)
+    k, giant = 40, 5000
+    hubs = giant + (leaves + 1) * np.arange(k)
+    s = np.r_[rng.integers(0, giant, 4 * giant), np.repeat(hubs, leaves), (hubs + leaves)[::2]]
+    d = np.r_[rng.integers(0, giant, 4 * giant), (hubs[:, None] + np.arange(1, leaves + 1)).ravel(), (hubs + leaves)[1::2]]
+    n = giant + (leaves + 1) * k
+    ids = rng.permutation(n)
+    s, d = (ids[x].astype(np.uint32) for x in (s, d))
+    with eg.Graph.from_edges(s, d, None, n=n) as g:
+        if sym:
+            g.prepare(8, eg._lib.PREP_SYM)
+        assert np.array_equal(g.run("cc", 0)[0], O.wcc(n, s, d))
+
+
 def test_long_chains_take_no_long_time():
     n = 1 << 22
     s, d = wheel(n)
