@@ -642,9 +642,9 @@ def main():
             run(alg, var)
     log(f"warmup {a.warmup} done")
 
-    # timed region: the default launch path; each run reports its device time from HIP events
-    # the library records on its own stream (first kernel to the end of the last working
-    # iteration), so a launch (one iteration) averages device time / working iterations
+    # timed region: the default launch path; each run reports its device time (first kernel to the
+    # fixpoint, by the device clock or by HIP events on the library's stream), so a launch (one
+    # iteration) averages device time / working iterations
     per_job = {j: [] for j in jobs}
     t0 = time.perf_counter()
     for k in range(a.steps):
@@ -666,18 +666,20 @@ def main():
         bytes_per_launch = c["bytes_alg"] / its
         avg_launch_ms = ksum / kn if kn else float("nan")
         key = f"{alg}/{var}"
+        # components of the dd variants are timed as union-find, whose iterations are no sweeps; their
+        # counted run propagates labels, so its bytes belong to other launches
+        union = alg == "cc" and var.endswith("_dd")
         per_alg[key] = {"gteps": m / ms / 1e6, "ms": round(ms, 4), "iterations": sts[0]["iterations"],
                         "edges_relaxed": c["edges_relaxed"], "label_updates": c["label_updates"],
                         "alg_bytes": c["bytes_alg"],
-                        "kernel_ms_avg": round(avg_launch_ms, 5),
-                        # CC is timed as union-find, its counted run propagates labels
-                        "alg_gbs": bytes_per_launch / avg_launch_ms / 1e6 if kn and alg != "cc" else None}
+                        "kernel_ms_avg": None if union else round(avg_launch_ms, 5),
+                        "alg_gbs": bytes_per_launch / avg_launch_ms / 1e6 if kn and not union else None}
         if alg == "pr":
             per_alg[key]["residual"] = sts[0]["pr_residual"]
-        if kn and (best is None or ksum > best[0]):
+        if kn and not union and (best is None or ksum > best[0]):
             best = (ksum, alg, var, bytes_per_launch, avg_launch_ms, kn)
 
-    kernel_names = {"bfs": "k_relax<BFS>", "sssp": "k_relax<SSSP>", "sswp": "k_relax<SSWP>", "cc": "k_cc_*",
+    kernel_names = {"bfs": "k_relax<BFS>", "sssp": "k_relax<SSSP>", "sswp": "k_relax<SSWP>", "cc": "k_relax<CC>",
                     "pr": "k_pr_stream+k_pr_finish" if best and best[2].startswith("sync") else "k_pr_pull+k_pr_fix+k_pr_reduce"}
     roofline = None
     if best:
@@ -725,8 +727,7 @@ def main():
                    "edges": m, "queries_per_step": len(jobs)},
         "timing": "value: wall time of the step's queries with the graph resident in HBM, labels "
                   "left on the device (no copy-out or un-permute, which add n x 4 bytes over PCIe "
-                  "per query); per-algorithm ms: device events from the first kernel to the end "
-                  "of the last working iteration",
+                  "per query); per-algorithm ms: device time from the first kernel to the fixpoint",
         "roofline": roofline,
         "cpu_baseline": cpu,
         "per_algorithm": per_alg,

@@ -122,7 +122,8 @@ typedef struct eeg_opts {
 } eeg_opts;
 
 typedef struct eeg_stats {
-    uint32_t iterations;        /* sweeps / frontier rounds that did work */
+    uint32_t iterations;        /* sweeps / frontier rounds that did work; 1 or 2 where CC is answered by
+                                   union-find, which has none and leaves the work counters at 0 */
     uint32_t launches;          /* relaxation kernels launched (includes no-op overshoot) */
     double ms_traversal;        /* device time from the first relaxation kernel to the fixpoint, or to
                                    the last iteration that a limit admits: the device clock as the
