@@ -337,7 +337,7 @@ eeg_status run_components(eeg_graph* g, eeg_stats* st, Work& w, hipStream_t s) {
     EEG_TRY(w.event(0, &e0));
     EEG_TRY(w.event(1, &e1));
     EEG_HIP(hipEventRecord(e0, s));
-    const unsigned gn = cc_grid(n), gv = cc_grid(n, 0x7fffffffu);
+    const unsigned gn = cc_grid(n), gv = cc_grid(n, 0xffffffu);  // (a launch holds fewer than 2^32 threads)
     uint32_t launches = 3;
     k_cc_init<<<gn, WG, 0, s>>>(c.rowp(), c.colp(), n, inv, parent, minid, ctl);
     if (c.m) {
