@@ -90,11 +90,14 @@ __device__ __forceinline__ float fed_contribution(float c, float hi, float lo, u
 // iterations after FP64 does; RMAT graphs are left alone.)
 constexpr double FEED_FROM = 1.5e-7, FEED_TO = 5e-8;
 enum Feed : uint32_t { FEED_WRITE = 1, FEED_READ = 2 };  // what an iteration does with the errors
-// Feed bits of the next iteration; `was`: of the one that ended.
-__device__ __forceinline__ uint32_t next_feed(double r, double last, double d, uint32_t was) {
-    const bool slow = r > (d + 0.25 * (1.0 - d)) * last;
-    if (!(r > FEED_TO && r <= FEED_FROM / (1.0 - d) && ((was & FEED_WRITE) || slow))) return 0u;
-    return FEED_WRITE | ((was & FEED_WRITE) ? FEED_READ : 0u);
+struct FeedRule {  // the two bounds for a damping
+    double factor, from;
+    explicit FeedRule(double d) : factor(d + 0.25 * (1.0 - d)), from(FEED_FROM / (1.0 - d)) {}
+};
+// Feed bits of the next iteration; `was`: of the one that ended, `wrote`: whether it could follow them.
+__device__ __forceinline__ uint32_t next_feed(double r, double last, const FeedRule& f, uint32_t was, bool wrote) {
+    if (!(r > FEED_TO && r <= f.from && ((was & FEED_WRITE) || r > f.factor * last))) return 0u;
+    return FEED_WRITE | ((was & FEED_WRITE) && wrote ? FEED_READ : 0u);
 }
 
 }  // namespace eeg

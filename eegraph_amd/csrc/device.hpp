@@ -136,13 +136,11 @@ struct Ctl {
     uint32_t done;                 // set once an iteration finds no work
     uint32_t iters;                // iterations that did work
     uint32_t err;                  // nonzero: a bound was hit (never written out of bounds)
-    uint32_t rounds;               // residual push: take passes that found work
+    uint32_t feed;                 // PR pull: Feed bits of the next iteration (compensated.hpp)
     unsigned long long stat[4];    // entries staged, vnodes pushed, edges relaxed, updates
     double residual[4];            // PR: L1 residual of the last iterations (slot i&3)
     double mass;                   // PR delta push / PPR: residual mass still unpushed
-    uint32_t feed;                 // PR pull: Feed bits of the next iteration (compensated.hpp)
-    uint32_t pad1;
-    double pad2[2];
+    double pad2[3];
 };
 
 }  // namespace eeg

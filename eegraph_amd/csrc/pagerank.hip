@@ -84,7 +84,9 @@ constexpr int PR_TILE = 2 * TILE_EDGES;
 // Virtual nodes of one entry in one tile beyond which a wave, not a thread, sums them.
 constexpr int PR_LONG = 32;
 
-template <int K>
+// FEED: rounding errors are fed back where the control block says so (a kernel of its own, which runs once
+// the host has seen that: 14.2 us a sweep of RMAT-16 against 13.2).
+template <int K, bool FEED>
 // At most 64 VGPRs, 8 waves per SIMD (K = 4: LDS holds 4 workgroups per CU, so 128): the
 // gathers are latency-bound, so the extra resident waves are worth more than the registers
 // (-4% per iteration against 71 VGPRs, 7 waves, at K = 8).
@@ -103,7 +105,7 @@ __global__ __launch_bounds__(WG, K >= 8 ? 8 : 4) void k_pr_pull(PullArgs a) {
     __shared__ double sRed[WG / WAVE];
 
     if (a.ctl->done) return;
-    const uint32_t feed = a.cerr ? a.ctl->feed : 0u;
+    const uint32_t feed = FEED ? a.ctl->feed : 0u;
     double res = 0.0;
     const uint32_t T = a.P, nE = a.nz;
     const uint32_t ntiles = (T + TV - 1) / TV;
@@ -352,9 +354,12 @@ __global__ void k_pr_isolated(const uint64_t* __restrict__ in_row, const uint32_
 // a tree), so the residual is deterministic.
 constexpr int RED_WG = 1024;
 __global__ __launch_bounds__(RED_WG) void k_pr_reduce(const double* __restrict__ part, uint32_t nparts, Ctl* ctl,
-                                                      uint32_t it, double eps, double damping) {
+                                                      uint32_t it, double eps, FeedRule rule,
+                                                      int fed) {
     __shared__ double sRed[RED_WG];
     if (ctl->done) return;
+    const double last = ctl->residual[(it - 1) & 3];
+    const uint32_t was = ctl->feed;
     // strided per thread, four loads in flight, added in index order (the same sum as one at
     // a time)
     double t = 0;
@@ -374,7 +379,7 @@ __global__ __launch_bounds__(RED_WG) void k_pr_reduce(const double* __restrict__
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        ctl->feed = next_feed(sRed[0], ctl->residual[(it - 1) & 3], damping, ctl->feed);
+        ctl->feed = next_feed(sRed[0], last, rule, was, fed);
         ctl->residual[it & 3] = sRed[0];
         ctl->iters = it;
         if (sRed[0] < eps) ctl->done = 1;
@@ -999,9 +1004,12 @@ eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_
     pa.pers_base = 1.0f - d;
     pa.strided = inplace ? 1u : 0u;
     pa.tstart = t.prstart.as<uint32_t>();
-    pa.cerr = stream ? nullptr : w.cerr.as<float>();
     double* red = w.red.as<double>();
-    auto pull_fn = (K == 4) ? k_pr_pull<4> : (K == 8) ? k_pr_pull<8> : (K == 16) ? k_pr_pull<16> : k_pr_pull<32>;
+    auto pull_fn = (K == 4) ? k_pr_pull<4, false> : (K == 8) ? k_pr_pull<8, false>
+                   : (K == 16) ? k_pr_pull<16, false> : k_pr_pull<32, false>;
+    auto pull_feed_fn = (K == 4) ? k_pr_pull<4, true> : (K == 8) ? k_pr_pull<8, true>
+                        : (K == 16) ? k_pr_pull<16, true> : k_pr_pull<32, true>;
+    bool feed = false;  // the pull has been seen to want its rounding errors fed back
 
     const bool nontemporal = (uint64_t)ps.ntiles * PS_TILE * 4 > PS_STREAM_BYTES;
     StreamArgs sa{};
@@ -1061,8 +1069,9 @@ eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_
             (pairs ? k_pr_finish<true> : k_pr_finish<false>)<<<grid_finish, WG, 0, s>>>(fa);
             EEG_HIP(hipGetLastError());
         } else if (t.P) {
+            pa.cerr = feed ? w.cerr.as<float>() : nullptr;
             void* args[] = {&pa};
-            EEG_HIP(hipLaunchKernel((const void*)pull_fn, dim3(grid_pull), dim3(WG), args, 0, s));
+            EEG_HIP(hipLaunchKernel((const void*)(feed ? pull_feed_fn : pull_fn), dim3(grid_pull), dim3(WG), args, 0, s));
         } else {
             EEG_HIP(hipMemsetAsync(red, 0, grid_pull * sizeof(double), s));
         }
@@ -1081,7 +1090,7 @@ eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_
             EEG_HIP(hipMemsetAsync(red + grid_pull + grid_fix, 0, grid_iso * sizeof(double), s));
         }
         // (the streamed gather sums the residual at the start of the next iteration)
-        if (!stream) k_pr_reduce<<<1, RED_WG, 0, s>>>(red, nparts, ctl, it, eps, (double)d);
+        if (!stream) k_pr_reduce<<<1, RED_WG, 0, s>>>(red, nparts, ctl, it, eps, FeedRule(d), feed);
         EEG_HIP(hipGetLastError());
         if (recorded.size() <= it) recorded.resize((size_t)it + 64, 0);
         recorded[it] = (rec || o.timing) ? 1 : 0;
@@ -1147,6 +1156,7 @@ eeg_status run_pagerank(eeg_graph* g, uint32_t algo, uint32_t source, const eeg_
             const uint32_t inflight = (it - 1) - h.iters, rem = remaining(h);
             chunk = rem > inflight ? std::min<uint32_t>(rem - inflight + 1, 16) : 1u;
             predicted_end = h.iters + rem;
+            feed = feed || (h.feed && w.cerr.p && !stream);
             cur ^= 1;
         }
     }

@@ -409,7 +409,7 @@ __global__ __launch_bounds__(WG) void k_pps_fix(PlaneArgsP a, double* res_part) 
 // workgroup with a load at a time, 9 us as this).
 // Decides as well what the next iteration does with the column's rounding errors (feed).
 __global__ __launch_bounds__(WG) void k_pps_reduce(const double* __restrict__ part, uint32_t nparts, uint32_t W,
-                                                   double* __restrict__ resid, double damping, uint32_t fresh,
+                                                   double* __restrict__ resid, FeedRule rule, uint32_t fresh,
                                                    PprColState* __restrict__ col_state) {
     __shared__ double s[WG / WAVE];
     const double* p = part + blockIdx.x;
@@ -435,7 +435,7 @@ __global__ __launch_bounds__(WG) void k_pps_reduce(const double* __restrict__ pa
                            (unsigned long long)__double_as_longlong(r), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         PprColState& c = col_state[blockIdx.x];
         const bool first = (fresh >> blockIdx.x) & 1u;
-        c.feed = next_feed(r, first ? r : c.last, damping, first ? 0u : c.feed);
+        c.feed = next_feed(r, first ? r : c.last, rule, first ? 0u : c.feed, true);
         c.last = r;
     }
 }
@@ -618,7 +618,7 @@ eeg_status PprPlane::iterate(eeg_graph* g, uint32_t j, const PprCols& cols, hipS
         k_pps_fix<32><<<grid_fix, WG, 0, s>>>(a, fix_part);
     }
     k_pps_reduce<<<W, WG, 0, s>>>(res_part.as<double>(), grid_pull + grid_fix, W, resid,
-                                  (double)damping, cols.fresh, col_state.as<PprColState>());
+                                  FeedRule(damping), cols.fresh, col_state.as<PprColState>());
     EEG_HIP(hipGetLastError());
     return EEG_OK;
 }
