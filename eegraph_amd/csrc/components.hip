@@ -16,9 +16,9 @@
 // and costs a step, never a lost link, and shortcuts are stored past the caches (agent scope).  The label of a
 // component is its smallest original id, as everywhere: whatever the order of the links, the
 // answer is unique.
-// Measured, device time against label propagation: RMAT-22 1.89 -> 0.21 ms with the symmetrised
-// list and 0.63 without (which saves its sort of 134 M pairs), 4096^2 grid 29 -> 2.6 / 2.5 ms,
-// RMAT-14 0.05 ms.  Bound by the line fetched for the first edges of every vertex.
+// Measured, device time against label propagation: RMAT-22 1.89 -> 0.20 ms with the symmetrised
+// list and 0.64 without (which saves its sort of 134 M pairs), 4096^2 grid 33 -> 1.6 / 1.8 ms,
+// RMAT-14 0.20 -> 0.04 / 0.05 ms.  Bound by the line fetched for the first edges of every vertex.
 #include <algorithm>
 #include <chrono>
 

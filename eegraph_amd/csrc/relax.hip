@@ -675,8 +675,8 @@ eeg_status run_traversal(eeg_graph* g, uint32_t algo, uint32_t source, const eeg
     Work& w = wk ? *wk : g->work;
     // Components by union-find where only the labels are asked for: a run that counts, times or
     // limits iterations, names a frontier kind other than the default or sweeps every virtual
-    // node propagates labels (device time of that against this: RMAT-22 1.9 / 0.21 ms,
-    // 4096^2 grid 29 / 2.6 ms)
+    // node propagates labels (device time of that against this: RMAT-22 1.9 / 0.20 ms,
+    // 4096^2 grid 33 / 1.6 ms)
     if (alg == A_CC && (by_default || mode == M_ASYNC) && !o.collect_activity && !o.count_work && !o.timing && !o.max_iters)
         return run_components(g, st, w, s);
     if (alg == A_CC) EEG_TRY(ensure_sym(g));
